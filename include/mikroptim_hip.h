@@ -128,10 +128,11 @@ int mko_gram_device(const double* jacobian, const double* r0, int runs, int vari
                     int64_t rows, double* a, double* g, void* stream);
 
 /* The same normal equations on FP64 MFMA (v_mfma_f64_16x16x4_f64, 16 x 16 tiles, FP64
- * accumulation): equal to mko_gram_device up to rounding (another summation order, so not
- * bitwise the host chain); up to 127 variables. Replaces gram_kernel
- * (src/cuda/normal_equations.cu:48) where bitwise parity with normal_equations_host is not
- * required (MKO_PRECISION_FP64_MFMA in the host layer). */
+ * accumulation); up to 127 variables. Replaces gram_kernel (src/cuda/normal_equations.cu:48)
+ * where bitwise parity with normal_equations_host is not required (MKO_PRECISION_FP64_MFMA in
+ * the host layer): a caller may count on rounding-level agreement with mko_gram_device only,
+ * whose kernel it runs today (up to 127 variables that one takes the same matrix instructions,
+ * which round as the chain does). */
 int mko_gram_mfma_device(const double* jacobian, const double* r0, int runs, int variables,
                          int64_t rows, double* a, double* g, void* stream);
 

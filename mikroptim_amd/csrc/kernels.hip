@@ -2463,15 +2463,143 @@ __global__ __launch_bounds__(256) void adjoint_normal_finalize_kernel(
     if (tid < Pn) g[size_t(v) * Pn + tid] = gacc;
 }
 
-// ---- Gram: A = [J r0]^T [J r0] per run -----------------------------------------------------
+// ---- Gram: A = J^T J, g = J^T r0 per run ----------------------------------------------------
 
-// 64 x 64 output tile per workgroup over the upper tiles of the (P+1) x (P+1) matrix, 256 threads
+typedef __attribute__((ext_vector_type(4))) double f64x4;
+
+// Each element is one FMA chain over the rows in ascending order starting from 0 (gram_dot,
+// normal_equations.hpp:19), products of the stored J values: bitwise the host definition.
+// v_mfma_f64_16x16x4_f64 adds its four products to the accumulator as that chain does (measured
+// bit for bit on MI355X against the VALU chain over rows of mixed signs and 24 decades; the GPU
+// tests hold it), so J^T J runs on it in 16 x 16 tiles; operand lane l: A(m = l % 16, k = l / 16),
+// B(k = l / 16, n = l % 16), result lane l, element e: row 4 e + l / 16, column l % 16. g is a
+// VALU chain per column beside the tiles: as a matrix column it would cost a row of tiles of its
+// own (10 instead of 6 at 48 variables).
+//
+// One workgroup of 8 waves per (run, part): the units (a wave of 64 columns of g, or one upper
+// tile) are cut into `parts` ranges, a wave takes kT of its range; the columns that the range
+// needs are staged kC rows at a time, one wave load per 64 rows of a column, the next rows
+// loaded into registers while the tiles run on the present ones. What bounds it: a tile's chain
+// is rows / 4 dependent matrix instructions of 16 passes (17920 rows: 0.12 ms however many runs),
+// so a few runs are spread over more workgroups, at most one tile per SIMD; with many runs the
+// reading of J (7 MB per run at 48 variables). Measured at 48 variables and 17920 rows, against
+// one 64 x 64 tile of 4 x 4 VALU chains per thread and workgroup: 1 run 0.31 (2.65) ms, 64 runs
+// 0.34 (3.21) ms, 1024 runs 1.79 (5.03) ms (3.9 TB/s of J); 1024 runs of 96 variables and 1200
+// rows 0.38 (1.16) ms.
+template <int kT, int kC, int kV>
+__global__ __launch_bounds__(512) void gram_kernel(const double* J, const double* r0, int P,
+                                                   int64_t rows, int parts, int upp, double* a,
+                                                   double* g, const int32_t* live) {
+    constexpr int kLd = kC + 2; // doubles; 2 modulo 32: a tile's 16 columns x 2 rows hit all banks
+    constexpr int kH = kC / 64; // wave loads per column and stage
+    extern __shared__ __align__(16) double Xs[]; // [16 tg + 1][kLd], r0 last
+    const int run = int(blockIdx.x) / parts, part = int(blockIdx.x) - run * parts;
+    if (live && run >= *live) return;
+    const int tg = (P + 15) / 16, gw = (P + 63) / 64;
+    const int units = gw + tg * (tg + 1) / 2;
+    const int first = part * upp, last = min(units, first + upp);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m = lane & 15, kk = lane >> 4;
+    f64x4 acc[kT];
+    double gacc[kT];
+    int tI[kT], tJ[kT]; // unit: tile (I, J); (-2, w): columns 64 w ... of g; (-1, .): none
+#pragma unroll
+    for (int i = 0; i < kT; ++i) {
+        acc[i] = f64x4{0.0, 0.0, 0.0, 0.0};
+        gacc[i] = 0.0;
+        tI[i] = tJ[i] = -1;
+        const int u = first + wave + 8 * i;
+        if (u < last) {
+            if (u < gw) {
+                tI[i] = -2;
+                tJ[i] = u;
+            } else {
+                tile_of(u - gw, tg, tI[i], tJ[i]);
+            }
+        }
+    }
+    // the columns staged: from the first tile's row panel on (all with a g unit)
+    int c0 = 0;
+    if (first >= gw) {
+        int J0;
+        tile_of(first - gw, tg, c0, J0);
+        c0 *= 16;
+    }
+    const bool with_r0 = first < gw;
+    const int ncols = P - c0 + (with_r0 ? 1 : 0);
+    const double* Jr = J + size_t(run) * P * rows;
+    const double* rr = r0 + size_t(run) * rows;
+    double* Xr = Xs + size_t(16 * tg) * kLd;
+    for (int e = tid; e < (16 * tg - P) * kLd; e += 512) Xs[size_t(P) * kLd + e] = 0.0;
+    double next[kV];
+    auto load = [&](int64_t base) {
+#pragma unroll
+        for (int i = 0; i < kV; ++i) {
+            const int x = wave + 8 * (i / kH); // staged column
+            const int64_t row = base + 64 * (i % kH) + lane;
+            const int c = c0 + x;
+            next[i] = 0.0;
+            if (x < ncols && row < rows) next[i] = c < P ? Jr[size_t(c) * rows + row] : rr[row];
+        }
+    };
+    load(0);
+    for (int64_t base = 0; base < rows; base += kC) {
+        const int n = int(rows - base < kC ? rows - base : kC);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kV; ++i) {
+            const int x = wave + 8 * (i / kH), c = c0 + x;
+            if (x < ncols) (c < P ? Xs + size_t(c) * kLd : Xr)[64 * (i % kH) + lane] = next[i];
+        }
+        __syncthreads();
+        if (base + kC < rows) load(base + kC);
+#pragma unroll
+        for (int i = 0; i < kT; ++i) {
+            if (tI[i] >= 0) {
+                const double* xa = Xs + size_t(tI[i] * 16 + m) * kLd + kk;
+                const double* xb = Xs + size_t(tJ[i] * 16 + m) * kLd + kk;
+                // rows beyond n are staged as zeros: their products leave the sums as they are
+                const int steps = (n + 3) / 4;
+#pragma unroll 8
+                for (int st = 0; st < steps; ++st)
+                    acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[4 * st], xb[4 * st], acc[i],
+                                                                  0, 0, 0);
+            } else if (tI[i] == -2) {
+                const int p = tJ[i] * 64 + lane;
+                const double* x = Xs + size_t(p < P ? p : 0) * kLd;
+#pragma unroll 8
+                for (int r = 0; r < n; ++r) gacc[i] = __fma_rn(x[r], Xr[r], gacc[i]);
+            }
+        }
+    }
+    double* A = a + size_t(run) * P * P;
+#pragma unroll
+    for (int i = 0; i < kT; ++i) {
+        if (tI[i] >= 0) {
+            const int col = tJ[i] * 16 + m;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = tI[i] * 16 + 4 * e + kk;
+                if (row < P && col < P) {
+                    A[size_t(row) * P + col] = acc[i][e];
+                    A[size_t(col) * P + row] = acc[i][e];
+                }
+            }
+        } else if (tI[i] == -2) {
+            const int p = tJ[i] * 64 + lane;
+            if (p < P) g[size_t(run) * P + p] = gacc[i];
+        }
+    }
+}
+
+// More than 127 variables (their columns do not fit the LDS stages above): 64 x 64 output tile per
+// workgroup over the upper tiles of the (P+1) x (P+1) matrix, 256 threads
 // each holding a 4 x 4 block of elements: 16 independent FMA chains per thread (the chains' latency
 // is what bounds a Gram of long columns). Rows are staged through LDS 32 at a time, row-major
 // [row][column], so a thread reads its 4 consecutive columns as two 16-byte words. Each element is
 // one FMA chain over the rows in ascending order starting from 0 (gram_dot,
 // normal_equations.hpp:19), products of the stored J values: bitwise the host definition.
-__global__ __launch_bounds__(256) void gram_kernel(const double* J, const double* r0, int runs, int P,
+__global__ __launch_bounds__(256) void gram_wide_kernel(const double* J, const double* r0, int runs, int P,
                                                    int64_t rows, double* a, double* g,
                                                    const int32_t* live) {
     constexpr int kT = 64, kC = 32, kLd = kT + 2; // row stride in doubles (16-byte aligned rows)
@@ -2540,82 +2668,6 @@ __global__ __launch_bounds__(256) void gram_kernel(const double* J, const double
                 gr[p] = v;
             } else if (p == P && q < P) {
                 gr[q] = v;
-            }
-        }
-    }
-}
-
-// ---- Gram on FP64 MFMA ----------------------------------------------------------------------
-
-typedef __attribute__((ext_vector_type(4))) double f64x4;
-
-// [J r0]^T [J r0] of one run per workgroup with v_mfma_f64_16x16x4_f64: the run's P + 1 columns
-// staged through LDS 32 rows at a time (doubles, row stride 33), the upper 16 x 16 tiles of the
-// (P + 1) x (P + 1) result spread over the 4 waves (kTiles per wave), FP64 accumulation in the
-// MFMA unit. Operand lane l: A(m = l % 16, k = l / 16), B(k = l / 16, n = l % 16); result lane l,
-// element e: row 4 e + l / 16, column l % 16 (measured on MI355X). Not the host's summation
-// order (unlike gram_kernel): the results differ from normal_equations_host by rounding.
-template <int kTiles>
-__global__ __launch_bounds__(256) void gram_mfma_kernel(const double* J, const double* r0, int P,
-                                                        int64_t rows, double* a, double* g) {
-    constexpr int kC = 32, kLd = kC + 1;
-    extern __shared__ double Xs[]; // [16 tg][kLd]
-    const int run = blockIdx.x;
-    const int Q = P + 1;
-    const int tg = (Q + 15) / 16, cols = 16 * tg;
-    const int ntiles = tg * (tg + 1) / 2;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    f64x4 acc[kTiles];
-    int tI[kTiles], tJ[kTiles];
-#pragma unroll
-    for (int i = 0; i < kTiles; ++i) {
-        acc[i] = f64x4{0.0, 0.0, 0.0, 0.0};
-        const int tt = wave + 4 * i;
-        tI[i] = -1;
-        tJ[i] = -1;
-        if (tt < ntiles) tile_of(tt, tg, tI[i], tJ[i]);
-    }
-    const double* Jr = J + size_t(run) * P * rows;
-    const double* rr = r0 + size_t(run) * rows;
-    const int m = lane & 15, kk = lane >> 4;
-    for (int64_t base = 0; base < rows; base += kC) {
-        for (int e = tid; e < cols * kC; e += 256) {
-            const int c = e / kC, rw = e - c * kC;
-            const int64_t row = base + rw;
-            double v = 0.0;
-            if (row < rows) v = c < P ? Jr[size_t(c) * rows + row] : c == P ? rr[row] : 0.0;
-            Xs[c * kLd + rw] = v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kTiles; ++i) {
-            if (tI[i] < 0) continue;
-            const double* xa = Xs + (tI[i] * 16 + m) * kLd + kk;
-            const double* xb = Xs + (tJ[i] * 16 + m) * kLd + kk;
-#pragma unroll
-            for (int st = 0; st < kC / 4; ++st)
-                acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[4 * st], xb[4 * st], acc[i], 0, 0,
-                                                              0);
-        }
-        __syncthreads();
-    }
-    double* A = a + size_t(run) * P * P;
-    double* gr = g + size_t(run) * P;
-#pragma unroll
-    for (int i = 0; i < kTiles; ++i) {
-        if (tI[i] < 0) continue;
-        const int col = tJ[i] * 16 + m;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = tI[i] * 16 + 4 * e + kk;
-            const double v = acc[i][e];
-            if (row < P && col < P) {
-                A[size_t(row) * P + col] = v;
-                A[size_t(col) * P + row] = v;
-            } else if (row < P && col == P) {
-                gr[row] = v;
-            } else if (row == P && col < P) {
-                gr[col] = v;
             }
         }
     }
@@ -3406,10 +3458,39 @@ int gram_chain(const double* jacobian, const double* r0, int runs, int variables
                double* a, double* g, void* stream, const int32_t* live) {
     MKO_TRY({
         if (runs <= 0) return 0;
-        const int T = (variables + 1 + 63) / 64;
-        const dim3 grid(unsigned(runs) * unsigned(T * (T + 1) / 2));
-        hipLaunchKernelGGL(gram_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream),
-                           jacobian, r0, runs, variables, rows, a, g, live);
+        const hipStream_t s = static_cast<hipStream_t>(stream);
+        if (variables > 127) {
+            const int T = (variables + 1 + 63) / 64;
+            hipLaunchKernelGGL(gram_wide_kernel, dim3(unsigned(runs) * unsigned(T * (T + 1) / 2)),
+                               dim3(256), 0, s, jacobian, r0, runs, variables, rows, a, g, live);
+            check_hip(hipGetLastError(), "gram launch");
+            return 0;
+        }
+        const int tg = (variables + 15) / 16, gw = (variables + 63) / 64;
+        const int units = gw + tg * (tg + 1) / 2;
+        // Workgroups per run: at least 4 units (one tile per SIMD) each, and only while the runs
+        // leave CUs idle (up to 512 workgroups): beyond that a second workgroup only reads most
+        // of the run's J again.
+        const int parts = std::max(1, std::min((units + 3) / 4, 512 / runs));
+        const int upp = (units + parts - 1) / parts;
+        const auto launch = [&](auto kernel, int stage) {
+            hipLaunchKernelGGL(kernel, dim3(unsigned(runs) * unsigned(parts)), dim3(512),
+                               size_t(16 * tg + 1) * size_t(stage + 2) * sizeof(double), s,
+                               jacobian, r0, variables, rows, parts, upp, a, g, live);
+        };
+        // staged values per thread: (variables + 1) columns / 8 waves x (rows of a stage) / 64;
+        // above 64 variables 64 rows at a time, so that the columns fit the LDS of two workgroups
+        if (variables < 56) {
+            if (upp <= 8) launch(gram_kernel<1, 128, 14>, 128);
+            else launch(gram_kernel<2, 128, 14>, 128);
+        } else if (variables <= 64) {
+            if (upp <= 8) launch(gram_kernel<1, 128, 18>, 128);
+            else launch(gram_kernel<2, 128, 18>, 128);
+        } else {
+            if (upp <= 8) launch(gram_kernel<1, 64, 16>, 64);
+            else if (upp <= 24) launch(gram_kernel<3, 64, 16>, 64);
+            else launch(gram_kernel<5, 64, 16>, 64);
+        }
         check_hip(hipGetLastError(), "gram launch");
     })
 }
@@ -3465,21 +3546,11 @@ int mko_df64_ops_device(int op, int64_t n, const float* a, const float* b, float
 
 int mko_gram_mfma_device(const double* jacobian, const double* r0, int runs, int variables,
                          int64_t rows, double* a, double* g, void* stream) {
-    MKO_TRY({
-        if (variables < 1 || variables > 127) throw std::invalid_argument("1 ... 127 variables");
-        if (rows < 0) throw std::invalid_argument("negative row count");
-        if (runs <= 0) return 0;
-        const int Q = variables + 1, tg = (Q + 15) / 16;
-        const size_t lds = size_t(16 * tg) * 33 * sizeof(double);
-        const hipStream_t s = static_cast<hipStream_t>(stream);
-        if (tg <= 4)
-            hipLaunchKernelGGL(gram_mfma_kernel<3>, dim3(unsigned(runs)), dim3(256), lds, s,
-                               jacobian, r0, variables, rows, a, g);
-        else
-            hipLaunchKernelGGL(gram_mfma_kernel<9>, dim3(unsigned(runs)), dim3(256), lds, s,
-                               jacobian, r0, variables, rows, a, g);
-        check_hip(hipGetLastError(), "gram mfma launch");
-    })
+    if (variables < 1 || variables > 127 || rows < 0) {
+        mko_detail::last_error = rows < 0 ? "negative row count" : "1 ... 127 variables";
+        return MKO_ERR_INVALID;
+    }
+    return mko_internal::gram_chain(jacobian, r0, runs, variables, rows, a, g, stream, nullptr);
 }
 
 size_t mko_vjp_workspace(int variants, int fields, int wavelengths, int variables) {
