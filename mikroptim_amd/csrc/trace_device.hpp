@@ -2,12 +2,13 @@
 // type R (double or df64 for the forward trace; double for the reverse sweep).
 //
 // Formulas and branch rules follow the reference's shared math core:
-//   surface steps        include/mikroptim/trace/surface_ops.hpp:122-203
+//   surface steps        include/mikroptim/trace/surface_ops.hpp:122-203 (FP64: the same
+//                        intersection and refraction in optical direction cosines)
 //   surface propagation  include/mikroptim/trace/trace.hpp:175-229 (stop/plane/sphere only)
 //   reference spheres    include/mikroptim/trace/reference_sphere.hpp:56-143
 //   reverse steps        include/mikroptim/trace/adjoint_backward.hpp:115-241, 373-464
-// The FP64 surface step spells its fmas out (no contraction left to the compiler, so every kernel
-// that inlines it computes the same bits); the rest is compiled with FMA contraction (hipcc
+// The FP64 surface steps spell their fmas out (no contraction left to the compiler, so every kernel
+// that inlines them computes the same bits); the rest is compiled with FMA contraction (hipcc
 // default). Results differ from the FP64 CPU oracle by rounding only, which the parity tests
 // bound per ray.
 #pragma once
@@ -85,45 +86,28 @@ __device__ __forceinline__ bool is_soft(uint8_t s) {
     return s == MKO_STATUS_SOFT_MISSED || s == MKO_STATUS_SOFT_TIR;
 }
 
-// Division, reciprocal and square root of the reverse sweep, of the state reconstruction and of
-// the fused kernel's forward trace: hardware reciprocal / reciprocal square root refined by
+// Division, reciprocal and square root of the FP64 traces and of the reverse sweep: hardware reciprocal / reciprocal square root refined by
 // Newton steps (a few ulp) instead of the correctly rounded IEEE sequences with their scaling and
 // fix-up steps. These paths need ~1e-15 relative accuracy (Jacobian columns are compared to
 // 1e-10, OPD to 1e-12 mm per ray); the df64 trace keeps its own operations.
-#ifndef MKO_REVERSE_FAST_MATH
-#define MKO_REVERSE_FAST_MATH 1
-#endif
 // Measured on MI355X (2^20 arguments over 2^+-30): v_rcp_f64 and v_rsq_f64 are accurate to
 // ~5e-8; one Newton step gives 2.1e-15, two give <= 0.5 ulp. The quotient a * r with one residual
 // correction and the square root after one Goldschmidt step plus one correction are within
 // 0.5 ulp (1.1e-16) as well.
 __device__ __forceinline__ double rcp_nr1(double b) {
-#if MKO_REVERSE_FAST_MATH
     const double r = __builtin_amdgcn_rcp(b);
     return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
-#else
-    return 1.0 / b;
-#endif
 }
 __device__ __forceinline__ double rev_rcp(double b) {
-#if MKO_REVERSE_FAST_MATH
     const double r = rcp_nr1(b);
     return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
-#else
-    return 1.0 / b;
-#endif
 }
 __device__ __forceinline__ double rev_div(double a, double b) {
-#if MKO_REVERSE_FAST_MATH
     const double r = rcp_nr1(b);
     const double q = a * r;
     return __builtin_fma(__builtin_fma(-b, q, a), r, q);
-#else
-    return a / b;
-#endif
 }
 __device__ __forceinline__ double rev_sqrt(double x) {
-#if MKO_REVERSE_FAST_MATH
     if (!(x > 0.0)) return __builtin_sqrt(x);
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
@@ -132,15 +116,11 @@ __device__ __forceinline__ double rev_sqrt(double x) {
     h = __builtin_fma(h, r, h);
     const double d = __builtin_fma(-g, g, x);
     return __builtin_fma(d, h, g);
-#else
-    return __builtin_sqrt(x);
-#endif
 }
 
 // rev_sqrt that also returns 1 / (2 sqrt(x)): the Goldschmidt iteration's refined half reciprocal
 // (~1e-15 relative), for callers that divide by twice the root.
 __device__ __forceinline__ double rev_sqrt_half_rcp(double x, double& half_rcp) {
-#if MKO_REVERSE_FAST_MATH
     if (!(x > 0.0)) {
         const double g = __builtin_sqrt(x);
         half_rcp = 0.5 / g;
@@ -154,11 +134,6 @@ __device__ __forceinline__ double rev_sqrt_half_rcp(double x, double& half_rcp) 
     const double d = __builtin_fma(-g, g, x);
     half_rcp = h;
     return __builtin_fma(d, h, g);
-#else
-    const double g = __builtin_sqrt(x);
-    half_rcp = 0.5 / g;
-    return g;
-#endif
 }
 
 template <class R>
@@ -166,17 +141,11 @@ struct RayAdj {
     V3<R> p, d;
 };
 
-// Forward-trace division / square root: IEEE, or the Newton-refined forms above (kFast, double).
-template <bool kFast, class R>
-__device__ __forceinline__ R fdiv(R a, R b) {
-    if constexpr (kFast) return rev_div(a, b);
-    else return a / b;
-}
-template <bool kFast, class R>
-__device__ __forceinline__ R fsqrt(R x) {
-    if constexpr (kFast) return rev_sqrt(x);
-    else return dsqrt(x);
-}
+// Forward-trace division / square root: the Newton-refined forms above in double, df64's own.
+__device__ __forceinline__ double fdiv(double a, double b) { return rev_div(a, b); }
+__device__ __forceinline__ df64 fdiv(df64 a, df64 b) { return a / b; }
+__device__ __forceinline__ double fsqrt(double x) { return rev_sqrt(x); }
+__device__ __forceinline__ df64 fsqrt(df64 x) { return dsqrt(x); }
 
 // Accumulator of soft ray failure (SoftFailure, surface_ops.hpp:94).
 struct Soft {
@@ -195,146 +164,19 @@ struct RayT {
 };
 using Ray = RayT<double>;
 
-// The FP64 surface step with its arithmetic spelled out: each product that fuses into a sum is
-// one fma and every other operation is rounded on its own (no contraction is left to the
-// compiler), so every kernel that inlines the step computes the same bits, in hard and in soft
-// failure mode.
-struct StepQuadratic {
-    double s0, px, py, H, B, D;
-};
-// transfer_to_tangent_plane and the coefficients of intersect_sphere's quadratic
-template <bool kFast>
-__device__ __forceinline__ StepQuadratic step_quadratic(const RayT<double>& r, double c,
-                                                        double t) {
-#pragma clang fp contract(off)
-    StepQuadratic q;
-    q.s0 = fdiv<kFast>(-(r.p.z - t), r.d.z);
-    q.px = __builtin_fma(q.s0, r.d.x, r.p.x);
-    q.py = __builtin_fma(q.s0, r.d.y, r.p.y);
-    q.H = c * __builtin_fma(q.py, q.py, q.px * q.px);
-    q.B = __builtin_fma(-c, __builtin_fma(r.d.y, q.py, r.d.x * q.px), r.d.z);
-    q.D = __builtin_fma(q.B, q.B, -(c * q.H));
-    return q;
-}
-__device__ __forceinline__ double dot_fma(V3<double> a, V3<double> b) {
-#pragma clang fp contract(off)
-    return __builtin_fma(a.z, b.z, __builtin_fma(a.y, b.y, a.x * b.x));
-}
-// the intersection p + s d (p.z = 0 on the tangent plane) and the surface normal there
-__device__ __forceinline__ V3<double> step_point(const StepQuadratic& q, V3<double> d, double s) {
-    return {__builtin_fma(s, d.x, q.px), __builtin_fma(s, d.y, q.py), __builtin_fma(s, d.z, 0.0)};
-}
-__device__ __forceinline__ V3<double> step_normal(V3<double> p, double c) {
-#pragma clang fp contract(off)
-    return {-c * p.x, -c * p.y, __builtin_fma(-c, p.z, 1.0)};
-}
-// refract_sphere: k = 1 - mu^2 (1 - cos^2 I) and, for k >= 0, mu d + (sqrt(k) - mu cos I) N
-__device__ __forceinline__ double refract_k(double mu, double cosI) {
-#pragma clang fp contract(off)
-    return __builtin_fma(-(mu * mu), __builtin_fma(-cosI, cosI, 1.0), 1.0);
-}
-__device__ __forceinline__ V3<double> refract_regular(V3<double> d, V3<double> N, double mu,
-                                                      double cosI, double sqrt_k) {
-#pragma clang fp contract(off)
-    const double g = __builtin_fma(-mu, cosI, sqrt_k);
-    return {__builtin_fma(N.x, g, d.x * mu), __builtin_fma(N.y, g, d.y * mu),
-            __builtin_fma(N.z, g, d.z * mu)};
-}
-
-// Hard failure mode: the step's operations run for every ray and one test of the four failure
-// conditions (backward, missed, no positive root, TIR; the precedence of the early returns of
-// the soft form) ends it, so a surface costs one exit of the surface loop instead of four. The
-// ray is updated in every case: the callers drop a ray whose step failed.
-template <bool kFast>
-__device__ __forceinline__ uint8_t surface_step_hard(RayT<double>& r, double c, double t,
-                                                     double nb, double mu) {
-#pragma clang fp contract(off)
-    const V3<double> d = r.d;
-    const StepQuadratic q = step_quadratic<kFast>(r, c, t);
-    const double denom = q.B + fsqrt<kFast>(q.D);
-    const double s = fdiv<kFast>(q.H, denom);
-    const V3<double> p = step_point(q, d, s);
-    const V3<double> N = step_normal(p, c);
-    const double cosI = dot_fma(d, N);
-    const double k = refract_k(mu, cosI);
-    r.opl = __builtin_fma(nb, q.s0 + s, r.opl);
-    r.p = p;
-    r.d = refract_regular(d, N, mu, cosI, fsqrt<kFast>(k));
-    const bool backward = !(d.z > 0.0), missed = q.D < 0.0 || !(denom > 0.0), tir = k < 0.0;
-    if (backward || missed || tir) [[unlikely]]
-        return backward ? uint8_t(MKO_STATUS_BACKWARD)
-               : missed ? uint8_t(MKO_STATUS_MISSED)
-                        : uint8_t(MKO_STATUS_TIR);
-    return MKO_STATUS_OK;
-}
-
-// Soft failure mode: a miss on a curved surface continues from the quadratic's vertex (s = B / c,
-// unit normal) and TIR continues along the surface tangent, each adding its penalty.
-template <bool kFast>
-__device__ __forceinline__ uint8_t surface_step_soft(RayT<double>& r, double c, double t,
-                                                     double nb, double mu, Soft& soft,
-                                                     uint8_t& branch) {
-#pragma clang fp contract(off)
-    const V3<double> d = r.d;
-    if (!(d.z > 0.0)) return MKO_STATUS_BACKWARD;
-    const StepQuadratic q = step_quadratic<kFast>(r, c, t);
-    double s;
-    bool missed = false;
-    if (q.D < 0.0) {
-        if (!(c > 0.0) && !(c < 0.0)) return MKO_STATUS_MISSED;
-        soft.add(-q.D, MKO_STATUS_SOFT_MISSED);
-        s = q.B / c;
-        missed = true;
-    } else {
-        const double denom = q.B + fsqrt<kFast>(q.D);
-        if (!(denom > 0.0)) return MKO_STATUS_MISSED;
-        s = fdiv<kFast>(q.H, denom);
-    }
-    const V3<double> p = step_point(q, d, s);
-    r.p = p;
-    r.opl = __builtin_fma(nb, q.s0 + s, r.opl);
-    V3<double> N = step_normal(p, c);
-    if (missed) {
-        const double w = 1.0 / __builtin_sqrt(dot_fma(N, N));
-        N = V3<double>{w * N.x, w * N.y, w * N.z};
-    }
-    const double cosI = dot_fma(d, N);
-    const double k = refract_k(mu, cosI);
-    if (k < 0.0) {
-        soft.add(-k, MKO_STATUS_SOFT_TIR);
-        const V3<double> tau{__builtin_fma(-cosI, N.x, d.x), __builtin_fma(-cosI, N.y, d.y),
-                             __builtin_fma(-cosI, N.z, d.z)};
-        const double w = 1.0 / __builtin_sqrt(dot_fma(tau, tau));
-        r.d = V3<double>{w * tau.x, w * tau.y, w * tau.z};
-        branch = uint8_t((missed ? kBranchSoftMissed : 0) | kBranchSoftTIR);
-        return MKO_STATUS_OK;
-    }
-    r.d = refract_regular(d, N, mu, cosI, fsqrt<kFast>(k));
-    branch = missed ? kBranchSoftMissed : kBranchRegular;
-    return MKO_STATUS_OK;
-}
-
-// One surface step (propagate_surface_local with transfer, sphere intersection and refraction).
-// c = effective curvature (0 for stop and plane), t = vertex distance from the previous surface,
-// nb = medium before, mu = nb / n_after. Returns a TraceStatus (Ok also for soft continuations,
-// whose kind goes to `soft` and whose branch bits go to `branch`). FP64 takes the spelled-out
-// forms above; FP32 (the prefilter) and df64 the general form below.
-template <bool kSoft, bool kFast = false, class R>
+// One surface step in df64 (propagate_surface_local with transfer, sphere intersection and
+// refraction; FP64 traces take momentum_step). c = effective curvature (0 for stop and plane), t =
+// vertex distance from the previous surface, nb = medium before, mu = nb / n_after. Returns a
+// TraceStatus (Ok also for soft continuations, whose kind goes to `soft` and whose branch bits go
+// to `branch`).
+template <bool kSoft, class R>
 __device__ __forceinline__ uint8_t surface_step(RayT<R>& r, R c, R t, R nb, R mu, Soft& soft,
                                                 uint8_t& branch) {
-    if constexpr (std::is_same_v<R, double>) {
-        if constexpr (kSoft) {
-            return surface_step_soft<kFast>(r, c, t, nb, mu, soft, branch);
-        } else {
-            branch = kBranchRegular;
-            return surface_step_hard<kFast>(r, c, t, nb, mu);
-        }
-    }
     const R zero = num<R>(0.0), one = num<R>(1.0);
     if (!(r.d.z > zero)) return MKO_STATUS_BACKWARD;
     // transfer_to_tangent_plane
     r.p.z -= t;
-    const R s0 = fdiv<kFast>(-r.p.z, r.d.z);
+    const R s0 = fdiv(-r.p.z, r.d.z);
     r.p.x += s0 * r.d.x;
     r.p.y += s0 * r.d.y;
     r.p.z = zero;
@@ -350,9 +192,9 @@ __device__ __forceinline__ uint8_t surface_step(RayT<R>& r, R c, R t, R nb, R mu
         s = B / c;
         missed = true;
     } else {
-        const R denom = B + fsqrt<kFast>(D);
+        const R denom = B + fsqrt(D);
         if (!(denom > zero)) return MKO_STATUS_MISSED;
-        s = fdiv<kFast>(H, denom);
+        s = fdiv(H, denom);
     }
     r.p = r.p + s * r.d;
     r.opl += nb * (s0 + s);
@@ -369,13 +211,13 @@ __device__ __forceinline__ uint8_t surface_step(RayT<R>& r, R c, R t, R nb, R mu
         branch = uint8_t((missed ? kBranchSoftMissed : 0) | kBranchSoftTIR);
         return MKO_STATUS_OK;
     }
-    r.d = mu * r.d + (fsqrt<kFast>(k) - mu * cosI) * N;
+    r.d = mu * r.d + (fsqrt(k) - mu * cosI) * N;
     branch = missed ? kBranchSoftMissed : kBranchRegular;
     return MKO_STATUS_OK;
 }
 
 // reference_sphere_step (kind last_surface) / image_sphere_step (image kinds).
-template <bool kSoft, bool kFast = false, class R>
+template <bool kSoft, class R>
 __device__ __forceinline__ uint8_t reference_step(RayT<R>& r, V3<R> M, R kappa, int kind,
                                                   R n_image, Soft& soft, uint8_t& branch) {
     const R zero = num<R>(0.0), one = num<R>(1.0);
@@ -394,11 +236,11 @@ __device__ __forceinline__ uint8_t reference_step(RayT<R>& r, V3<R> M, R kappa, 
             branch = kBranchSoftMissed;
             return MKO_STATUS_SOFT_MISSED;
         }
-        const R root = fsqrt<kFast>(disc);
+        const R root = fsqrt(disc);
         const bool real_image = M.z >= zero;
         const R denom = real_image ? b + root : b - root;
         if (!(real_image ? denom > zero : denom < zero)) return MKO_STATUS_MISSED;
-        const R s = fdiv<kFast>(g, denom);
+        const R s = fdiv(g, denom);
         r.p = r.p + s * r.d;
         r.opl += n_image * s;
         return MKO_STATUS_OK;
@@ -409,7 +251,7 @@ __device__ __forceinline__ uint8_t reference_step(RayT<R>& r, V3<R> M, R kappa, 
     R step;
     uint8_t st = MKO_STATUS_OK;
     if (disc >= zero) {
-        step = b - fdiv<kFast>(kappa * t, fsqrt<kFast>(disc) + one);
+        step = b - fdiv(kappa * t, fsqrt(disc) + one);
     } else if (kSoft && disc < zero) {
         step = b - kappa * t;
         st = MKO_STATUS_SOFT_MISSED;
@@ -617,139 +459,276 @@ __device__ __forceinline__ R reference_step_backward(V3<R> p, V3<R> d, V3<R> M, 
     return center_adj.z;
 }
 
-// ---- state reconstruction for the reverse sweep (no per-ray record) -----------------------------
+// ---- the trace and the reverse sweep in optical direction cosines ---------------------------------
 //
-// A regular (hard-mode) surface step maps the ray state on surface s (position in the frame of s,
-// direction in medium n_s) to the state on surface j = s + 1 and is invertible: refraction is
-// reversible (the tangential direction component scales by n_j / n_s, the normal component stays
-// positive), and the segment in gap s is recovered by intersecting the reversed ray with surface
-// s. inverse_step returns the state on s from the state (q, d1) on j; it is the forward transfer
-// and intersection of surface_step in the frame mirrored at z = 0 (z -> -z, curvature -> -c),
-// applied to the reversed ray, so it uses the same Spencer-Murty root.
-
-template <class R>
-struct RayState {
-    V3<R> p, d;
+// State on a surface: the point p in its frame and the momentum P = n d (n d the optical direction
+// cosines). Constants of the step from surface s - 1 to s, staged once per (variant, wavelength);
+// 64 bytes, read as 16-byte words by wave-uniform addresses.
+struct alignas(16) Step {
+    double c;   // effective curvature of surface s (0 for stop and plane)
+    double t;   // vertex distance from surface s - 1 to s
+    double ni2; // -1 / n^2, n the medium before the surface
+    double n2;  // n^2
+    double cn2; // c n^2
+    double dn2; // n_after^2 - n^2
+    double n;   // n_after
+    double cna; // c n_after^2
 };
 
-// State on surface s (curvature c_s, vertex t_s before surface j) from the state on surface j
-// (curvature c_j); n_s, n_j: media before and after surface j.
-__device__ __forceinline__ RayState<double> inverse_step(V3<double> q, V3<double> d1, double c_s,
-                                                         double t_s, double c_j, double n_s,
-                                                         double n_j) {
-    // inverse refraction at j: d = mu' d1 + (sqrt(k') - mu' cos') N, mu' = n_j / n_s
-    const V3<double> N{-c_j * q.x, -c_j * q.y, 1.0 - c_j * q.z};
-    const double mu = rev_div(n_j, n_s);
-    const double cosI = dot(d1, N);
-    const double k = 1.0 - mu * mu * (1.0 - cosI * cosI);
-    const V3<double> d = mu * d1 + (rev_sqrt(k) - mu * cosI) * N;
-    // reversed ray in the mirrored frame of s: origin (q.x, q.y, -(q.z + t_s)), direction
-    // (-d.x, -d.y, d.z); transfer to the tangent plane z = 0 and intersect curvature -c_s
-    const double s0 = rev_div(q.z + t_s, d.z);
-    const double x = q.x - s0 * d.x;
-    const double y = q.y - s0 * d.y;
-    const double cm = -c_s;
-    const double H = cm * (x * x + y * y);
-    const double B = d.z + cm * (x * d.x + y * d.y);
-    const double D = B * B - cm * H;
-    const double s = rev_div(H, B + rev_sqrt(D));
-    RayState<double> out;
-    out.p = V3<double>{x - s * d.x, y - s * d.y, -(s * d.z)};
-    out.d = d;
-    return out;
+// sqrt(x) and 1 / (2 sqrt(x)) for x > 0 (rev_sqrt_half_rcp without its branch); 0 for x = 0. A
+// negative or NaN x gives an unspecified value: the callers test x.
+__device__ __forceinline__ double sqrt_pos(double x, double& half_rcp) {
+    const double y = __builtin_amdgcn_rsq(__builtin_fmax(x, 0x1p-900));
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    half_rcp = h;
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ double sqrt_pos(double x) {
+    double h;
+    return sqrt_pos(x, h);
 }
 
-// One reverse step of a regular (hard-mode) ray for the fused kernel: reconstructs the state on
-// surface s from the state (q, d1) on surface j = s + 1 and propagates the adjoint (seed: OPL)
-// through the surface-j step, sharing the quantities both need. With N the unit normal at q:
-// d1 . N = sqrt(k) of the forward refraction, and the incidence cosine d . N equals the
-// intersection's sqrt(D) (B - c s = sqrt(D) on the sphere), so the reverse step needs two square
-// roots instead of four. mu = n_s / n_j, imu = n_j / n_s. Formulas: inverse_step above and
-// refracting_step_backward (adjoint_backward.hpp:119-241) specialised to the regular branch.
-// kIndex: also the adjoints of the indices before (n_s) and after the surface, added to nbb and
-// nab (glass variables), with 1 / n_after formed as mu / n_s.
-template <bool kIndex = false>
-__device__ __forceinline__ RayState<double> fused_step_backward(
-    V3<double> q, V3<double> d1, double c, double cs, double t, double n_s, double mu, double imu,
-    RayAdj<double>& adj, double& tb, double& cb_out, double* nbb = nullptr,
-    double* nab = nullptr) {
-    // reconstruction
-    const V3<double> N{-c * q.x, -c * q.y, 1.0 - c * q.z};
-    const double root_k = dot(d1, N);
-    const double kp = 1.0 - imu * imu * (1.0 - root_k * root_k);
-    double inv; // 1 / (2 cos_i)
-    const double cos_i = rev_sqrt_half_rcp(kp, inv); // = sqrt(D) of the forward intersection
-    const V3<double> d = imu * d1 + (cos_i - imu * root_k) * N;
-    const double rdz = rev_rcp(d.z);
-    const double s = q.z * rdz;
-    const double x = q.x - s * d.x;
-    const double y = q.y - s * d.y;
-    const double s0p = (q.z + t) * rdz;
-    const double xp = q.x - s0p * d.x;
-    const double yp = q.y - s0p * d.y;
-    const double cm = -cs;
-    const double Hp = cm * (xp * xp + yp * yp);
-    const double Bp = d.z + cm * (xp * d.x + yp * d.y);
-    const double Dp = Bp * Bp - cm * Hp;
-    const double sp = rev_div(Hp, Bp + rev_sqrt(Dp));
-    RayState<double> prev;
-    prev.p = V3<double>{xp - sp * d.x, yp - sp * d.y, -(sp * d.z)};
-    prev.d = d;
-    const double s0 = t * rdz + sp;
-    // adjoint of the step from s to j
-    const double rr = x * x + y * y;
-    const double xd = x * d.x + y * d.y;
-    const V3<double> qb_out = adj.p;
-    const V3<double> d1b = adj.d;
-    RayAdj<double> in{{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-    const double a = root_k - mu * cos_i;
-    in.d += mu * d1b;
-    V3<double> nb = a * d1b;
-    const double ab = dot(d1b, N);
-    const double kb = rev_div(ab, 2.0 * root_k);
-    const double cosb = -ab * mu + kb * 2.0 * mu * mu * cos_i;
-    in.d += cosb * N;
-    nb += cosb * d;
-    const V3<double> qb = qb_out + (-c) * nb;
-    double cb = -dot(q, nb);
-    double xb = qb.x;
-    double yb = qb.y;
-    const double sb = dot(qb, d) + n_s;
-    in.d += s * qb;
-    double s0b = n_s;
-    const double hb = sb * inv;
-    const double bb = -sb * s * 2.0 * inv;
-    cb += sb * s * s * inv;
-    cb += hb * rr;
-    xb += hb * 2.0 * c * x;
-    yb += hb * 2.0 * c * y;
-    in.d.z += bb;
-    cb += -bb * xd;
-    xb += -bb * c * d.x;
-    yb += -bb * c * d.y;
-    in.d.x += -bb * c * x;
-    in.d.y += -bb * c * y;
-    in.p.x += xb;
-    in.p.y += yb;
-    s0b += xb * d.x + yb * d.y;
-    in.d.x += xb * s0;
-    in.d.y += yb * s0;
-    const double qq = s0b * rdz;
-    tb += qq;
-    in.p.z += -qq;
-    in.d.z += -qq * s0;
-    cb_out += cb;
-    if constexpr (kIndex) {
-        // mu = n_s / n_after: d(OPL)/d mu through the refraction, then the chain to both indices;
-        // the segment in medium n_s has length s0 + s
-        const double sin2 = 1.0 - cos_i * cos_i;
-        const double mub = dot(d1b, d) - ab * cos_i - kb * 2.0 * mu * sin2;
-        const double rna = rev_div(mu, n_s);
-        *nbb += mub * rna + (s0 + s);
-        *nab += -mub * mu * rna;
+// The line through Q (in the frame of surface s) along +-P: its point nearest the vertex, where
+// Q0 . P = 0, then the sphere from there: with H = c |Q0|^2 - 2 Q0_z the incidence term
+// (P . N)^2 = D = P_z^2 - c n^2 H, the distance (in units of P) to the sphere is H / (P_z +
+// sqrt(D)), without cancellation for P_z > 0, and P . N = sqrt(D) there (N the unit normal towards
+// +z). No division by d_z, no product of direction and normal: one division and one root.
+struct StepFoot {
+    double l0, x, y, z, H, E, D;
+};
+__device__ __forceinline__ StepFoot step_foot(V3<double> Q, V3<double> P, double c, double ni2,
+                                              double cn2) {
+#pragma clang fp contract(off)
+    StepFoot f;
+    f.l0 = __builtin_fma(Q.z, P.z, __builtin_fma(Q.y, P.y, Q.x * P.x)) * ni2;
+    f.x = __builtin_fma(f.l0, P.x, Q.x);
+    f.y = __builtin_fma(f.l0, P.y, Q.y);
+    f.z = __builtin_fma(f.l0, P.z, Q.z);
+    const double q2 = __builtin_fma(f.z, f.z, __builtin_fma(f.y, f.y, f.x * f.x));
+    f.H = __builtin_fma(c, q2, -(f.z + f.z));
+    f.E = P.z * P.z;
+    f.D = __builtin_fma(-cn2, f.H, f.E);
+    return f;
+}
+
+// One surface step in hard failure mode: (p, P, opl) from surface s - 1 to s. Every operation runs
+// for every ray and one test ends a failed one (precedence: backward, missed, TIR; its state is
+// then of no use). Missed: no intersection (D < 0), or the ray meets the tangent plane beyond the
+// sphere's visible cap (d_z - c (x d_x + y d_y) <= 0 there, the reference's intersect_sphere),
+// which is P_z^2 + c n^2 Q0_z <= 0. Products and sums are spelled out, so that every kernel that
+// inlines the step computes the same bits. a: P . N at the surface.
+__device__ __forceinline__ uint8_t momentum_step(V3<double>& p, V3<double>& P, double& opl,
+                                                 const Step& k, double& a) {
+#pragma clang fp contract(off)
+    const StepFoot f = step_foot(V3<double>{p.x, p.y, p.z - k.t}, P, k.c, k.ni2, k.cn2);
+    const bool backward = !(P.z > 0.0);
+    a = sqrt_pos(f.D);
+    const double lam = rev_div(f.H, P.z + a);
+    p = V3<double>{__builtin_fma(lam, P.x, f.x), __builtin_fma(lam, P.y, f.y),
+                   __builtin_fma(lam, P.z, f.z)};
+    opl = __builtin_fma(k.n2, f.l0 + lam, opl);
+    const double k2 = f.D + k.dn2;
+    const double g = sqrt_pos(k2) - a;
+    const double cg = k.c * g;
+    const double pz = P.z + g;
+    P = V3<double>{__builtin_fma(-cg, p.x, P.x), __builtin_fma(-cg, p.y, P.y),
+                   __builtin_fma(-cg, p.z, pz)};
+    const bool missed = !(f.D >= 0.0) || !(__builtin_fma(k.cn2, f.z, f.E) > 0.0);
+    if (backward || missed || k2 < 0.0) [[unlikely]]
+        return backward ? uint8_t(MKO_STATUS_BACKWARD)
+               : missed ? uint8_t(MKO_STATUS_MISSED)
+                        : uint8_t(MKO_STATUS_TIR);
+    return MKO_STATUS_OK;
+}
+
+// Soft continuations of a step (rare): p on the surface or, after a miss, nearest the sphere's
+// centre; a = P . N and k2 = a^2 + dn2 of a hit. Direction space: unit normal after a miss, TIR
+// continues along the surface tangent.
+__device__ __forceinline__ void soft_refract(V3<double> p, V3<double>& P, const Step& k, double nb,
+                                             double a, double k2, bool missed, Soft& soft,
+                                             uint8_t& branch) {
+#pragma clang fp contract(off)
+    V3<double> N{-k.c * p.x, -k.c * p.y, __builtin_fma(-k.c, p.z, 1.0)};
+    const V3<double> d{P.x / nb, P.y / nb, P.z / nb};
+    const double mu = nb / k.n;
+    double cosI = a / nb, kk = k2 / (k.n * k.n);
+    if (missed) {
+        const double w = 1.0 / __builtin_sqrt(N.x * N.x + N.y * N.y + N.z * N.z);
+        N = V3<double>{w * N.x, w * N.y, w * N.z};
+        cosI = d.x * N.x + d.y * N.y + d.z * N.z;
+        kk = 1.0 - mu * mu * (1.0 - cosI * cosI);
     }
-    adj = in;
-    return prev;
+    branch = missed ? kBranchSoftMissed : kBranchRegular;
+    V3<double> e;
+    if (kk < 0.0) {
+        soft.add(-kk, MKO_STATUS_SOFT_TIR);
+        branch = uint8_t(branch | kBranchSoftTIR);
+        e = V3<double>{d.x - cosI * N.x, d.y - cosI * N.y, d.z - cosI * N.z};
+        const double w = 1.0 / __builtin_sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
+        e = V3<double>{w * e.x, w * e.y, w * e.z};
+    } else {
+        const double g = __builtin_sqrt(kk) - mu * cosI;
+        e = V3<double>{mu * d.x + g * N.x, mu * d.y + g * N.y, mu * d.z + g * N.z};
+    }
+    P = V3<double>{k.n * e.x, k.n * e.y, k.n * e.z};
+}
+
+// The step in soft failure mode (nb: the medium before): a miss on a curved surface continues from
+// the line's point nearest the sphere's centre (the vertex of the intersection's quadratic), TIR
+// along the surface, each adding its penalty; a regular ray takes momentum_step's operations.
+__device__ __forceinline__ uint8_t momentum_step_soft(V3<double>& p, V3<double>& P, double& opl,
+                                                      const Step& k, double nb, double& a,
+                                                      Soft& soft, uint8_t& branch) {
+#pragma clang fp contract(off)
+    if (!(P.z > 0.0)) return MKO_STATUS_BACKWARD;
+    const StepFoot f = step_foot(V3<double>{p.x, p.y, p.z - k.t}, P, k.c, k.ni2, k.cn2);
+    double lam;
+    const bool missed = f.D < 0.0;
+    a = 0.0;
+    if (missed) {
+        if (!(k.c > 0.0) && !(k.c < 0.0)) return MKO_STATUS_MISSED;
+        soft.add(f.D * k.ni2, MKO_STATUS_SOFT_MISSED);
+        lam = P.z / k.cn2;
+    } else {
+        a = sqrt_pos(f.D);
+        if (!(f.D >= 0.0) || !(__builtin_fma(k.cn2, f.z, f.E) > 0.0)) return MKO_STATUS_MISSED;
+        lam = rev_div(f.H, P.z + a);
+    }
+    p = V3<double>{__builtin_fma(lam, P.x, f.x), __builtin_fma(lam, P.y, f.y),
+                   __builtin_fma(lam, P.z, f.z)};
+    opl = __builtin_fma(k.n2, f.l0 + lam, opl);
+    const double k2 = f.D + k.dn2;
+    if (missed || k2 < 0.0) [[unlikely]] {
+        soft_refract(p, P, k, nb, a, k2, missed, soft, branch);
+        return MKO_STATUS_OK;
+    }
+    const double g = sqrt_pos(k2) - a;
+    const double cg = k.c * g;
+    const double pz = P.z + g;
+    P = V3<double>{__builtin_fma(-cg, p.x, P.x), __builtin_fma(-cg, p.y, P.y),
+                   __builtin_fma(-cg, p.z, pz)};
+    branch = kBranchRegular;
+    return MKO_STATUS_OK;
+}
+
+// Reverse sweep of one regular ray (no soft continuation) from its state on the last surface.
+//
+// By Fermat's principle the optical path to the reference sphere changes, for a change of a
+// parameter, by the change of the path's own pieces at fixed points of incidence, plus P . dE for
+// the displacement dE of the ray's end on the reference sphere, which is not zero where the ray
+// leaves the sphere's normal. That second part is a linear functional of the ray; pulled back
+// through the system it is carried by one neighbouring ray (dq, dP), because the map of rays is
+// symplectic. So with K the change of the local path as a function of the ray,
+//     d(OPL)/d(theta) = K + dK along (dq, dP):
+//   thickness t_s:  K = P_z in the gap
+//   curvature c_j:  K = (P . N - P' . N) |q|^2 / 2 (the surface moves along N by |q|^2 / 2)
+//   index n_s:      K = the length of the ray in the medium
+// The sweep traces the ray backwards (no record of its states) and the neighbouring ray with it.
+// A general adjoint state (six components through every operation of the step) took 162 vector
+// instructions per surface, this form about 90. Equivalent to backward_ray's sums
+// (adjoint_backward.hpp:119-241), checked against them and against 64-bit tangents.
+struct SweepState {
+    V3<double> q, P, dq, dP, N;
+    double a, ha; // P . N and 1 / (2 P . N)
+};
+
+// The neighbouring ray of a linear functional A . dq + B . dP of the ray (p, P) on a surface with
+// normal N: dq = B modulo P on the tangent plane, dP = -A modulo N and normal to P.
+__device__ __forceinline__ SweepState sweep_start(V3<double> p, V3<double> P, V3<double> A,
+                                                  V3<double> B, double c) {
+    SweepState w;
+    w.q = p;
+    w.P = P;
+    w.N = V3<double>{-c * p.x, -c * p.y, 1.0 - c * p.z};
+    w.a = dot(P, w.N);
+    const double ra = rev_rcp(w.a);
+    w.ha = 0.5 * ra;
+    const double mu = dot(w.N, B) * ra, nu = dot(P, A) * ra;
+    w.dq = V3<double>{B.x - mu * P.x, B.y - mu * P.y, B.z - mu * P.z};
+    w.dP = V3<double>{nu * w.N.x - A.x, nu * w.N.y - A.y, nu * w.N.z - A.z};
+    return w;
+}
+
+// Backwards through the refraction at surface j (k: its step): P and dP become those before the
+// surface; returns the curvature gradient. On entry a = P' . N.
+__device__ __forceinline__ double sweep_refract(SweepState& w, const Step& k) {
+    double h;
+    const double a = sqrt_pos(__builtin_fma(w.a, w.a, -k.dn2), h);
+    const double g = w.a - a;
+    const double u = dot(w.dP, w.N) - k.c * dot(w.P, w.dq); // change of P' . N
+    const double dg = u * g * (h + h);                      // minus the change of g
+    const double cg = k.c * g;
+    w.P = V3<double>{w.P.x - g * w.N.x, w.P.y - g * w.N.y, w.P.z - g * w.N.z};
+    w.dP = V3<double>{w.dP.x + (dg * w.N.x + cg * w.dq.x), w.dP.y + (dg * w.N.y + cg * w.dq.y),
+                      w.dP.z + (dg * w.N.z + cg * w.dq.z)};
+    const double r = 0.5 * dot(w.q, w.q);
+    return dg * r - g * (r + dot(w.q, w.dq));
+}
+
+// Backwards through the gap between surface s = j - 1 (curvature c, cna = c n^2) and j (k: its
+// step): the state and the neighbouring ray on surface s. kIndex: length is the gradient with
+// respect to the gap's index.
+template <bool kIndex>
+__device__ __forceinline__ void sweep_transfer(SweepState& w, const Step& k, double c, double cna,
+                                               double n, double& length) {
+    const StepFoot f = step_foot(V3<double>{w.q.x, w.q.y, w.q.z + k.t}, w.P, c, k.ni2, cna);
+    w.a = sqrt_pos(f.D, w.ha);
+    const double lam = rev_div(f.H, w.P.z + w.a);
+    w.q = V3<double>{f.x + lam * w.P.x, f.y + lam * w.P.y, f.z + lam * w.P.z};
+    const double back = f.l0 + lam; // q = Q + back P
+    w.N = V3<double>{-c * w.q.x, -c * w.q.y, 1.0 - c * w.q.z};
+    const double before = kIndex ? dot(w.P, w.dq) : 0.0;
+    w.dq = V3<double>{w.dq.x + back * w.dP.x, w.dq.y + back * w.dP.y, w.dq.z + back * w.dP.z};
+    const double mu = dot(w.N, w.dq) * (w.ha + w.ha);
+    w.dq = V3<double>{w.dq.x - mu * w.P.x, w.dq.y - mu * w.P.y, w.dq.z - mu * w.P.z};
+    if constexpr (kIndex) // n |back| + (P . dq_j - P . dq_s) / n, 1 / n = -n ni2
+        length = -n * (back + k.ni2 * (before - dot(w.P, w.dq)));
+}
+
+// The functional of a regular ray at the reference sphere (reference_step): V = n step(p, d), A =
+// dV/dp + P, B = dV/dP, and with it the sweep's start; mz: the gradient with respect to M_z, step:
+// the path's length to the sphere.
+__device__ __forceinline__ SweepState sweep_reference(V3<double> p, V3<double> d, V3<double> M,
+                                                      double kappa, int kind, double n,
+                                                      double c_last, double& mz, double& step) {
+    const V3<double> q = p - M;
+    const double b = -dot(q, d);
+    const V3<double> P{n * d.x, n * d.y, n * d.z};
+    V3<double> A, B;
+    if (kind == MKO_REF_LAST_SURFACE) {
+        const double g = dot(p, p - 2.0 * M);
+        double h;
+        const double root = rev_sqrt_half_rcp(b * b - g, h);
+        const double sigma = M.z >= 0.0 ? 1.0 : -1.0;
+        step = rev_div(g, b + sigma * root);
+        const double gb = n * sigma * h;       // dV/dg
+        const double bb = -2.0 * gb * step;    // dV/db
+        const double wq = 2.0 * gb;
+        A = V3<double>{P.x - bb * d.x + wq * q.x, P.y - bb * d.y + wq * q.y,
+                       P.z - bb * d.z + wq * q.z};
+        const double rb = -rev_div(bb, n);
+        B = V3<double>{rb * q.x, rb * q.y, rb * q.z};
+        mz = bb * d.z - wq * p.z;
+    } else {
+        const V3<double> cr = cross(q, d);
+        const double t = -dot(cr, cr);
+        double h;
+        const double u = rev_sqrt_half_rcp(1.0 + kappa * kappa * t, h);
+        step = b - kappa * rev_div(t, u + 1.0);
+        const double tb = -n * kappa * h; // dV/dt
+        const V3<double> dc = cross(d, cr), cq = cross(cr, q);
+        const V3<double> pb{-n * d.x - 2.0 * tb * dc.x, -n * d.y - 2.0 * tb * dc.y,
+                            -n * d.z - 2.0 * tb * dc.z};
+        A = pb + P;
+        const double rn = rev_rcp(n);
+        B = V3<double>{-q.x - 2.0 * tb * cq.x * rn, -q.y - 2.0 * tb * cq.y * rn,
+                       -q.z - 2.0 * tb * cq.z * rn};
+        mz = -pb.z;
+    }
+    return sweep_start(p, P, A, B, c_last);
 }
 
 } // namespace mkod
