@@ -87,6 +87,9 @@ struct ParamMap {
     int glass;
     int32_t glass_col[MKO_MAX_SURFACES][3];
     double omega[kMaxWavelengths];
+    // columns that no ray's sweep reaches (bit p): the curvature of a stop or plane, the index of
+    // the medium before the first surface
+    uint64_t unswept[2];
 };
 
 // ---- tuple geometry ------------------------------------------------------------------------
@@ -1633,7 +1636,7 @@ __global__ __launch_bounds__(kBlock) void fd_difference_kernel(
 
 // ---- ADJOINT Jacobian -----------------------------------------------------------------------
 
-// Writes one seed's per-ray parameter adjoints into J rows: value * factor at column p, row.
+// Writes one ray's parameter gradients into its J row: value * factor at column p.
 struct RowSink {
     double* col0; // J of the variant
     int64_t rows; // R
@@ -1644,7 +1647,8 @@ struct RowSink {
     }
 };
 
-// backward_ray (adjoint_backward.hpp:496-580) over the record of a ray.
+// backward_ray (adjoint_backward.hpp:496-580) over the record of a ray with a soft continuation.
+// The thickness columns less the common part n (sweep_ray's kFine form).
 template <class Sink>
 __device__ __forceinline__ void backward_ray(const TraceParams& P, const Step* L,
                                              const ParamMap& map, const Record& rec,
@@ -1684,7 +1688,7 @@ __device__ __forceinline__ void backward_ray(const TraceParams& P, const Step* L
                                                    next_branch, seed_opl, seed_pen, adj, tb, cb,
                                                    nbb, nab);
             if ((P.sphere_mask >> j) & 1ull) sink.write(map.curv_col[j], cb);
-            sink.write(map.thick_col[s], tb);
+            sink.write(map.thick_col[s], tb - seed_opl * L[s].n);
             index_sink(j, nab + n_carry);
             n_carry = nbb;
         }
@@ -1692,24 +1696,89 @@ __device__ __forceinline__ void backward_ray(const TraceParams& P, const Step* L
     }
 }
 
-// One workgroup per (variant = run, tuple). Raw per-ray gradients go straight into the
-// column-major J of the variant (J[v][p][row]); after the tuple's piston reduction the
-// workgroup projects its rows in place: J(k,p) = s sqrt(W_k) (g_k - gbar_p) for rays in the
-// piston, 0 otherwise (adjoint_jacobian.cpp:462-479). Penalty rows (soft mode) get
-// pscale sqrt(W_k) times the penalty gradient. r0 rows and the status are written as by
-// RESIDUALS.
-template <bool kSoft, int kRpl>
+// A soft ray's second trace, with its record, and the sweep over it.
+template <class Sink>
+__device__ __forceinline__ void soft_backward(const TraceParams& P, const Step* L,
+                                           const ParamMap& map, const Ray& start, V3<double> M,
+                                           double kappa, double seed_opl, double seed_pen,
+                                           const Sink& sink, int l) {
+    Record rec;
+    rec.count = 0;
+    rec.image_branch = 0;
+    Ray r = start;
+    Soft soft{0.0, MKO_STATUS_OK};
+    const uint8_t st = trace_ray<true>(P, L, r, M, kappa, soft, rec);
+    const bool reached = mkod::in_piston(st);
+    backward_ray(P, L, map, rec, reached, M, kappa, reached ? seed_opl : 0.0, seed_pen, sink, l);
+}
+
+// The gradients of a regular ray (backward_ray, adjoint_backward.hpp:496-580, with seed 1 for the
+// optical path) from its state (p, d) on the last surface, by mkod's reverse sweep. kGlass: the
+// index gradients as well, into the glass variables' columns of each medium
+// (dn/d(n0, nu1, nu2) = 1, w_l, w_l^2). kFine: a thickness gradient P_z + dP_z is given less its
+// common part n, as dP_z - (P_x^2 + P_y^2) / (n + P_z): the projections that follow remove what
+// the rays of a tuple have in common (1e4 to 1e5 times the variation for weak beams), and the
+// variation then keeps its digits.
+template <bool kGlass, bool kFine, class Sink>
+__device__ __forceinline__ void sweep_ray(const TraceParams& P, const Step* L, const ParamMap& map,
+                                          V3<double> p, V3<double> d, V3<double> M, double kappa,
+                                          const Sink& sink, int l) {
+    const int S = P.S;
+    double mz, length;
+    mkod::SweepState w = mkod::sweep_reference(p, d, M, kappa, P.ref_kind, L[S - 1].n, L[S - 1].c,
+                                               mz, length);
+    sink.write(map.thick_col[S - 1], mz);
+    if constexpr (kGlass) length -= mkod::rev_div(mkod::dot(w.P, w.dq), L[S - 1].n);
+    for (int j = S - 1;; --j) {
+        if constexpr (kGlass) {
+            const double wl = map.omega[l];
+            sink.write(map.glass_col[j][0], length);
+            sink.write(map.glass_col[j][1], length * wl);
+            sink.write(map.glass_col[j][2], length * (wl * wl));
+        }
+        const double cb = mkod::sweep_refract(w, L[j]);
+        if ((P.sphere_mask >> j) & 1ull) sink.write(map.curv_col[j], cb);
+        if (kFine) {
+            const double n = L[j - 1].n;
+            const double t2 = w.P.x * w.P.x + w.P.y * w.P.y;
+            sink.write(map.thick_col[j - 1], w.dP.z - mkod::rev_div(t2, n + w.P.z));
+        } else {
+            sink.write(map.thick_col[j - 1], w.P.z + w.dP.z);
+        }
+        if (j == 1) break;
+        mkod::sweep_transfer<kGlass>(w, L[j], L[j - 1].c, L[j - 1].cna, L[j - 1].n, length);
+    }
+}
+
+// Stored Jacobian: one workgroup of up to 4 waves per (variant = run, tuple), kRpl rays per lane.
+// Each ray is traced and swept backwards at once (no record of its states in memory: only a ray
+// with a soft continuation is traced again for its record), its raw gradients going straight into
+// the column-major J (J[v][p][row]: a wave writes 512 contiguous bytes per column). After the
+// tuple's piston sums the waves take the columns in turn, a column's rays in registers: weighted
+// mean, then J(k,p) = s sqrt(W_k) (g_k - gbar_p) for rays in the piston, 0 otherwise
+// (adjoint_jacobian.cpp:462-479), one read and one write of J and no barrier per column. Penalty
+// rows (soft mode) get pscale sqrt(W_k) times the penalty gradient. r0 rows and the status are
+// written as by RESIDUALS. What bounds it: the vector ALU (a trace and a sweep, about 4000
+// instructions per ray at 25 surfaces) and 3 x 8 P bytes of J per ray: 0.36 ms for 64 runs x 17920
+// rays x 48 variables (1.24 ms with a record of the states in private memory, a pass that cleared
+// J and two passes and four barriers per column for the projection).
+// wr: weight and s sqrt(W) of each ray of the tuple (0, 0 outside the piston).
+template <bool kSoft, bool kGlass, int kRpl>
 __global__ __launch_bounds__(kBlock) void adjoint_kernel(TraceParams P, ParamMap map, double* J,
                                                          double* r0, uint8_t* status) {
-    __shared__ Step steps[MKO_MAX_SURFACES + 1];
-    const Step* L = steps;
+    extern __shared__ __align__(16) unsigned char adj_lds[];
     __shared__ SampleTable ST;
-    __shared__ double red[kWaves];
+    __shared__ double red[2][kWaves];
     if (P.live && int(blockIdx.x) / P.T >= *P.live) return;
     const Tuple t = tuple_of(P, blockIdx.x);
+    Step* steps = reinterpret_cast<Step*>(adj_lds);
+    double2* wr = reinterpret_cast<double2*>(adj_lds + size_t(P.S + 1) * sizeof(Step));
+    const Step* L = steps;
     stage_samples(P, t, ST);
     stage_steps(P, t.v, t.l, steps);
     __syncthreads();
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int threads = int(blockDim.x), waves = threads >> 6;
     const size_t vf = size_t(t.v) * P.F + t.f;
     const double a = P.pupil_radius[t.v];
     double sin_t, cos_t;
@@ -1723,46 +1792,60 @@ __global__ __launch_bounds__(kBlock) void adjoint_kernel(TraceParams P, ParamMap
     uint8_t st[kRpl];
     double pen[kRpl];
     double sw = 0.0, swo = 0.0;
-    Record rec;
 #pragma unroll
     for (int i = 0; i < kRpl; ++i) {
-        const int k = threadIdx.x + i * kBlock;
+        const int k = tid + i * threads;
         st[i] = MKO_STATUS_UNSUPPORTED;
         opl[i] = 0.0;
         pen[i] = 0.0;
         if (k >= t.n) continue;
         const int64_t row = t.offset + k;
-        for (int p = 0; p < map.P; ++p) {
-            col0[int64_t(p) * R + row] = 0.0;
-            if (kSoft) col0[int64_t(p) * R + P.rays + row] = 0.0;
-        }
         const Sample s = sample_at(P, t, ST, k);
-        Ray r = source_ray(P, t, s, a, sin_t, cos_t, L[0].n);
+        const Ray start = source_ray(P, t, s, a, sin_t, cos_t, L[0].n);
+        Ray r = start;
         Soft soft{0.0, MKO_STATUS_OK};
-        rec.count = 0;
-        rec.image_branch = 0;
-        st[i] = trace_ray<kSoft>(P, L, r, M, kappa, soft, rec);
-        opl[i] = r.opl;
+        LastState last{};
+        st[i] = trace_ray<kSoft>(P, L, r, M, kappa, soft, last);
         pen[i] = soft.penalty;
         const bool reached = mkod::in_piston(st[i]);
         if (reached) {
+            opl[i] = r.opl;
             sw += s.weight;
             swo += s.weight * r.opl;
-            backward_ray(P, L, map, rec, true, M, kappa, 1.0, 0.0,
-                                     RowSink{col0, R, row, 1.0}, t.l);
         }
-        if (kSoft && soft.first != MKO_STATUS_OK) {
-            backward_ray(P, L, map, rec, reached, M, kappa, 0.0, 1.0,
-                                     RowSink{col0, R, P.rays + row, t.pscale * s.rootw}, t.l);
+        wr[k] = reached ? double2{s.weight, t.scale * s.rootw} : double2{0.0, 0.0};
+        if (st[i] == MKO_STATUS_OK)
+            sweep_ray<kGlass, true>(P, L, map, last.p, last.d, M, kappa,
+                                    RowSink{col0, R, row, 1.0}, t.l);
+        if constexpr (kSoft) {
+            // penalty rows: zero but for a ray with a continuation, whose sweep may end early
+            for (int p = 0; p < map.P; ++p) col0[int64_t(p) * R + P.rays + row] = 0.0;
+            if (soft.first != MKO_STATUS_OK) {
+                if (reached)
+                    soft_backward(P, L, map, start, M, kappa, 1.0, 0.0,
+                                  RowSink{col0, R, row, 1.0}, t.l);
+                soft_backward(P, L, map, start, M, kappa, 0.0, 1.0,
+                              RowSink{col0, R, P.rays + row, t.pscale * s.rootw}, t.l);
+            }
         }
     }
-    const double w_ok = block_sum(sw, red);
-    const double sum = block_sum(swo, red);
+    sw = wave_sum(sw);
+    swo = wave_sum(swo);
+    if (lane == 0) {
+        red[0][wave] = sw;
+        red[1][wave] = swo;
+    }
+    __syncthreads(); // also publishes the raw gradients to the workgroup's other waves
+    double w_ok = red[0][0], sum = red[1][0];
+    for (int w = 1; w < waves; ++w) {
+        w_ok += red[0][w];
+        sum += red[1][w];
+    }
     const bool valid = w_ok > 0.0;
     const double piston = valid ? sum / w_ok : 0.0;
 #pragma unroll
     for (int i = 0; i < kRpl; ++i) {
-        const int k = threadIdx.x + i * kBlock;
+        const int k = tid + i * threads;
         if (k >= t.n) continue;
         const Sample s = sample_at(P, t, ST, k);
         const bool ok = valid && mkod::in_piston(st[i]);
@@ -1777,100 +1860,205 @@ __global__ __launch_bounds__(kBlock) void adjoint_kernel(TraceParams P, ParamMap
         }
         if (status) status[size_t(t.v) * P.rays + row] = st[i];
     }
-    __threadfence_block();
-    __syncthreads();
-    // piston projection, one column at a time (sums in FP64, fixed order)
-    for (int p = 0; p < map.P; ++p) {
+    // piston projection: a wave per column, 64 rays at a time in registers (sums in FP64, fixed
+    // order); columns that no sweep writes (map.unswept) are zero
+    constexpr int kSlots = 4 * kRpl; // 64 lanes, up to 256 kRpl rays
+    for (int p = wave; p < map.P; p += waves) {
         double* col = col0 + int64_t(p) * R + t.offset;
-        double part = 0.0;
+        const bool swept = !((map.unswept[p >> 6] >> (p & 63)) & 1ull);
+        double g[kSlots], part = 0.0;
 #pragma unroll
-        for (int i = 0; i < kRpl; ++i) {
-            const int k = threadIdx.x + i * kBlock;
-            if (k < t.n && mkod::in_piston(st[i])) part += sample_at(P, t, ST, k).weight * col[k];
+        for (int i = 0; i < kSlots; ++i) {
+            const int k = lane + 64 * i;
+            g[i] = 0.0;
+            if (k < t.n) {
+                const double w = wr[k].x;
+                if (swept && w != 0.0) g[i] = col[k];
+                part += w * g[i];
+            }
         }
-        const double mean = valid ? block_sum(part, red) / w_ok : 0.0;
+        const double mean = valid ? wave_sum(part) / w_ok : 0.0;
 #pragma unroll
-        for (int i = 0; i < kRpl; ++i) {
-            const int k = threadIdx.x + i * kBlock;
-            if (k >= t.n) continue;
-            const Sample s = sample_at(P, t, ST, k);
-            const bool ok = valid && mkod::in_piston(st[i]);
-            col[k] = ok ? t.scale * s.rootw * (col[k] - mean) : 0.0;
+        for (int i = 0; i < kSlots; ++i) {
+            const int k = lane + 64 * i;
+            if (k < t.n) col[k] = wr[k].y * (g[i] - mean);
         }
     }
 }
 
 // ---- vector-Jacobian product J^T v without J ---------------------------------------------
-
-// Sink of the VJP sweep: lane `lane` adds each column's value into its own slot of acc [P][64]
-// (a column is written once per ray and sweep; the lane's rays follow one another).
-struct AccSink {
-    double* acc;
-    int lane;
-    __device__ __forceinline__ void write(int p, double value) const {
-        if (p >= 0) acc[p * 64 + lane] += value;
-    }
-};
-
-// J^T v of one (variant = run, tuple), one wave per tuple, the tuple's rays 64 at a time. The
-// reverse sweep is linear in its seeds (ray_gradient_rows, ray_jacobian.hpp:93), so each ray
-// runs it once with
+//
+// J^T v of one (variant = run, tuple) per workgroup. The sweep is linear in its seeds
+// (ray_gradient_rows, ray_jacobian.hpp:93), so each ray runs it once with
 //   seed_opl = s (v_k sqrt(W_k) - W_k m),  m = sum_j v_j sqrt(W_j) / W_ok (rays in the piston),
 //   seed_pen = pscale sqrt(W_k) u_k      (soft mode, rays with a failure),
 // v and u being the cotangents of the ray's residual and penalty rows: sum_k v_k J(k, p) with
 // J(k, p) = s sqrt(W_k) (g_kp - gbar_p) equals sum_k g_kp s (v_k sqrt(W_k) - W_k m), so neither
-// J nor the piston-projected columns are formed. A first pass traces the tuple for W_ok and the
-// sum behind m. part[tuple][p]: the tuple's share, lanes summed in a fixed tree.
-template <bool kSoft>
-__global__ __launch_bounds__(64) void vjp_kernel(TraceParams P, ParamMap map, const double* grad,
-                                                 int64_t gstride, double* part) {
-    extern __shared__ double acc[]; // [P][64]
-    __shared__ Step steps[MKO_MAX_SURFACES + 1];
-    const Step* L = steps;
+// J nor the piston-projected columns are formed. The seeds sum to zero, so the common part n of a
+// thickness column drops out and is left away (kFine). part[tuple][p]: the tuple's share.
+
+// Hard failure mode: up to 4 waves per tuple, kRpl rays per lane. A first pass traces the rays,
+// for W_ok and the sum behind m, and keeps their last states in registers for the sweeps. A
+// column's products are summed over groups of 4 lanes by one matrix instruction with a vector of
+// ones (v_mfma_f64_4x4x4_4b: lane l holds the sum of the group l / 4 in all four lanes) and added
+// to the wave's own 16 sums of the column: 128 bytes of LDS per column and wave, a quarter of a
+// slot per lane, so 5 workgroups fit a CU at 48 variables (0.42 ms for 128 runs x 17920 rays; 1.99
+// ms with two traces, a record in private memory and a slot per lane: 1.5 waves per SIMD). Every lane of a wave runs the sweep
+// (the matrix instruction takes all lanes); those without a regular ray give zeros.
+struct GroupSink {
+    double* acc; // [P][16] of this wave
+    int slot;    // lane / 4
+    double beta;
+    __device__ __forceinline__ void write(int p, double value) const {
+        if (p < 0) return;
+        const double x = beta != 0.0 ? beta * value : 0.0;
+        const double sum = __builtin_amdgcn_mfma_f64_4x4x4f64(x, 1.0, 0.0, 0, 0, 0);
+        acc[p * 16 + slot] += sum; // the group's four lanes write the same value
+    }
+};
+
+template <bool kGlass, int kRpl>
+__global__ __launch_bounds__(kBlock) void vjp_kernel(TraceParams P, ParamMap map,
+                                                     const double* grad, int64_t gstride,
+                                                     double* part) {
+    extern __shared__ __align__(16) unsigned char vjp_lds[];
+    __shared__ SampleTable ST;
+    __shared__ double red[2][kWaves];
     const Tuple t = tuple_of(P, blockIdx.x);
+    Step* steps = reinterpret_cast<Step*>(vjp_lds);
+    const Step* L = steps;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int threads = int(blockDim.x), waves = threads >> 6;
+    double* acc0 = reinterpret_cast<double*>(vjp_lds + size_t(P.S + 1) * sizeof(Step));
+    double* acc = acc0 + size_t(wave) * map.P * 16;
+    stage_samples(P, t, ST);
     stage_steps(P, t.v, t.l, steps);
+    for (int e = lane; e < map.P * 16; e += 64) acc[e] = 0.0;
     __syncthreads();
-    const int lane = threadIdx.x;
-    for (int p = 0; p < map.P; ++p) acc[p * 64 + lane] = 0.0;
     const size_t vf = size_t(t.v) * P.F + t.f;
     const double a = P.pupil_radius[t.v];
     double sin_t, cos_t;
     sincos(P.field_angle[vf], &sin_t, &cos_t);
     const V3<double> M{0.0, P.field_target[vf], L[P.S].t};
     const double kappa = P.ref_kind != MKO_REF_LAST_SURFACE ? P.reference_curvature[vf] : 0.0;
-    const double* gv = grad + size_t(t.v) * size_t(gstride);
+    const double* gv = grad + size_t(t.v) * size_t(gstride) + t.offset;
+    V3<double> lp[kRpl], ld[kRpl];
+    double vr[kRpl], wt[kRpl]; // v sqrt(W) and W of a regular ray, else 0
+    double sw = 0.0, svw = 0.0;
+#pragma unroll
+    for (int i = 0; i < kRpl; ++i) {
+        const int k = tid + i * threads;
+        lp[i] = V3<double>{0.0, 0.0, 0.0};
+        ld[i] = V3<double>{0.0, 0.0, 1.0};
+        vr[i] = wt[i] = 0.0;
+        if (k >= t.n) continue;
+        const Sample smp = sample_at(P, t, ST, k);
+        Ray r = source_ray(P, t, smp, a, sin_t, cos_t, L[0].n);
+        Soft soft{0.0, MKO_STATUS_OK};
+        LastState last{};
+        if (trace_ray<false>(P, L, r, M, kappa, soft, last) == MKO_STATUS_OK) {
+            lp[i] = last.p;
+            ld[i] = last.d;
+            wt[i] = smp.weight;
+            vr[i] = gv[k] * smp.rootw;
+            sw += wt[i];
+            svw += vr[i];
+        }
+    }
+    sw = wave_sum(sw);
+    svw = wave_sum(svw);
+    if (lane == 0) {
+        red[0][wave] = sw;
+        red[1][wave] = svw;
+    }
+    __syncthreads();
+    double W = red[0][0], SV = red[1][0];
+    for (int w = 1; w < waves; ++w) {
+        W += red[0][w];
+        SV += red[1][w];
+    }
+    const double m = W > 0.0 ? SV / W : 0.0;
+#pragma unroll
+    for (int i = 0; i < kRpl; ++i) {
+        const double beta = wt[i] != 0.0 ? t.scale * (vr[i] - wt[i] * m) : 0.0;
+        if (__ballot(beta != 0.0) == 0) continue; // uniform
+        sweep_ray<kGlass, true>(P, L, map, lp[i], ld[i], M, kappa, GroupSink{acc, lane >> 2, beta},
+                                t.l);
+    }
+    __syncthreads();
+    for (int p = tid; p < map.P; p += threads) {
+        double total = 0.0;
+        for (int w = 0; w < waves; ++w)
+            for (int i = 0; i < 16; ++i) total += acc0[(size_t(w) * map.P + p) * 16 + i];
+        part[size_t(blockIdx.x) * map.P + p] = total;
+    }
+}
+
+// Soft failure mode: one wave per tuple, the tuple's rays 64 at a time, each lane adding into its
+// own slot of acc [P][64] (rays with soft continuations take their sweeps at different surfaces).
+struct AccSink {
+    double* acc;
+    int lane;
+    double factor;
+    __device__ __forceinline__ void write(int p, double value) const {
+        if (p >= 0) acc[p * 64 + lane] += factor * value;
+    }
+};
+
+template <bool kGlass>
+__global__ __launch_bounds__(64) void vjp_soft_kernel(TraceParams P, ParamMap map,
+                                                      const double* grad, int64_t gstride,
+                                                      double* part) {
+    extern __shared__ __align__(16) unsigned char vjp_lds[];
+    const Tuple t = tuple_of(P, blockIdx.x);
+    Step* steps = reinterpret_cast<Step*>(vjp_lds);
+    const Step* L = steps;
+    double* acc = reinterpret_cast<double*>(vjp_lds + size_t(P.S + 1) * sizeof(Step)); // [P][64]
+    const int lane = threadIdx.x;
+    stage_steps(P, t.v, t.l, steps);
+    for (int p = 0; p < map.P; ++p) acc[p * 64 + lane] = 0.0;
+    __syncthreads();
+    const size_t vf = size_t(t.v) * P.F + t.f;
+    const double a = P.pupil_radius[t.v];
+    double sin_t, cos_t;
+    sincos(P.field_angle[vf], &sin_t, &cos_t);
+    const V3<double> M{0.0, P.field_target[vf], L[P.S].t};
+    const double kappa = P.ref_kind != MKO_REF_LAST_SURFACE ? P.reference_curvature[vf] : 0.0;
+    const double* gv = grad + size_t(t.v) * size_t(gstride) + t.offset;
     double sw = 0.0, svw = 0.0;
     for (int k = lane; k < t.n; k += 64) {
         const Sample smp = sample_of(P, t, k);
         Ray r = source_ray(P, t, smp, a, sin_t, cos_t, L[0].n);
         Soft soft{0.0, MKO_STATUS_OK};
         NoRecord nr;
-        const uint8_t st = trace_ray<kSoft>(P, L, r, M, kappa, soft, nr);
-        if (mkod::in_piston(st)) {
+        if (mkod::in_piston(trace_ray<true>(P, L, r, M, kappa, soft, nr))) {
             sw += smp.weight;
-            svw += gv[t.offset + k] * smp.rootw;
+            svw += gv[k] * smp.rootw;
         }
     }
     const double W = wave_sum(sw), SV = wave_sum(svw);
     const bool valid = W > 0.0;
     const double m = valid ? SV / W : 0.0;
-    Record rec;
     for (int k = lane; k < t.n; k += 64) {
         const Sample smp = sample_of(P, t, k);
-        Ray r = source_ray(P, t, smp, a, sin_t, cos_t, L[0].n);
+        const Ray start = source_ray(P, t, smp, a, sin_t, cos_t, L[0].n);
+        Ray r = start;
         Soft soft{0.0, MKO_STATUS_OK};
-        rec.count = 0;
-        rec.image_branch = 0;
-        const uint8_t st = trace_ray<kSoft>(P, L, r, M, kappa, soft, rec);
-        const bool reached = mkod::in_piston(st);
-        const double beta =
-            valid && reached ? t.scale * (gv[t.offset + k] * smp.rootw - smp.weight * m) : 0.0;
-        double gamma = 0.0;
-        if (kSoft && soft.first != MKO_STATUS_OK)
-            gamma = t.pscale * smp.rootw * gv[P.rays + t.offset + k];
+        LastState last{};
+        const uint8_t st = trace_ray<true>(P, L, r, M, kappa, soft, last);
+        const double beta = valid && mkod::in_piston(st)
+                                ? t.scale * (gv[k] * smp.rootw - smp.weight * m)
+                                : 0.0;
+        if (st == MKO_STATUS_OK) {
+            if (beta != 0.0)
+                sweep_ray<kGlass, true>(P, L, map, last.p, last.d, M, kappa,
+                                        AccSink{acc, lane, beta}, t.l);
+            continue;
+        }
+        const double gamma =
+            soft.first != MKO_STATUS_OK ? t.pscale * smp.rootw * gv[P.rays + k] : 0.0;
         if (beta != 0.0 || gamma != 0.0)
-            backward_ray(P, L, map, rec, reached, M, kappa, beta, gamma,
-                                         AccSink{acc, lane}, t.l);
+            soft_backward(P, L, map, start, M, kappa, beta, gamma, AccSink{acc, lane, 1.0}, t.l);
     }
     for (int p = 0; p < map.P; ++p) {
         const double total = wave_sum(acc[p * 64 + lane]);
@@ -1962,35 +2150,6 @@ struct SwzSink {
         if (leader) pilot[p] = c;
     }
 };
-
-// The gradients of a regular ray (backward_ray, adjoint_backward.hpp:496-580, with seed 1 for the
-// optical path) from its state (p, d) on the last surface, by mkod's reverse sweep. kGlass: the
-// index gradients as well, into the glass variables' columns of each medium
-// (dn/d(n0, nu1, nu2) = 1, w_l, w_l^2).
-template <bool kGlass, class Sink>
-__device__ __forceinline__ void sweep_ray(const TraceParams& P, const Step* L, const ParamMap& map,
-                                          V3<double> p, V3<double> d, V3<double> M, double kappa,
-                                          const Sink& sink, int l) {
-    const int S = P.S;
-    double mz, length;
-    mkod::SweepState w = mkod::sweep_reference(p, d, M, kappa, P.ref_kind, L[S - 1].n, L[S - 1].c,
-                                               mz, length);
-    sink.write(map.thick_col[S - 1], mz);
-    if constexpr (kGlass) length -= mkod::rev_div(mkod::dot(w.P, w.dq), L[S - 1].n);
-    for (int j = S - 1;; --j) {
-        if constexpr (kGlass) {
-            const double wl = map.omega[l];
-            sink.write(map.glass_col[j][0], length);
-            sink.write(map.glass_col[j][1], length * wl);
-            sink.write(map.glass_col[j][2], length * (wl * wl));
-        }
-        const double cb = mkod::sweep_refract(w, L[j]);
-        if ((P.sphere_mask >> j) & 1ull) sink.write(map.curv_col[j], cb);
-        sink.write(map.thick_col[j - 1], w.P.z + w.dP.z);
-        if (j == 1) break;
-        mkod::sweep_transfer<kGlass>(w, L[j], L[j - 1].c, L[j - 1].cna, L[j - 1].n, length);
-    }
-}
 
 // Lane k's value of x (k wave-uniform).
 __device__ __forceinline__ double lane_value(double x, int k) {
@@ -2239,7 +2398,7 @@ void adjoint_normal_kernel(TraceParams P, ParamMap map,
             sw += wk;
             swo += wk * opl;
             const bool leader = lane == int(__builtin_ctzll(okmask));
-            sweep_ray<kGlass>(P, L, map, last.p, last.d, M, kappa,
+            sweep_ray<kGlass, false>(P, L, map, last.p, last.d, M, kappa,
                               SwzSink<kNW>{G, own_pilot, tid, leader}, t.l);
         }
         __syncthreads();
@@ -2818,11 +2977,15 @@ int pack_segment(const TraceParams& P, bool packable) {
     return seg;
 }
 
-int rays_per_lane(const TraceParams& P) {
+int largest_tuple(const TraceParams& P) {
     int nmax = 0;
     for (int f = 0; f < P.F; ++f)
         nmax = std::max(nmax, P.rings * (P.pupil_mode[f] == MKO_PUPIL_AXIS ? 1 : P.spokes));
-    const int r = (nmax + kBlock - 1) / kBlock;
+    return nmax;
+}
+
+int rays_per_lane(const TraceParams& P) {
+    const int r = (largest_tuple(P) + kBlock - 1) / kBlock;
     return r <= 1 ? 1 : r <= 2 ? 2 : r <= 4 ? 4 : 8;
 }
 
@@ -2970,6 +3133,14 @@ ParamMap make_map(const mko_variables& vars, const mko_batch& batch, bool allow_
             slot = k;
         }
     }
+    for (int s = 0; s < S; ++s) {
+        const auto unswept = [&](int col) {
+            if (col >= 0) m.unswept[col >> 6] |= uint64_t(1) << (col & 63);
+        };
+        if (s == 0 || batch.type[s] != MKO_SURFACE_SPHERE) unswept(m.curv_col[s]);
+        if (s == 0)
+            for (int c = 0; c < 3; ++c) unswept(m.glass_col[s][c]);
+    }
     if (m.glass) {
         const OmegaTable t = omega_table(batch);
         if (!t.valid)
@@ -2980,20 +3151,49 @@ ParamMap make_map(const mko_variables& vars, const mko_batch& batch, bool allow_
     return m;
 }
 
-template <bool kSoft>
-void launch_adjoint_rpl(int rpl, const TraceParams& P, const ParamMap& m, double* J, double* r0,
-                        uint8_t* st, hipStream_t stream) {
-    const dim3 grid(unsigned(P.V) * unsigned(P.T));
-#define MKO_LAUNCH(R)                                                                            \
-    hipLaunchKernelGGL((adjoint_kernel<kSoft, R>), grid, dim3(kBlock), 0, stream, P,  \
-                       m, J, r0, st)
-    switch (rpl) {
-    case 1: MKO_LAUNCH(1); break;
-    case 2: MKO_LAUNCH(2); break;
-    case 4: MKO_LAUNCH(4); break;
-    default: MKO_LAUNCH(8); break;
+// Lanes of a workgroup for tuples of at most nmax rays: as many waves as they fill, up to 4.
+int tuple_lanes(int nmax) { return std::min(kBlock, 64 * ((nmax + 63) / 64)); }
+
+template <bool kSoft, bool kGlass>
+void launch_adjoint(const TraceParams& P, const ParamMap& m, double* J, double* r0, uint8_t* st,
+                    hipStream_t stream) {
+    const int nmax = largest_tuple(P);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(P.V) * unsigned(P.T)), dim3(tuple_lanes(nmax)),
+                           size_t(P.S + 1) * sizeof(Step) + size_t(nmax) * sizeof(double2), stream,
+                           P, m, J, r0, st);
+    };
+    switch (rays_per_lane(P)) {
+    case 1: launch(adjoint_kernel<kSoft, kGlass, 1>); break;
+    case 2: launch(adjoint_kernel<kSoft, kGlass, 2>); break;
+    case 4: launch(adjoint_kernel<kSoft, kGlass, 4>); break;
+    default: launch(adjoint_kernel<kSoft, kGlass, 8>); break;
     }
-#undef MKO_LAUNCH
+}
+
+template <bool kGlass>
+void launch_vjp(const TraceParams& P, const ParamMap& m, const double* grad, int64_t gstride,
+                double* part, hipStream_t stream) {
+    const int nmax = largest_tuple(P), lanes = tuple_lanes(nmax);
+    const dim3 grid(unsigned(P.V) * unsigned(P.T));
+    const size_t table = size_t(P.S + 1) * sizeof(Step);
+    if (P.soft) {
+        hipLaunchKernelGGL(vjp_soft_kernel<kGlass>, grid, dim3(64),
+                           table + size_t(m.P) * 64 * sizeof(double), stream, P, m, grad, gstride,
+                           part);
+        return;
+    }
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(lanes),
+                           table + size_t(lanes / 64) * m.P * 16 * sizeof(double), stream, P, m,
+                           grad, gstride, part);
+    };
+    switch (rays_per_lane(P)) {
+    case 1: launch(vjp_kernel<kGlass, 1>); break;
+    case 2: launch(vjp_kernel<kGlass, 2>); break;
+    case 4: launch(vjp_kernel<kGlass, 4>); break;
+    default: launch(vjp_kernel<kGlass, 8>); break;
+    }
 }
 
 #define MKO_TRY(...)                                                                               \
@@ -3480,15 +3680,16 @@ int adjoint_jacobian(const mko_batch* batch, const mko_residual_settings* settin
         const ParamMap m = make_map(*vars, *batch, true);
         if (P.V == 0) return 0;
         if (int64_t(P.V) * P.T > 0x7fffffffLL) throw std::invalid_argument("batch too large");
-        const int rpl = rays_per_lane(P);
         const hipStream_t s = static_cast<hipStream_t>(stream);
         // MKO_PRECISION_MIXED computes the stored Jacobian in FP64 as well: on this hardware
         // the reduced-precision stage is the MFMA normal equations of the fused LM path.
         if (precision != MKO_PRECISION_FP64 && precision != MKO_PRECISION_MIXED)
             throw std::invalid_argument("unknown precision");
         double* Jd = static_cast<double*>(jacobian);
-        if (P.soft) launch_adjoint_rpl<true>(rpl, P, m, Jd, r0, status, s);
-        else launch_adjoint_rpl<false>(rpl, P, m, Jd, r0, status, s);
+        if (P.soft) m.glass ? launch_adjoint<true, true>(P, m, Jd, r0, status, s)
+                            : launch_adjoint<true, false>(P, m, Jd, r0, status, s);
+        else m.glass ? launch_adjoint<false, true>(P, m, Jd, r0, status, s)
+                     : launch_adjoint<false, false>(P, m, Jd, r0, status, s);
         check_hip(hipGetLastError(), "adjoint launch");
     })
 }
@@ -3613,14 +3814,8 @@ int mko_vjp_device(const mko_batch* batch, const mko_residual_settings* settings
             throw std::invalid_argument("workspace too small");
         const hipStream_t s = static_cast<hipStream_t>(stream);
         double* part = static_cast<double*>(workspace);
-        const dim3 grid(unsigned(P.V) * unsigned(P.T));
-        const size_t lds = size_t(m.P) * 64 * sizeof(double);
-        if (P.soft)
-            hipLaunchKernelGGL(vjp_kernel<true>, grid, dim3(64), lds, s, P, m, grad, grad_stride,
-                               part);
-        else
-            hipLaunchKernelGGL(vjp_kernel<false>, grid, dim3(64), lds, s, P, m, grad, grad_stride,
-                               part);
+        if (m.glass) launch_vjp<true>(P, m, grad, grad_stride, part, s);
+        else launch_vjp<false>(P, m, grad, grad_stride, part, s);
         check_hip(hipGetLastError(), "vjp launch");
         const int64_t n = int64_t(P.V) * m.P;
         hipLaunchKernelGGL(vjp_finalize_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s,
