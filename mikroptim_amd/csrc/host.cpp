@@ -888,10 +888,13 @@ public:
         const bool fused = glass_fused || (!fd && precision == MKO_PRECISION_MIXED && !J && !r0 &&
                                            (a || g) && fused_ok(s, vars));
         const bool pattern = fd || rp.count() > 0;
+        // FD differences whose residuals pass through memory
+        const bool fd_stored =
+            fd && !(rp.count() == 0 && mko_internal::fd_direct(base, s, vars));
         const int per_run = fd ? 2 * P + 1 : 1;
         const size_t Tt = size_t(base.fields) * base.wavelengths, S = size_t(base.surfaces);
         const size_t per = size_t(per_run) * (Strides(base).doubles() * 8 +
-                                              (fd ? size_t(R) * 8 + size_t(rays) : 0) +
+                                              (fd_stored ? size_t(R) * 8 + size_t(rays) : 0) +
                                               (fd && rp.Et ? (Tt + 1) * S * 16 : 0)) +
                            (fused ? Tt * (size_t(P) * P * 4 + size_t(P) * 64 + 24) + 1024 +
                                         (glass_fused ? size_t(rays) * 56 + Tt * 16 + 32 : 0)
@@ -1086,10 +1089,13 @@ public:
         const bool fused = !fd && precision == MKO_PRECISION_MIXED &&
                            fused_ok(s, vars_host_dev_, states != nullptr);
         const bool pattern = fd || rp.count() > 0;
+        // FD differences whose residuals pass through memory
+        const bool fd_stored =
+            fd && !(rp.count() == 0 && mko_internal::fd_direct(tmpl, s, vars_host_dev_));
         const int per_run = fd ? 2 * P + 1 : 1;
         const size_t Tt = size_t(tmpl.fields) * tmpl.wavelengths, S = size_t(tmpl.surfaces);
         const size_t per = size_t(per_run) * (Strides(tmpl).doubles() * 8 +
-                                              (fd ? size_t(R) * 8 + size_t(rays) : 0) +
+                                              (fd_stored ? size_t(R) * 8 + size_t(rays) : 0) +
                                               (fd && rp.Et ? (Tt + 1) * S * 16 : 0)) +
                            (fused ? Tt * (size_t(P) * P * 4 + size_t(P) * 64 + 24) + 1024
                                   : size_t(P) * R * 8 + size_t(R) * 8) +
@@ -1438,12 +1444,20 @@ private:
                size_t(P + 1) * rp.count() * 8 + cand;
     }
 
-    // FD Jacobian of the central FD batch fdb (count runs x (2P + 1) variants): RESIDUALS of
+    // FD Jacobian of the central FD batch fdb (count runs x (2P + 1) variants): without constraint
+    // rows straight from the batch (fd_jacobian), else RESIDUALS of
     // every variant with its constraint rows (traced rows from the variant's own extrema) at
     // stride R, then fd_derivative of all R rows (fd_jacobian_cpu, src/optim/fd_jacobian.cpp:182).
     void fd_rows(const mko_batch& fdb, const mko_residual_settings& s, const RowPlan& rp,
                  int count, int P, const double* dsp, const double* dsm, const uint8_t* dsten,
                  int64_t T, int64_t R, int64_t rays, double* dJ, double* dr0) {
+        if (rp.count() == 0 && mko_internal::fd_direct(fdb, s, vars_host_dev_)) {
+            timer.run(kTrace, [&] {
+                dev_check(mko_internal::fd_jacobian(&fdb, &s, &vars_host_dev_, count, dsp, dsm,
+                                                    dsten, dJ, dr0, R, nullptr));
+            });
+            return;
+        }
         const size_t n = size_t(count) * (2 * P + 1);
         const size_t Tt = size_t(fdb.fields) * fdb.wavelengths, S = size_t(fdb.surfaces);
         double* fres = fdres_.as<double>(n * R);

@@ -130,6 +130,17 @@ int adjoint_jacobian(const mko_batch* batch, const mko_residual_settings* settin
 int gram_chain(const double* jacobian, const double* r0, int runs, int variables, int64_t rows,
                double* a, double* g, void* stream, const int32_t* live);
 
+// FD Jacobian of the trace rows and r0 straight from the central FD batch (runs x (2 P + 1)
+// variants, device), J / r0 rows at jstride: the values of RESIDUALS of every variant and
+// mko_fd_difference_device, bit for bit, without the differences' residuals in memory.
+// fd_direct: whether it applies (FP64 trace, no glass variable on the medium before the first
+// surface, up to 320 variables whose moved steps fit the LDS); vars: host arrays.
+bool fd_direct(const mko_batch& batch, const mko_residual_settings& s, const mko_variables& vars);
+int fd_jacobian(const mko_batch* fd_batch, const mko_residual_settings* settings,
+                const mko_variables* vars, int runs, const double* step_plus,
+                const double* step_minus, const uint8_t* stencil, double* jacobian, double* r0,
+                int64_t jstride, void* stream);
+
 // mko_fd_difference_device with J column (i, p) at jacobian + (i * P + p) * jstride + joffset,
 // r0 of run i at r0 + i * jstride + joffset; status / status_changes may be NULL.
 int fd_difference(const double* rows, int64_t stride, const uint8_t* status, int64_t rays,

@@ -1587,6 +1587,16 @@ __global__ void point_batch_kernel(ConstBatchPtrs src, BatchPtrs dst, int runs, 
     }
 }
 
+// fd_derivative (fd_formula.hpp:39) from the residual at the point and at its two differences.
+__device__ __forceinline__ double fd_derivative(double a0, double aa, double ab, double da,
+                                                double db, uint8_t stencil) {
+    if (stencil == MKO_STENCIL_ONE_SIDED) {
+        const double ga = aa - a0, gb = ab - a0;
+        return (db * db * ga - da * da * gb) / (da * db * (db - da));
+    }
+    return (aa - ab) / (da - db);
+}
+
 // J[i][k][r] = fd_derivative (fd_formula.hpp:39) from the FD residuals; block (i, P) copies r0.
 // Status changes per (i, k): rays whose Ok-ness differs between x0 and either point.
 __global__ __launch_bounds__(kBlock) void fd_difference_kernel(
@@ -1611,15 +1621,7 @@ __global__ __launch_bounds__(kBlock) void fd_difference_kernel(
     const uint8_t sten = stencil[size_t(i) * P + k];
     double* col = J + (size_t(i) * P + k) * jstride + joffset;
     for (int64_t r = threadIdx.x; r < rows; r += kBlock) {
-        const double a0 = r_0[r], aa = ra[r], ab = rb[r];
-        double v;
-        if (sten == MKO_STENCIL_ONE_SIDED) {
-            const double ga = aa - a0, gb = ab - a0;
-            v = (db * db * ga - da * da * gb) / (da * db * (db - da));
-        } else {
-            v = (aa - ab) / (da - db);
-        }
-        col[r] = v;
+        col[r] = fd_derivative(r_0[r], ra[r], rb[r], da, db, sten);
     }
     if (!st) return;
     int c = 0;
@@ -1632,6 +1634,252 @@ __global__ __launch_bounds__(kBlock) void fd_difference_kernel(
     }
     const int total = block_sum(c, ired);
     if (threadIdx.x == 0) changes[size_t(i) * P + k] = total;
+}
+
+// ---- FD Jacobian without the differences' residuals -----------------------------------------
+
+// The variables in the order of the first step their differences change: a curvature the step to
+// its surface, a thickness the step after it (the last one only the reference sphere, first = S),
+// a glass coefficient the steps to its surface and to the next one.
+constexpr int kFdMaxVariables = 320;
+struct FdPlan {
+    int P, parts;
+    int32_t var[kFdMaxVariables]; // variable | first step << 16 | glass << 24
+};
+
+// FD Jacobian of the trace rows, J[i][k][row] at jstride, and r0, one workgroup of up to 4 waves per
+// (run, tuple) of the central FD batch P (runs x (2 plan.P + 1) variants). A difference of a
+// variable leaves the rays alone up to the variable's surface: the workgroup takes the rays of the
+// run's point through the surfaces once, and at each surface sends a copy of them through the rest
+// of the system for both differences of the variables that start there. About half of the
+// surface steps of tracing every variant (P = 48, 25 surfaces: 1250 instead of 2328 per ray), and
+// the differences' residuals stay in registers: 32 runs x 17920 rays 3.5 + 0.2 ms (every variant
+// traced, then differenced in a second kernel) -> 1.95 ms, 0.74 of the vector ALU's issue slots.
+// Registers capped for 4 waves per SIMD up to 512 rays per tuple in hard mode (28 bytes of spill).
+// Both differences of a ray in one pass of the surface loop (two chains): 1.92 ms, not kept. Same
+// step, reference sphere, sums
+// in the order of trace_kernel's and difference formula, so J and r0 are those of the two kernels
+// bit for bit.
+template <bool kSoft, int kRpl>
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(kSoft ? (kRpl <= 1 ? 3 : 1) : kRpl <= 2 ? 4 : 1)))
+void fd_jacobian_kernel(TraceParams P, FdPlan plan,
+                                                             const double* step_plus,
+                                                             const double* step_minus,
+                                                             const uint8_t* stencil, double* J,
+                                                             double* r0, int64_t jstride) {
+    extern __shared__ __align__(16) unsigned char fd_lds[];
+    __shared__ SampleTable ST;
+    __shared__ double red[2][4][kWaves];
+    const int Pn = plan.P;
+    const int tuple = int(blockIdx.x) / plan.parts;
+    const int part = int(blockIdx.x) - tuple * plan.parts;
+    const int run = tuple / P.T, tt = tuple - run * P.T;
+    const int v0 = run * (2 * Pn + 1);
+    const Tuple t = tuple_of(P, v0 * P.T + tt);
+    Step* steps = reinterpret_cast<Step*>(fd_lds);
+    Step* moved = steps + (P.S + 1); // [P][2 differences][2 steps], in plan order
+    const Step* L = steps;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int threads = int(blockDim.x), waves = threads >> 6;
+    stage_samples(P, t, ST);
+    stage_steps(P, v0, t.l, steps);
+    for (int e = tid; e < 4 * Pn; e += threads) {
+        const int k = plan.var[e >> 2] & 0xffff, first = (plan.var[e >> 2] >> 16) & 0xff;
+        const int s = first + (e & 1);
+        if (s <= P.S) moved[e] = step_at(P, v0 + 2 * k + 1 + ((e >> 1) & 1), t.l, s);
+    }
+    __syncthreads();
+    const size_t vf = size_t(t.v) * P.F + t.f;
+    const double a = P.pupil_radius[t.v];
+    double sin_t, cos_t;
+    sincos(P.field_angle[vf], &sin_t, &cos_t);
+    const V3<double> M{0.0, P.field_target[vf], L[P.S].t};
+    const double kappa = P.ref_kind != MKO_REF_LAST_SURFACE ? P.reference_curvature[vf] : 0.0;
+
+    // a ray on its way: momentum in r.d; st != Ok: it failed
+    struct Way {
+        Ray r;
+        double pen;
+        uint8_t st, first;
+    };
+    const auto advance = [&](Way& w, const Step& k, double nb) {
+        if (w.st != MKO_STATUS_OK) return;
+        double n_dot;
+        if constexpr (kSoft) {
+            Soft soft{w.pen, w.first};
+            uint8_t branch = 0;
+            w.st = mkod::momentum_step_soft(w.r.p, w.r.d, w.r.opl, k, nb, n_dot, soft, branch);
+            w.pen = soft.penalty;
+            w.first = soft.first;
+        } else {
+            w.st = mkod::momentum_step(w.r.p, w.r.d, w.r.opl, k, n_dot);
+        }
+    };
+    // the reference sphere: final status in w.st
+    const auto finish = [&](Way& w, double n_last, double mz) {
+        if (w.st != MKO_STATUS_OK) return;
+        const double rn = mkod::rev_rcp(n_last);
+        w.r.d = V3<double>{rn * w.r.d.x, rn * w.r.d.y, rn * w.r.d.z};
+        if (!(w.r.d.z > 0.0)) {
+            w.st = MKO_STATUS_BACKWARD;
+            return;
+        }
+        Soft soft{w.pen, w.first};
+        uint8_t rb = 0;
+        const uint8_t rst = mkod::reference_step<kSoft>(w.r, V3<double>{M.x, M.y, mz}, kappa,
+                                                        P.ref_kind, n_last, soft, rb);
+        if constexpr (kSoft) {
+            w.pen = soft.penalty;
+            w.first = soft.first;
+        }
+        w.st = !mkod::in_piston(rst) ? rst : kSoft ? soft.first : uint8_t(MKO_STATUS_OK);
+    };
+    // weight and weighted path of a finished ray
+    const auto count = [&](const Way& w, double weight, double& sw, double& swo) {
+        if (mkod::in_piston(w.st)) {
+            sw += weight;
+            swo += weight * w.r.opl;
+        }
+    };
+    const auto penalty_row = [&](const Way& w, double rootw) {
+        const double fp = w.st == MKO_STATUS_OK ? 0.0 : mkod::is_soft(w.st) ? w.pen : w.pen + 1.0;
+        return t.pscale * rootw * fp;
+    };
+
+    double weight[kRpl], rootw[kRpl], base_r[kRpl], base_p[kRpl];
+    Way way[kRpl];
+    const auto start = [&](int i) {
+        Way w{};
+        const int k = tid + i * threads;
+        w.st = MKO_STATUS_UNSUPPORTED;
+        if (k < t.n) {
+            const Sample s = sample_at(P, t, ST, k);
+            w.r = source_ray(P, t, s, a, sin_t, cos_t, L[0].n);
+            const double n0 = L[0].n;
+            w.r.d = V3<double>{n0 * w.r.d.x, n0 * w.r.d.y, n0 * w.r.d.z};
+            w.st = MKO_STATUS_OK;
+            w.first = MKO_STATUS_OK;
+            weight[i] = s.weight;
+            rootw[i] = s.rootw;
+        }
+        return w;
+    };
+    // the point itself: r0
+    {
+        double sw = 0.0, swo = 0.0;
+#pragma unroll
+        for (int i = 0; i < kRpl; ++i) {
+            weight[i] = rootw[i] = 0.0;
+            Way w = start(i);
+            for (int s = 1; s < P.S; ++s) advance(w, L[s], L[s - 1].n);
+            finish(w, L[P.S - 1].n, M.z);
+            count(w, weight[i], sw, swo);
+            base_r[i] = mkod::in_piston(w.st) ? w.r.opl : __builtin_nan("");
+            base_p[i] = kSoft ? penalty_row(w, rootw[i]) : 0.0;
+        }
+        sw = wave_sum(sw);
+        swo = wave_sum(swo);
+        if (lane == 0) {
+            red[0][0][wave] = sw;
+            red[0][1][wave] = swo;
+        }
+        __syncthreads();
+        double W = red[0][0][0], O = red[0][1][0];
+        for (int w = 1; w < waves; ++w) {
+            W += red[0][0][w];
+            O += red[0][1][w];
+        }
+        const double piston = W > 0.0 ? O / W : 0.0;
+#pragma unroll
+        for (int i = 0; i < kRpl; ++i) {
+            const int k = tid + i * threads;
+            const bool ok = W > 0.0 && !__builtin_isnan(base_r[i]);
+            const double e = ok ? base_r[i] - piston : 0.0;
+            base_r[i] = t.scale * rootw[i] * e;
+            if (k < t.n && part == 0) {
+                double* out = r0 + size_t(run) * jstride + t.offset + k;
+                out[0] = base_r[i];
+                if (kSoft) out[P.rays] = base_p[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kRpl; ++i) way[i] = start(i);
+    int q = 0, parity = 0;
+    for (int s = 1; s <= P.S; ++s) {
+        // `way` is on surface s - 1: the differences whose first step is s
+        for (; q < Pn && ((plan.var[q] >> 16) & 0xff) == s; ++q) {
+            if (q % plan.parts != part) continue;
+            parity ^= 1;
+            const int k = plan.var[q] & 0xffff;
+            const bool glass = (plan.var[q] >> 24) != 0;
+            const size_t ik = size_t(run) * Pn + k;
+            double opl[2][kRpl], pen[2][kRpl], sw[2] = {0.0, 0.0}, swo[2] = {0.0, 0.0};
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                const Step* mv = moved + (4 * q + 2 * side);
+                const double n_last = glass && s == P.S - 1 ? mv[0].n : L[P.S - 1].n;
+                const double mz = s == P.S ? mv[0].t : M.z;
+#pragma unroll
+                for (int i = 0; i < kRpl; ++i) {
+                    Way w = way[i];
+                    for (int j = s; j < P.S; ++j) {
+                        const bool second = glass && j == s + 1;
+                        const Step* kj = j == s ? mv : second ? mv + 1 : L + j;
+                        advance(w, *kj, second ? mv[0].n : L[j - 1].n);
+                    }
+                    finish(w, n_last, mz);
+                    count(w, weight[i], sw[side], swo[side]);
+                    opl[side][i] = mkod::in_piston(w.st) ? w.r.opl : __builtin_nan("");
+                    pen[side][i] = kSoft ? penalty_row(w, rootw[i]) : 0.0;
+                }
+                sw[side] = wave_sum(sw[side]);
+                swo[side] = wave_sum(swo[side]);
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    red[parity][2 * side][wave] = sw[side];
+                    red[parity][2 * side + 1][wave] = swo[side];
+                }
+            }
+            __syncthreads(); // the other half of red is free: every wave has read it by now
+            double W[2], piston[2];
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                double x = red[parity][2 * side][0], o = red[parity][2 * side + 1][0];
+                for (int w = 1; w < waves; ++w) {
+                    x += red[parity][2 * side][w];
+                    o += red[parity][2 * side + 1][w];
+                }
+                W[side] = x;
+                piston[side] = x > 0.0 ? o / x : 0.0;
+            }
+            const double da = step_plus[ik], db = step_minus[ik];
+            const uint8_t sten = stencil[ik];
+#pragma unroll
+            for (int i = 0; i < kRpl; ++i) {
+                const int kr = tid + i * threads;
+                if (kr >= t.n) continue;
+                double r[2];
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    const bool ok = W[side] > 0.0 && !__builtin_isnan(opl[side][i]);
+                    const double e = ok ? opl[side][i] - piston[side] : 0.0;
+                    r[side] = t.scale * rootw[i] * e;
+                }
+                double* col = J + ik * jstride + t.offset + kr;
+                col[0] = fd_derivative(base_r[i], r[0], r[1], da, db, sten);
+                if (kSoft)
+                    col[P.rays] = fd_derivative(base_p[i], pen[0][i], pen[1][i], da, db, sten);
+            }
+        }
+        if (s < P.S) {
+#pragma unroll
+            for (int i = 0; i < kRpl; ++i) advance(way[i], L[s], L[s - 1].n);
+        }
+    }
 }
 
 // ---- ADJOINT Jacobian -----------------------------------------------------------------------
@@ -3732,6 +3980,67 @@ int gram_chain(const double* jacobian, const double* r0, int runs, int variables
             else launch(gram_kernel<5, 64, 16>, 64);
         }
         check_hip(hipGetLastError(), "gram launch");
+    })
+}
+
+// Dynamic LDS of fd_jacobian_kernel: the point's steps and two per difference.
+static size_t fd_lds_bytes(int S, int P) { return size_t(S + 1 + 4 * P) * sizeof(Step); }
+
+bool fd_direct(const mko_batch& batch, const mko_residual_settings& s, const mko_variables& vars) {
+    if (s.precision != MKO_PRECISION_FP64 || vars.count > kFdMaxVariables ||
+        fd_lds_bytes(batch.surfaces, vars.count) > size_t(96) << 10)
+        return false;
+    for (int k = 0; k < vars.count; ++k)
+        if (vars.type[k] == MKO_VAR_GLASS && vars.batch_surface[k] == 0) return false;
+    return true;
+}
+
+int fd_jacobian(const mko_batch* fd_batch, const mko_residual_settings* settings,
+                const mko_variables* vars, int runs, const double* step_plus,
+                const double* step_minus, const uint8_t* stencil, double* jacobian, double* r0,
+                int64_t jstride, void* stream) {
+    MKO_TRY({
+        TraceParams P = make_params(*fd_batch, *settings);
+        if (runs <= 0) return 0;
+        const int S = P.S;
+        FdPlan plan{};
+        plan.P = vars->count;
+        int at = 0;
+        for (int first = 1; first <= S; ++first)
+            for (int k = 0; k < vars->count; ++k) {
+                const int s = vars->batch_surface[k];
+                if (s < 0 || s >= S) throw std::invalid_argument("variable surface out of range");
+                const bool glass = vars->type[k] == MKO_VAR_GLASS;
+                const bool curv = vars->type[k] == MKO_VAR_CURVATURE;
+                // the curvature of the first surface (the stop) changes nothing: its differences
+                // run through the reference sphere only
+                const int f = curv && s == 0 ? S : glass || curv ? s : s + 1;
+                if (f == first) plan.var[at++] = k | (f << 16) | (int(glass) << 24);
+            }
+        if (int64_t(runs) * P.T > 0x1fffffffLL) throw std::invalid_argument("batch too large");
+        // A tuple's variables are dealt out to 1, 2 or 4 workgroups (each traces the point itself,
+        // 2 of the about 2 + P passes) where there are few tuples: 1024 workgroups run at once, and
+        // 1120 (32 runs of the 35-tuple objective) leave most of a second round empty (2.25 ms in
+        // one part, 1.95 in two)
+        plan.parts = runs * P.T >= 4096 || plan.P < 8 ? 1 : runs * P.T >= 1024 || plan.P < 16 ? 2 : 4;
+        const hipStream_t st = static_cast<hipStream_t>(stream);
+        const auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(unsigned(runs) * unsigned(P.T * plan.parts)),
+                               dim3(tuple_lanes(largest_tuple(P))), fd_lds_bytes(S, vars->count),
+                               st, P, plan, step_plus, step_minus, stencil, jacobian, r0, jstride);
+        };
+        const int rpl = rays_per_lane(P);
+        if (P.soft)
+            rpl == 1   ? launch(fd_jacobian_kernel<true, 1>)
+            : rpl == 2 ? launch(fd_jacobian_kernel<true, 2>)
+            : rpl == 4 ? launch(fd_jacobian_kernel<true, 4>)
+                       : launch(fd_jacobian_kernel<true, 8>);
+        else
+            rpl == 1   ? launch(fd_jacobian_kernel<false, 1>)
+            : rpl == 2 ? launch(fd_jacobian_kernel<false, 2>)
+            : rpl == 4 ? launch(fd_jacobian_kernel<false, 4>)
+                       : launch(fd_jacobian_kernel<false, 8>);
+        check_hip(hipGetLastError(), "fd jacobian launch");
     })
 }
 

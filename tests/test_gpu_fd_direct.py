@@ -1,0 +1,157 @@
+"""The FD Jacobian whose differences restart at the variable's surface (fd_jacobian) against the
+general path it replaces: RESIDUALS of every difference's point and the difference formula, bit for
+bit, for every kind of variable (curvatures of spheres, of a plane and of the stop, thicknesses,
+working distance, glass coefficients on the first, inner and last media), central, one-sided and
+truncated stencils, hard and soft failure with failing rays, tuples of 1 ... 2048 rays, image
+reference spheres and a point source. And what keeps the general path: constraint rows, df64."""
+
+import numpy as np
+import pytest
+
+from mikroptim_amd import abi, systems
+from mikroptim_amd.batch import ResidualSettings, VariableSet, residual_rows
+from oracle_lib import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _general(engine, base, s, v, x):
+    """J and r0 of the points x from RESIDUALS of every difference's point."""
+    J, r0 = [], []
+    for xi in x:
+        _, plus, minus, sp, sm, sten = oracle().fd_pattern(base, v, xi)
+        pts = [xi]
+        for k in range(v.size):
+            for value in (plus[k], minus[k]):
+                p = xi.copy()
+                p[k] = value
+                pts.append(p)
+        b = base.take(np.zeros(len(pts), dtype=np.int64))
+        v.apply(b, np.array(pts))
+        r, _, _ = engine.residuals(b, s)
+        cols = []
+        for k in range(v.size):
+            aa, ab, da, db = r[2 * k + 1], r[2 * k + 2], sp[k], sm[k]
+            if sten[k] == 1:
+                # as the device compiles it: fused multiply-adds, checked to rounding below
+                ga, gb = aa - r[0], ab - r[0]
+                cols.append((db * db * ga - da * da * gb) / (da * db * (db - da)))
+            else:
+                cols.append((aa - ab) / (da - db))
+        J.append(cols)
+        r0.append(r[0])
+    return np.array(J), np.array(r0)
+
+
+def _check(engine, base, s, v, x):
+    J, r0, _, _ = engine.jacobian(base, s, v, x, method="fd", precision="fp64")
+    Jg, rg = _general(engine, base, s, v, x)
+    assert np.array_equal(r0, rg)
+    for i, xi in enumerate(x):
+        sten = oracle().fd_pattern(base, v, xi)[5]
+        for k in range(v.size):
+            if sten[k] == 1:
+                # the one-sided formula's two products of db^2 ga and da^2 gb cancel to a third of
+                # their size; a fused and an unfused evaluation differ by a few roundings of them
+                assert np.allclose(J[i, k], Jg[i, k], rtol=1e-14,
+                                   atol=1e-14 * np.max(np.abs(Jg[i, k]), initial=0.0))
+            else:
+                assert np.array_equal(J[i, k], Jg[i, k]), (i, k)
+    return J
+
+
+@pytest.mark.parametrize("failure", [abi.FAILURE_HARD, abi.FAILURE_SOFT])
+@pytest.mark.parametrize("rings,spokes", [(1, 1), (4, 16), (5, 13), (16, 16), (1, 257), (9, 57),
+                                          (16, 128)])
+def test_tuple_shapes(engine, rings, spokes, failure):
+    b, v = systems.singlet(4)
+    x = v.extract(b)[:2].copy()
+    v.upper[:2] = 0.3
+    x[1, 0] = 0.21  # front radius near the pupil radius: rays fail
+    s = ResidualSettings(rings=rings, spokes=spokes, failure=failure)
+    _check(engine, b.take([0]), s, v, x)
+
+
+@pytest.mark.parametrize("failure", [abi.FAILURE_HARD, abi.FAILURE_SOFT])
+@pytest.mark.parametrize("topology", [0, 6, 13])
+def test_uneven_topologies(engine, topology, failure):
+    b, v = systems.uneven_topology(topology, variants=3)
+    s = systems.uneven_settings(failure)
+    _check(engine, b.take([0]), s, v, v.extract(b)[1:])
+
+
+def test_objective(engine):
+    b, v = systems.objective(variants=3, seed=2)
+    s = ResidualSettings(rings=6, spokes=32, failure=abi.FAILURE_HARD)
+    _check(engine, b.take([0]), s, v, v.extract(b)[1:2])
+
+
+def _variables(items, lower, upper):
+    n = len(items)
+    return VariableSet(type=np.array([t for t, _, _ in items], dtype=np.int32),
+                       batch_surface=np.array([q for _, q, _ in items], dtype=np.int32),
+                       lower=np.array(lower), upper=np.array(upper), typical=np.full(n, 0.01),
+                       names=[str(i) for i in range(n)],
+                       component=np.array([c for _, _, c in items], dtype=np.int32))
+
+
+def test_every_variable_kind_and_stencil(engine):
+    """Stop curvature, a plane's curvature, thickness 0, inner thickness, working distance, glass
+    before the last surface and behind it; bounds that make central, one-sided and truncated
+    stencils."""
+    b, _ = systems.glass_singlet(2)
+    b.buchdahl[:, 2, :] = (1.0, 0.0, 0.0, 0.0)
+    C, T, W, G = (abi.VAR_CURVATURE, abi.VAR_THICKNESS, abi.VAR_WORKING_DISTANCE, abi.VAR_GLASS)
+    items = [(T, 1, 0), (C, 2, 0), (G, 2, 0), (C, 0, 0), (G, 1, 1), (W, 2, 0), (C, 1, 0), (T, 0, 0),
+             (G, 1, 0), (G, 2, 1)]
+    base = b.take([0])
+    v = _variables(items, [-1e3] * 10, [1e3] * 10)
+    x = v.extract(base)
+    s = ResidualSettings(rings=5, spokes=9, failure=abi.FAILURE_HARD)
+    _check(engine, base, s, v, x)
+    # c[1] at its lower bound (one-sided), working distance in a box of 1e-7 (truncated)
+    v.lower[6] = x[0, 6]
+    v.lower[5], v.upper[5] = x[0, 5] - 5e-8, x[0, 5] + 5e-8
+    stencils = oracle().fd_pattern(base, v, x[0])[5]
+    assert {0, 1, 2} == set(int(q) for q in stencils)
+    _check(engine, base, s, v, x)
+    base.type = base.type.copy()
+    base.type[2] = abi.SURFACE_PLANE
+    base.curvature[:, 2] = 0.0
+    v = _variables(items, [-1e3] * 10, [1e3] * 10)
+    J = _check(engine, base, s, v, v.extract(base))
+    assert np.all(J[:, [1, 3]] == 0.0)
+
+
+@pytest.mark.parametrize("kind", [abi.REF_IMAGE_EXIT_PUPIL, abi.REF_IMAGE_INFINITE])
+def test_image_references(engine, kind):
+    b, v = systems.singlet(2)
+    b.reference_sphere = kind
+    b.reference_curvature = np.full((2, b.fields), 0.0 if kind == abi.REF_IMAGE_INFINITE else 0.009)
+    s = ResidualSettings(rings=6, spokes=11, failure=abi.FAILURE_SOFT)
+    _check(engine, b.take([0]), s, v, v.extract(b)[1:])
+
+
+def test_point_source(engine):
+    b, v = systems.point_singlet()
+    s = ResidualSettings(rings=7, spokes=9, failure=abi.FAILURE_HARD)
+    _check(engine, b.take([0]), s, v, v.extract(b)[:2])
+
+
+def test_general_path_kept(engine):
+    """Constraint rows and the df64 trace take the general path; its trace rows agree."""
+    import copy
+
+    b, v = systems.singlet(3)
+    s = systems.singlet_settings(abi.FAILURE_HARD)
+    base, x = b.take([0]), v.extract(b)[:2]
+    J = engine.jacobian(base, s, v, x, method="fd")[0]
+    sc = copy.copy(s)
+    sc.constraints = systems.singlet_constraints()
+    Jc = engine.jacobian(base, sc, v, x, method="fd")[0]
+    R = residual_rows(base, s)
+    assert Jc.shape[2] == R + len(sc.constraints) and np.array_equal(Jc[:, :, :R], J)
+    sd = copy.copy(s)
+    sd.precision = abi.PRECISION_DF64
+    Jd = engine.jacobian(base, sd, v, x, method="fd")[0]
+    assert np.all(np.linalg.norm(Jd - J, axis=2) <= 1e-2 * np.linalg.norm(J, axis=2))
