@@ -2331,10 +2331,6 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 constexpr int kMaxVariablesFused = 96;
-constexpr int kFusedSlots = 4; // S / Tr slots per tuple in the workspace, one per wave (<= 4)
-#ifndef MKO_FUSED_WAVES_PER_EU
-#define MKO_FUSED_WAVES_PER_EU 3
-#endif
 
 // Per-(run, tuple) partial of the normal equations. With a per-tuple shift c (near the tuple's
 // weighted mean gradient), o (near its weighted mean OPL) and u_k = sqrt(W_k) (g_k - c) over the
@@ -2380,82 +2376,110 @@ __device__ __forceinline__ double first_lane(double x) {
     return __hiloint2double(hi, lo);
 }
 
-// Gradient sink of the fused kernel. Every column is written at most once per ray and, in hard
-// mode, at the same sweep step by every lane whose ray reached the image, so the lanes of a wave
-// write column p together: the value of the wave's first such lane (pilot) goes to pilot[p] and
-// each lane stores its difference to it in float. The float then carries the variation of the
-// gradient over the pupil, not its (often much larger) common part.
-template <int kNW>
+// Gradient sink of the fused kernel. Every lane of the wave runs the sweep (those without a
+// reached ray on a placeholder state), so column p is written by all lanes together: the value of
+// the wave's first lane with a reached ray (pilot) is kept in lane p mod 64 of the wave's pilot
+// registers and each lane stores its difference to it in float. The float then carries the
+// variation of the gradient over the pupil, not its (often much larger) common part.
+template <int kRows>
+struct Pilots {
+    int lo[kRows] = {}, hi[kRows] = {};
+    __device__ __forceinline__ double value(int h) const { return __hiloint2double(hi[h], lo[h]); }
+};
+// v with lane `lane`'s value replaced by x (both wave-uniform)
+__device__ int write_lane(int x, int lane, int v) __asm("llvm.amdgcn.writelane.i32");
+template <int kNW, int kRows>
 struct SwzSink {
     unsigned char* G; // gradient block
-    double* pilot;    // [P] of this wave
-    int k;            // ray of the chunk (thread)
-    bool leader;      // first lane of the wave with a reached ray
+    Pilots<kRows>& pilots;
+    int k;      // ray of the chunk (thread)
+    int leader; // the wave's first lane with a reached ray (uniform)
     __device__ __forceinline__ void write(int p, double value) const {
         if (p < 0) return;
-        const double c = first_lane(value);
-        *reinterpret_cast<float*>(G + GradLayout<kNW>::float_off(p, k)) = float(value - c);
-        if (leader) pilot[p] = c;
+        const int lo = __builtin_amdgcn_readlane(__double2loint(value), leader);
+        const int hi = __builtin_amdgcn_readlane(__double2hiint(value), leader);
+        *reinterpret_cast<float*>(G + GradLayout<kNW>::float_off(p, k)) =
+            float(value - __hiloint2double(hi, lo));
+        if (kRows == 1 || p < 64) {
+            pilots.lo[0] = write_lane(lo, p, pilots.lo[0]);
+            pilots.hi[0] = write_lane(hi, p, pilots.hi[0]);
+        } else {
+            pilots.lo[kRows - 1] = write_lane(lo, p - 64, pilots.lo[kRows - 1]);
+            pilots.hi[kRows - 1] = write_lane(hi, p - 64, pilots.hi[kRows - 1]);
+        }
     }
 };
 
-// Lane k's value of x (k wave-uniform).
-__device__ __forceinline__ double lane_value(double x, int k) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(x), k);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), k);
+// Orders a wave's LDS accesses across its lanes (they execute in order; this keeps the compiler
+// from moving them).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Value of lane I of the caller's row of 16 lanes.
+template <int I>
+__device__ __forceinline__ double row_lane(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x150 + I, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x150 + I, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
 
-// Row sums of one wave's 64 rays in the gradient block, transposed: lane p returns
-// A[h] = sum_k W_k G[p'][k] and B[h] = sum_k V_k G[p'][k] for row p' = p + 64 h (h < kRows), G the
-// stored floats of ray k of the wave, W_k and V_k lane k's values, summed in ray order (one FMA
-// chain per row). Each lane reads its row's 64 floats as 16-byte words; rows >= P give 0.
+// Row sums of one wave's 64 rays in the gradient block: A[h] = sum_k W_k G[p][k] and
+// B[h] = sum_k V_k G[p][k] for row p = lane + 64 h, G the stored floats of ray k of the wave, W_k and
+// V_k lane k's values. 16 rows at a time: a row of 16 lanes takes the rays of its own 16 lanes
+// (their W and V broadcast along the row once), 16-byte words of G; then the four rows of lanes
+// are added. One lane per row with W and V by readlane took twice the instructions (16 of 64 lanes
+// idle at 48 rows, four readlanes per ray).
 template <int kNW, int kRows>
 __device__ __forceinline__ void wave_row_sums(const unsigned char* G, int Pn, int wave, int lane,
-                                              double wk, double vk, double (&A)[2],
-                                              double (&B)[2]) {
+                                              double wk, double vk, double (&A)[kRows],
+                                              double (&B)[kRows]) {
     using Lay = GradLayout<kNW>;
-    A[0] = A[1] = B[0] = B[1] = 0.0;
+    const int r = lane & 15, seg = lane >> 4;
+    double w[16], v[16];
+    const auto spread = [&](auto I) {
+        constexpr int i = decltype(I)::value;
+        w[i] = row_lane<i>(wk);
+        v[i] = row_lane<i>(vk);
+    };
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (spread(std::integral_constant<int, I>{}), ...);
+    }(std::make_integer_sequence<int, 16>{});
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        A[h] = B[h] = 0.0;
 #pragma unroll 1
-    for (int j = 0; j < 8; ++j) {
-        float gv[kRows][8];
+        for (int q = 0; q < 4; ++q) {
+            const int first = 64 * h + 16 * q;
+            if (first >= Pn) break; // uniform
+            const int p = min(first + r, Pn - 1); // rows >= P: the last one again, not used
+            const unsigned char* row = G + size_t(p) * Lay::kRowBytes;
+            double a = 0.0, b = 0.0;
 #pragma unroll
-        for (int h = 0; h < kRows; ++h) {
-            const int p = lane + 64 * h;
-            float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f), y = x;
-            if (p < Pn) {
-                const unsigned char* at =
-                    G + size_t(p) * Lay::kRowBytes + 32 * ((8 * wave + j) ^ (p & Lay::kMask));
-                x = *reinterpret_cast<const float4*>(at);
-                y = *reinterpret_cast<const float4*>(at + 16);
+            for (int g2 = 0; g2 < 2; ++g2) {
+                const unsigned char* at = row + 32 * ((8 * wave + 2 * seg + g2) ^ (p & Lay::kMask));
+                const float4 x = *reinterpret_cast<const float4*>(at);
+                const float4 y = *reinterpret_cast<const float4*>(at + 16);
+                const float gv[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const double g = double(gv[i]);
+                    a = __fma_rn(w[8 * g2 + i], g, a);
+                    b = __fma_rn(v[8 * g2 + i], g, b);
+                }
             }
-            gv[h][0] = x.x; gv[h][1] = x.y; gv[h][2] = x.z; gv[h][3] = x.w;
-            gv[h][4] = y.x; gv[h][5] = y.y; gv[h][6] = y.z; gv[h][7] = y.w;
-        }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const double w = lane_value(wk, 8 * j + i), v = lane_value(vk, 8 * j + i);
-#pragma unroll
-            for (int h = 0; h < kRows; ++h) {
-                const double g = double(gv[h][i]);
-                A[h] = __fma_rn(w, g, A[h]);
-                B[h] = __fma_rn(v, g, B[h]);
+            for (int off = 16; off <= 32; off <<= 1) {
+                a += __shfl_xor(a, off, 64);
+                b += __shfl_xor(b, off, 64);
+            }
+            if (seg == q) {
+                A[h] = a;
+                B[h] = b;
             }
         }
     }
-}
-
-template <int kNW, class T>
-__device__ __forceinline__ T block_sum_n(T v, T* lds) {
-    v = wave_sum(v);
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) lds[wave] = v;
-    __syncthreads();
-    T total = lds[0];
-#pragma unroll
-    for (int w = 1; w < kNW; ++w) total += lds[w];
-    __syncthreads();
-    return total;
 }
 
 // C tile t of the upper triangle of a tg x tg grid of 32 x 32 tiles, row-major: (I, J), I <= J.
@@ -2468,103 +2492,68 @@ __device__ __forceinline__ void tile_of(int t, int tg, int& I, int& J) {
     J = I + t;
 }
 
-// C of one 32 x 32 tile over the chunk's rays: operand lane = (m = lane % 32, kb = lane / 32),
-// 8 rays per operand, hi*hi + hi*lo + lo*hi; on the diagonal the B operands are the A operands.
-template <int kNW>
-__device__ __forceinline__ void tile_products(const unsigned char* G, int Pn, int I, int J,
-                                              int lane, f32x16& acc) {
-    using Lay = GradLayout<kNW>;
-    const int m = lane & 31, kb = lane >> 5;
-    const int pa = I * 32 + m, pb = J * 32 + m;
-    // lanes of rows >= P (the padding of the tile) load nothing and take zeros
-    const bool va = pa < Pn, vb = pb < Pn;
-    bf16x8 zero;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) zero[e] = __builtin_bit_cast(__bf16, uint16_t(0));
-#pragma unroll 4
-    for (int step = 0; step < Lay::kRow / 16; ++step) {
-        const int grp = 2 * step + kb;
-        bf16x8 ahi = zero, alo = zero;
-        if (va) {
-            const int s = Lay::slot(grp, pa);
-            ahi = *reinterpret_cast<const bf16x8*>(G + Lay::hi_off(pa, s));
-            alo = *reinterpret_cast<const bf16x8*>(G + Lay::lo_off(pa, s));
-        }
-        bf16x8 bhi = ahi, blo = alo;
-        if (I != J) {
-            bhi = zero;
-            blo = zero;
-            if (vb) {
-                const int s = Lay::slot(grp, pb);
-                bhi = *reinterpret_cast<const bf16x8*>(G + Lay::hi_off(pb, s));
-                blo = *reinterpret_cast<const bf16x8*>(G + Lay::lo_off(pb, s));
-            }
-        }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, bhi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, blo, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(alo, bhi, acc, 0, 0, 0);
-    }
-}
-
-// C tile out: lane holds column n = lane % 32 of rows 8 (e / 4) + 4 (lane / 32) + e % 4.
-__device__ __forceinline__ void store_tile(float* C, int Pn, int I, int J, int lane,
-                                           const f32x16& acc) {
-    const int col = J * 32 + (lane & 31);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int row = I * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-        if (row < Pn && col < Pn) C[size_t(row) * Pn + col] = acc[e];
-    }
-}
-
 // Dynamic LDS of adjoint_normal_kernel<kNW> for P variables and S surfaces: the step table, the
-// gradient block, then the waves' pilots [kNW][P] and the shift [P] (doubles). The table is sized
-// by the batch: at 25 surfaces and 48 variables a workgroup of 4 waves takes 53.2 KB and three
-// fit a CU, with a table for 64 surfaces two (2.69 instead of 2.26 ms per 512 runs).
+// gradient block (at least the 4 KB per wave that the waves' sums of a tile take at the end), then
+// one double per variable and wave. The table is sized by the batch: at 25 surfaces and 48
+// variables a workgroup of 4 waves takes 52.8 KB and three fit a CU, with a table for 64 surfaces
+// two (2.69 instead of 2.26 ms per 512 runs).
+template <int kNW>
+constexpr size_t fused_block_bytes(int Pn) {
+    const size_t block = size_t(Pn) * GradLayout<kNW>::kRowBytes, tiles = size_t(kNW) * 4096;
+    return kNW > 1 && block < tiles ? tiles : block;
+}
 template <int kNW>
 constexpr size_t fused_lds_bytes(int Pn, int S) {
-    return size_t(S + 1) * sizeof(Step) + size_t(Pn) * GradLayout<kNW>::kRowBytes +
-           size_t(kNW + 1) * Pn * sizeof(double);
+    return size_t(S + 1) * sizeof(Step) + fused_block_bytes<kNW>(Pn) +
+           size_t(kNW) * Pn * sizeof(double);
 }
 
 // One workgroup of kNW waves per (run, tuple); the tuple's rays in chunks of 64 kNW, one ray per
-// thread. Per chunk: the forward trace in double (or, kStates, the last state and OPL of each ray
-// from a MERIT trace of the same point, mko_internal::RayStates), the reverse sweep over
-// reconstructed states into the LDS gradient block (pilot-relative floats); S and Tr of each
-// wave's rays in FP64 by transposed wave sums (per-lane accumulators, summed over the waves in
-// index order at the end); the block rewritten in place as bf16 hi / lo; C on MFMA
-// (v_mfma_f32_32x32x16_bf16, 3 products, the upper tiles of the 32 x 32 tile grid spread over
-// the waves; kPMax 96: up to 3 x 3 tiles). The shift c is the weight-averaged pilot of the waves
-// of the first chunk that holds a reached ray, o its weighted mean OPL. kStream (kNW 1, tuples of
-// at most 64 rays, one chunk): the wave's tiles are formed and stored one after another.
+// thread. A wave keeps to its own 64 rays of a chunk, so that after the first chunk the waves run
+// without barriers and one wave's sweep overlaps another's products. Per chunk: the forward trace
+// in double (or, kStates, the last state and OPL of each ray from a MERIT trace of the same point,
+// mko_internal::RayStates; the next chunk's are loaded while this one is worked on), the reverse
+// sweep into the LDS gradient block (pilot-relative floats); S and Tr of the wave's rays in FP64
+// from row sums, lane p holding variable p's (p + 64 in a second set); the wave's part of the
+// block rewritten in place as bf16 hi / lo, 8 rays of a row per lane; C on MFMA
+// (v_mfma_f32_32x32x16_bf16, 3 products, every upper tile of the 32 x 32 tile grid in each wave).
+// At the end the waves' C, S and Tr are added in wave order through the LDS. The shift c is the
+// weighted mean gradient of the first chunk that holds a reached ray, o its weighted mean OPL; its
+// exchange between the waves is the chunk loop's only barriers. kNW 1: tuples of at most 64 rays,
+// one chunk.
+// What bounds it: FP64 issue on the vector ALU; 3 waves per SIMD (LDS: 192 bytes per ray at 48
+// variables), 2 above 64 variables, whose 6 tiles take 96 registers. Measured against tiles spread
+// over the waves, a barrier between every phase, a ray per lane in the conversion and S and Tr
+// slots per wave in memory: 256 runs x 17920 rays x 48 variables on stored states 0.85 -> 0.81 ms,
+// 512 runs with their own trace 2.21 -> 2.04, 301 runs of 20 tuples of 48 rays 0.058 -> 0.047; the
+// sweep with its sink is 112 of the vector instructions per ray-surface.
 template <int kNW, int kPMax, bool kStates, bool kGlass>
-__global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(MKO_FUSED_WAVES_PER_EU)))
-void adjoint_normal_kernel(TraceParams P, ParamMap map,
-                                                                  float* partC, double* partST,
-                                                                  TupleNormal* partT,
-                                                                  mko_internal::RayStates states) {
+__global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(kPMax > 64 ? 2 : 3)))
+void adjoint_normal_kernel(TraceParams P, ParamMap map, float* partC, double* partST,
+                           TupleNormal* partT, mko_internal::RayStates states) {
     using Lay = GradLayout<kNW>;
     constexpr int kThreads = 64 * kNW;
     constexpr int kTileGrid = (kPMax + 31) / 32;
-    constexpr int kTilesAll = kTileGrid * (kTileGrid + 1) / 2;
-    constexpr bool kStream = kNW == 1;
-    constexpr int kTiles = kStream ? 1 : (kTilesAll + kNW - 1) / kNW;
-    constexpr int kGroups = (kPMax + 15) / 16;
+    constexpr int kTiles = kTileGrid * (kTileGrid + 1) / 2;
+    constexpr int kRows = kPMax > 64 ? 2 : 1; // variables per lane
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ double red[kNW];
     __shared__ double wsum_l[kNW], osum_l[kNW];
     if (P.live && int(blockIdx.x) / P.T >= *P.live) return;
     const Tuple t = tuple_of(P, blockIdx.x);
     Step* L = reinterpret_cast<Step*>(lds);
     stage_steps(P, t.v, t.l, L);
-    __syncthreads();
     const int Pn = map.P;
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = kNW == 1 ? 0 : tid >> 6;
     unsigned char* G = lds + size_t(P.S + 1) * sizeof(Step);
-    double* pilot = reinterpret_cast<double*>(G + size_t(Pn) * Lay::kRowBytes);
-    double* shift = pilot + kNW * Pn;
-    double* own_pilot = pilot + wave * Pn;
+    double* xchg = reinterpret_cast<double*>(G + fused_block_bytes<kNW>(Pn)); // [kNW][P]
+    // every column that a sweep reaches is written for every ray; the others stay zero
+    {
+        float4* z = reinterpret_cast<float4*>(G);
+        const int words = Pn * (Lay::kRowBytes / 16);
+        for (int e = tid; e < words; e += kThreads) z[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    __syncthreads();
     const size_t vf = size_t(t.v) * P.F + t.f;
     // block-uniform values in scalar registers (they stay live across the sweep)
     const double a = first_lane(P.pupil_radius[t.v]);
@@ -2576,56 +2565,48 @@ void adjoint_normal_kernel(TraceParams P, ParamMap map,
     const double kappa =
         first_lane(P.ref_kind != MKO_REF_LAST_SURFACE ? P.reference_curvature[vf] : 0.0);
     const int tg = (Pn + 31) / 32;
-    const int ntiles = tg * (tg + 1) / 2;
     const size_t tuple = size_t(blockIdx.x);
     f32x16 acc[kTiles];
 #pragma unroll
     for (int i = 0; i < kTiles; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-    // this wave's slot of the tuple's S and Tr in the workspace ([tuple][4][2 P]): each chunk adds
-    // its sums (the first one stores), so no accumulator stays live across the sweeps
-    double* slot_st = partST + (tuple * kFusedSlots + wave) * 2 * Pn;
-    bool accumulated = false;
+    double S_p[kRows] = {}, T_p[kRows] = {}, shift[kRows] = {};
     double sw = 0.0, swo = 0.0, o_shift = 0.0;
     bool shift_ready = false;
-    const int nchunks = (t.n + kThreads - 1) / kThreads;
+    const int nchunks = kNW == 1 ? 1 : (t.n + kThreads - 1) / kThreads;
     // when the tuple's spoke count divides the chunk, a lane's spoke (k mod M) is the same in every
     // chunk: its angle is formed once here and a ray's sample needs only its ring (the same
     // functions as sample_of, hence the same bits)
     const bool fixed_spoke = !kStates && kThreads % t.M == 0;
     Sample spoke{};
     if (fixed_spoke) spoke_of(P, t, tid % t.M, spoke);
+    double st[7];
+    const auto load_states = [&](int k) {
+        st[6] = __builtin_nan("");
+        if (k < t.n) {
+            const double* at = states.data + state_index(states, t.v, 0, t.offset + k);
+            const int64_t stride = states.slots * states.rays;
+#pragma unroll
+            for (int c = 0; c < 7; ++c) st[c] = at[c * stride];
+        }
+    };
+    if constexpr (kStates) load_states(tid);
     for (int ch = 0; ch < nchunks; ++ch) {
         const int k = ch * kThreads + tid;
-        double st[7];
-        if constexpr (kStates) {
-            st[6] = __builtin_nan("");
-            if (k < t.n) {
-                const int64_t row = t.offset + k;
-#pragma unroll
-                for (int c = 0; c < 7; ++c) st[c] = states.data[state_index(states, t.v, c, row)];
-            }
-        }
-        // the block (all threads, 16-byte words) and this wave's pilots start at zero
-        {
-            float4* z = reinterpret_cast<float4*>(G);
-            const int words = Pn * (Lay::kRowBytes / 16);
-            for (int e = tid; e < words; e += kThreads) z[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-        for (int p = lane; p < Pn; p += 64) own_pilot[p] = 0.0;
-        __syncthreads();
         double wk = 0.0, opl = 0.0;
         bool ok = false;
-        Sample smp{};
-        LastState last;
+        LastState last{V3<double>{0.0, 0.0, 0.0}, V3<double>{0.0, 0.0, 1.0}, 0};
         if (k < t.n) {
+            Sample smp{};
             if constexpr (kStates) {
                 ring_of(P, t, k / t.M, smp);
                 opl = st[6];
                 ok = !__builtin_isnan(opl);
-                last.p = V3<double>{st[0], st[1], st[2]};
-                last.d = V3<double>{st[3], st[4], st[5]};
+                if (ok) {
+                    last.p = V3<double>{st[0], st[1], st[2]};
+                    last.d = V3<double>{st[3], st[4], st[5]};
+                }
             } else {
                 if (fixed_spoke) {
                     smp = spoke;
@@ -2639,17 +2620,25 @@ void adjoint_normal_kernel(TraceParams P, ParamMap map,
                      MKO_STATUS_OK;
                 opl = r.opl;
             }
+            wk = ok ? smp.weight : 0.0;
         }
+        Pilots<kRows> pilots;
+        if (!ok) opl = 0.0;
+        sw += wk;
+        swo += wk * opl;
         const uint64_t okmask = __ballot(ok);
-        if (ok) {
-            wk = smp.weight;
-            sw += wk;
-            swo += wk * opl;
-            const bool leader = lane == int(__builtin_ctzll(okmask));
+        if (okmask) { // uniform
             sweep_ray<kGlass, false>(P, L, map, last.p, last.d, M, kappa,
-                              SwzSink<kNW>{G, own_pilot, tid, leader}, t.l);
+                                     SwzSink<kNW, kRows>{G, pilots, tid,
+                                                         int(__builtin_ctzll(okmask))},
+                                     t.l);
         }
-        __syncthreads();
+        if (!ok)
+            for (int p = 0; p < Pn; ++p)
+                *reinterpret_cast<float*>(G + Lay::float_off(p, tid)) = 0.0f;
+        if constexpr (kStates)
+            if (ch + 1 < nchunks) load_states(k + kThreads);
+        wave_sync();
         // this wave's weight sum W_w; the first chunk with a reached ray fixes o = sum W OPL / W
         const double ww = wave_sum(wk);
         double W = 0.0;
@@ -2666,167 +2655,185 @@ void adjoint_normal_kernel(TraceParams P, ParamMap map,
                 W += wsum_l[w];
                 WO += osum_l[w];
             }
-            if (!(W > 0.0)) continue; // no reached ray yet: nothing of this chunk counts
+            if (!(W > 0.0)) { // no reached ray yet: nothing of this chunk counts
+                __syncthreads();
+                continue;
+            }
             o_shift = WO / W;
         }
         // A_p = sum_k W_k G_pk and B_p = sum_k W_k (OPL_k - o) G_pk over the wave's rays, G the
         // stored floats relative to the wave's pilot: the parts of S and Tr that do not depend on
         // the shift c (S = A + (pilot - c) W_w, Tr = B + (pilot - c) V_w)
-        const double ow = ok ? opl - o_shift : 0.0;
-        const double vk = wk * ow;
-        double A[2], B[2];
-        if constexpr (kPMax > 64) {
-            if (Pn > 64) wave_row_sums<kNW, 2>(G, Pn, wave, lane, wk, vk, A, B);
-            else wave_row_sums<kNW, 1>(G, Pn, wave, lane, wk, vk, A, B);
-        } else {
-            wave_row_sums<kNW, 1>(G, Pn, wave, lane, wk, vk, A, B);
-        }
+        const double vk = ok ? wk * (opl - o_shift) : 0.0;
+        double A[kRows], B[kRows];
+        wave_row_sums<kNW, kRows>(G, Pn, wave, lane, wk, vk, A, B);
         const double vw = wave_sum(vk);
         if (!shift_ready) {
-            // c0: the weight-averaged pilot of the waves; then c = c0 + S0 / W with S0 the sum of
-            // W (g - c0) over the chunk, i.e. the chunk's weighted mean gradient (the waves' S0
-            // pass through their slots of the workspace, summed in wave order)
-            for (int p = tid; p < Pn; p += kThreads) {
-                double c = 0.0;
+            // c = sum_w (W_w pilot_w + A_w) / W, the chunk's weighted mean gradient
 #pragma unroll
-                for (int w = 0; w < kNW; ++w) c += wsum_l[w] * pilot[w * Pn + p];
-                shift[p] = c / W;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < kRows; ++h) {
                 const int p = lane + 64 * h;
-                if (p < Pn) slot_st[p] = A[h] + (own_pilot[p] - shift[p]) * ww;
+                if (p < Pn)
+                    xchg[wave * Pn + p] = __fma_rn(ww, pilots.value(h), A[h]);
             }
-            __threadfence_block();
             __syncthreads();
-            for (int p = tid; p < Pn; p += kThreads) {
-                const double* st0 = partST + tuple * kFusedSlots * 2 * Pn + p;
-                double s0 = st0[0];
 #pragma unroll
-                for (int w = 1; w < kNW; ++w) s0 += st0[w * 2 * Pn];
-                shift[p] += s0 / W;
+            for (int h = 0; h < kRows; ++h) {
+                const int p = lane + 64 * h;
+                if (p < Pn) {
+                    double c = xchg[p];
+#pragma unroll
+                    for (int w = 1; w < kNW; ++w) c += xchg[w * Pn + p];
+                    shift[h] = c / W;
+                }
             }
             shift_ready = true;
-            __syncthreads();
         }
-        // S and Tr of this wave's rays into its slot; the wave's deltas pilot - c, as floats
-        // over its pilots (read by the bf16 conversion below)
-        float* delta = reinterpret_cast<float*>(own_pilot);
-        double d[2] = {0.0, 0.0};
+        // S and Tr of the wave's rays; delta = pilot - c for the bf16 conversion
+        float delta[kRows];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int p = lane + 64 * h;
-            if (p < Pn) {
-                d[h] = own_pilot[p] - shift[p];
-                double* dst = slot_st + p;
-                const double s = A[h] + d[h] * ww, tr = B[h] + d[h] * vw;
-                dst[0] = accumulated ? dst[0] + s : s;
-                dst[Pn] = accumulated ? dst[Pn] + tr : tr;
-            }
+        for (int h = 0; h < kRows; ++h) {
+            const double d = pilots.value(h) - shift[h];
+            S_p[h] += A[h] + d * ww;
+            T_p[h] += B[h] + d * vw;
+            delta[h] = float(d);
         }
-        __syncthreads();
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int p = lane + 64 * h;
-            if (p < Pn) delta[p] = float(d[h]);
-        }
-        __syncthreads();
-        accumulated = true;
-        // u = sqrt(W) (g - c) of the thread's ray, split into bf16 hi + lo in place (the ray's
-        // 32-byte group belongs to 8 lanes of this wave: its floats are read before they are
-        // overwritten)
+        // u = sqrt(W) (g - c), split into bf16 hi + lo in place: a lane takes 8 rays (32 bytes) of
+        // one row at a time
         {
-            const float swk = __builtin_sqrtf(float(wk));
-            const int grp = tid >> 3, i = tid & 7;
-            // rows in blocks of 16: for p = p0 + j (p0 a multiple of 16) the swizzle p & kMask is
-            // m = j & kMask, so float_off(p, tid) = p RB + (4 tid ^ 32 m), hi_off(p, grp ^ m) + 2 i
-            // = p RB + (hbase ^ (32 m + 16 ((m >> 3) & 1))) and lo_off(...) + 2 i = that ^ 16;
-            // two rows at a time share the packed bf16 conversions
-            const int fbase = 4 * tid;
-            const int hbase = 32 * grp + 16 * ((grp >> 3) & 1) + 2 * i;
-            for (int p0 = 0; p0 < Pn; p0 += 16) {
-                unsigned char* row = G + size_t(p0) * Lay::kRowBytes;
+            const float root = __builtin_sqrtf(float(wk));
+            const int g8 = lane & 7, r8 = lane >> 3;
+            float sq[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sq[i] = __shfl(root, 8 * g8 + i, 64);
+            const int rows8 = (Pn + 7) / 8;
 #pragma unroll 2
-                for (int j = 0; j < 16; j += 2) {
-                    if (p0 + j < Pn) {
-                        const bool two = p0 + j + 1 < Pn;
-                        const int m0 = j & Lay::kMask, m1 = (j + 1) & Lay::kMask;
-                        unsigned char* r0 = row + j * Lay::kRowBytes;
-                        unsigned char* r1 = r0 + Lay::kRowBytes;
-                        f32x2 u;
-                        u.x = swk * (*reinterpret_cast<const float*>(r0 + (fbase ^ (32 * m0))) +
-                                     delta[p0 + j]);
-                        u.y = two ? swk * (*reinterpret_cast<const float*>(
-                                               r1 + (fbase ^ (32 * m1))) +
-                                           delta[p0 + j + 1])
-                                  : 0.0f;
-                        const bf16x2 hi = __builtin_convertvector(u, bf16x2);
-                        const f32x2 d{u.x - float(hi[0]), u.y - float(hi[1])};
-                        const bf16x2 lo = __builtin_convertvector(d, bf16x2);
-                        const int h0 = hbase ^ (32 * m0 + 16 * ((m0 >> 3) & 1));
-                        const int h1 = hbase ^ (32 * m1 + 16 * ((m1 >> 3) & 1));
-                        *reinterpret_cast<__bf16*>(r0 + h0) = hi[0];
-                        *reinterpret_cast<__bf16*>(r0 + (h0 ^ 16)) = lo[0];
-                        if (two) {
-                            *reinterpret_cast<__bf16*>(r1 + h1) = hi[1];
-                            *reinterpret_cast<__bf16*>(r1 + (h1 ^ 16)) = lo[1];
-                        }
+            for (int it = 0; it < rows8; ++it) {
+                const int p = r8 + 8 * it;
+                float d = __shfl(delta[0], p & 63, 64);
+                if (kRows == 2 && it >= 8) d = __shfl(delta[kRows - 1], p & 63, 64);
+                if (p < Pn) {
+                    const int slot = Lay::slot(8 * wave + g8, p);
+                    unsigned char* at = G + size_t(p) * Lay::kRowBytes + 32 * slot;
+                    const float4 x = *reinterpret_cast<const float4*>(at);
+                    const float4 y = *reinterpret_cast<const float4*>(at + 16);
+                    const float g[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+                    bf16x8 hi, lo;
+#pragma unroll
+                    for (int i = 0; i < 8; i += 2) {
+                        const f32x2 u{sq[i] * (g[i] + d), sq[i + 1] * (g[i + 1] + d)};
+                        const bf16x2 h2 = __builtin_convertvector(u, bf16x2);
+                        const f32x2 rest{u.x - float(h2[0]), u.y - float(h2[1])};
+                        const bf16x2 l2 = __builtin_convertvector(rest, bf16x2);
+                        hi[i] = h2[0];
+                        hi[i + 1] = h2[1];
+                        lo[i] = l2[0];
+                        lo[i + 1] = l2[1];
                     }
+                    const int swap = ((slot >> 3) & 1) << 4;
+                    *reinterpret_cast<bf16x8*>(at + swap) = hi;
+                    *reinterpret_cast<bf16x8*>(at + (swap ^ 16)) = lo;
                 }
             }
         }
-        __syncthreads();
-        if constexpr (kStream) {
-            float* C = partC + tuple * size_t(Pn) * Pn;
-            for (int tt = 0; tt < ntiles; ++tt) {
-                int I, J;
-                tile_of(tt, tg, I, J);
+        wave_sync();
+        // C over the wave's 64 rays, 16 at a time: operand lane = (row lane % 32 of a 32-row block,
+        // rays 8 (lane / 32) ...), hi*hi + hi*lo + lo*hi. Rows >= P take the last row's values:
+        // their products are not stored.
+        {
+            const int m = lane & 31, kb = lane >> 5;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[0][e] = 0.0f;
-                tile_products<kNW>(G, Pn, I, J, lane, acc[0]);
-                store_tile(C, Pn, I, J, lane, acc[0]);
+            for (int step = 0; step < 4; ++step) {
+                const int grp = 8 * wave + 2 * step + kb;
+                bf16x8 hi[kTileGrid], lo[kTileGrid];
+#pragma unroll
+                for (int I = 0; I < kTileGrid; ++I) {
+                    const int p = min(I * 32 + m, Pn - 1);
+                    const int slot = Lay::slot(grp, p);
+                    hi[I] = *reinterpret_cast<const bf16x8*>(G + Lay::hi_off(p, slot));
+                    lo[I] = *reinterpret_cast<const bf16x8*>(G + Lay::lo_off(p, slot));
+                }
+                int i = 0;
+#pragma unroll
+                for (int I = 0; I < kTileGrid; ++I)
+#pragma unroll
+                    for (int J = I; J < kTileGrid; ++J, ++i) {
+                        if (J >= tg) continue; // uniform
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi[I], hi[J], acc[i], 0, 0, 0);
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi[I], lo[J], acc[i], 0, 0, 0);
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo[I], hi[J], acc[i], 0, 0, 0);
+                    }
             }
-        } else {
+        }
+        wave_sync();
+    }
+    // the waves' sums added in wave order. A tile's lane holds column n = lane % 32 of rows
+    // 8 (e / 4) + 4 (lane / 32) + e % 4.
+    float* C = partC + tuple * size_t(Pn) * Pn;
+    int i = 0;
 #pragma unroll
-            for (int i = 0; i < kTiles; ++i) {
-                const int tt = wave + i * kNW;
-                if (tt < ntiles) {
-                    int I, J;
-                    tile_of(tt, tg, I, J);
-                    tile_products<kNW>(G, Pn, I, J, lane, acc[i]);
+    for (int I = 0; I < kTileGrid; ++I)
+#pragma unroll
+        for (int J = I; J < kTileGrid; ++J, ++i) {
+            if (J >= tg) continue; // uniform
+            const auto put = [&](int e, float value) {
+                const int row = I * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+                const int col = J * 32 + (lane & 31);
+                if (row < Pn && col < Pn) C[size_t(row) * Pn + col] = value;
+            };
+            if constexpr (kNW == 1) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) put(e, acc[i][e]);
+            } else {
+                float* X = reinterpret_cast<float*>(G); // [kNW][16][64]
+                __syncthreads();
+#pragma unroll
+                for (int e = 0; e < 16; ++e) X[(wave * 16 + e) * 64 + lane] = acc[i][e];
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < 16 / kNW; ++q) {
+                    const int e = wave * (16 / kNW) + q;
+                    float x = X[e * 64 + lane];
+#pragma unroll
+                    for (int w = 1; w < kNW; ++w) x += X[(w * 16 + e) * 64 + lane];
+                    put(e, x);
                 }
             }
         }
-        __syncthreads();
+    sw = wave_sum(sw);
+    swo = wave_sum(swo);
+    double* X = reinterpret_cast<double*>(G); // [kNW][2 P]
+    __syncthreads();
+    if (lane == 0) {
+        wsum_l[wave] = sw;
+        osum_l[wave] = swo;
     }
-    if constexpr (kStream) {
-        if (!shift_ready) {
-            // no reached ray in the tuple: C = 0
-            float* C = partC + tuple * size_t(Pn) * Pn;
-            for (int e = tid; e < Pn * Pn; e += kThreads) C[e] = 0.0f;
-        }
-    } else {
-        float* C = partC + tuple * size_t(Pn) * Pn;
 #pragma unroll
-        for (int i = 0; i < kTiles; ++i) {
-            const int tt = wave + i * kNW;
-            if (tt < ntiles) {
-                int I, J;
-                tile_of(tt, tg, I, J);
-                store_tile(C, Pn, I, J, lane, acc[i]);
-            }
+    for (int h = 0; h < kRows; ++h) {
+        const int p = lane + 64 * h;
+        if (p < Pn) {
+            X[wave * 2 * Pn + p] = S_p[h];
+            X[wave * 2 * Pn + Pn + p] = T_p[h];
         }
     }
-    const double w_ok = block_sum_n<kNW>(sw, red);
-    const double sum = block_sum_n<kNW>(swo, red);
-    // a tuple without a reached ray: its slots hold zeros (the finalize sums kNW slots)
-    if (!accumulated)
-        for (int e = lane; e < 2 * Pn; e += 64) slot_st[e] = 0.0;
+    __syncthreads();
+    double* slot_st = partST + tuple * 2 * Pn;
+    for (int e = tid; e < 2 * Pn; e += kThreads) {
+        double x = X[e];
+#pragma unroll
+        for (int w = 1; w < kNW; ++w) x += X[w * 2 * Pn + e];
+        slot_st[e] = x;
+    }
     if (tid == 0) {
-        const bool valid = w_ok > 0.0;
+        double w_ok = wsum_l[0], sum = osum_l[0];
+#pragma unroll
+        for (int w = 1; w < kNW; ++w) {
+            w_ok += wsum_l[w];
+            sum += osum_l[w];
+        }
         // piston - o, the OPL shift of Tr
-        partT[tuple] = TupleNormal{w_ok, valid ? sum / w_ok - o_shift : 0.0, t.scale * t.scale};
+        partT[tuple] = TupleNormal{w_ok, w_ok > 0.0 ? sum / w_ok - o_shift : 0.0,
+                                   t.scale * t.scale};
     }
 }
 
@@ -2842,8 +2849,8 @@ constexpr int kFinalizeEntries = (kMaxVariablesFused * (kMaxVariablesFused + 1) 
 
 template <int kE>
 __global__ __launch_bounds__(256) void adjoint_normal_finalize_kernel(
-    int T, int Pn, int slots, const float* partC, const double* partST, const TupleNormal* partT,
-    double* a, double* g, const int32_t* live) {
+    int T, int Pn, const float* partC, const double* partST, const TupleNormal* partT, double* a,
+    double* g, const int32_t* live) {
     __shared__ double S_l[kFinalizeChunk][2 * kMaxVariablesFused];
     __shared__ double f1[kFinalizeChunk], f2[kFinalizeChunk], pist[kFinalizeChunk];
     const int v = blockIdx.x;
@@ -2869,12 +2876,8 @@ __global__ __launch_bounds__(256) void adjoint_normal_finalize_kernel(
     for (int t0 = 0; t0 < T; t0 += kFinalizeChunk) {
         const int nt = min(kFinalizeChunk, T - t0);
         for (int e = tid; e < nt * 2 * Pn; e += 256) {
-            // the waves' slots of S and Tr, summed in wave order
             const int tt = e / (2 * Pn), i = e - tt * 2 * Pn;
-            const double* st = partST + (size_t(v) * T + t0 + tt) * kFusedSlots * 2 * Pn + i;
-            double x = st[0];
-            for (int w = 1; w < slots; ++w) x += st[w * 2 * Pn];
-            S_l[tt][i] = x;
+            S_l[tt][i] = partST[(size_t(v) * T + t0 + tt) * 2 * Pn + i];
         }
         if (tid < nt) {
             const TupleNormal tn = partT[size_t(v) * T + t0 + tid];
@@ -3564,7 +3567,7 @@ int adjoint_normal_states(const mko_batch* batch, const mko_residual_settings* s
         double* partST = reinterpret_cast<double*>(w + up(tuples * m.P * m.P * sizeof(float)));
         TupleNormal* partT = reinterpret_cast<TupleNormal*>(
             w + up(tuples * m.P * m.P * sizeof(float)) +
-            up(tuples * kFusedSlots * 2 * m.P * sizeof(double)));
+            up(tuples * 2 * m.P * sizeof(double)));
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const int nw = fused_waves(P, waves ? waves : g_tuning.fused_waves);
         if (states.data) {
@@ -3581,7 +3584,7 @@ int adjoint_normal_states(const mko_batch* batch, const mko_residual_settings* s
         const auto finalize = nu <= 5 * 256    ? adjoint_normal_finalize_kernel<5>
                               : nu <= 10 * 256 ? adjoint_normal_finalize_kernel<10>
                                                : adjoint_normal_finalize_kernel<kFinalizeEntries>;
-        hipLaunchKernelGGL(finalize, dim3(unsigned(P.V)), dim3(256), 0, s, P.T, m.P, nw, partC,
+        hipLaunchKernelGGL(finalize, dim3(unsigned(P.V)), dim3(256), 0, s, P.T, m.P, partC,
                            partST, partT, a, g, live);
         check_hip(hipGetLastError(), "adjoint normal finalize launch");
     })
@@ -4066,7 +4069,7 @@ size_t mko_adjoint_normal_workspace(int variants, int fields, int wavelengths, i
     const size_t tuples = size_t(variants) * size_t(fields) * size_t(wavelengths);
     const size_t P = size_t(variables);
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-    return up(tuples * P * P * sizeof(float)) + up(tuples * kFusedSlots * 2 * P * sizeof(double)) +
+    return up(tuples * P * P * sizeof(float)) + up(tuples * 2 * P * sizeof(double)) +
            up(tuples * sizeof(TupleNormal));
 }
 
