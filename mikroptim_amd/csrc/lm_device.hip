@@ -8,11 +8,10 @@
 // square root (__ddiv_rn, __dsqrt_rn), std::max / std::min as (a < b) ? b : a / (b < a) ? b : a.
 // Given the same normal equations and merits, device and host control take bit-identical
 // trajectories. Sums keep the host order (that of the reference's cholesky / cholesky_solve,
-// src/optim/levenberg_marquardt.cpp:70-112): the Cholesky factor (right-looking) and the forward
-// substitution run lane-parallel over rows, each entry receiving its subtractions in the host's
-// order; the back substitution forms each row's products on the lanes and subtracts them in
-// ascending order; the step model (lin, quad) runs on lane 0; maxima (order-independent) are
-// wave reductions.
+// src/optim/levenberg_marquardt.cpp:70-112): the Cholesky factor and the forward substitution run
+// lane-parallel over rows, each entry receiving its subtractions in the host's order; the back
+// substitution and the step model (lin, quad) form their products on the lanes and add them in
+// ascending order; maxima (order-independent) are wave reductions.
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -53,222 +52,253 @@ __device__ __forceinline__ double wave_max(double v) {
     return v;
 }
 
-// Packed lower triangle of an f x f matrix, column-major: element (row i, column j), i >= j.
-__device__ __forceinline__ int tri(int j, int i, int f) { return j * f - (j * (j - 1)) / 2 + (i - j); }
-// entries of the packed lower triangle of a P x P matrix
-__host__ __device__ __forceinline__ int tri_size(int P) { return P * (P + 1) / 2; }
-
-struct SolveScalars {
-    double diag;
-    int f;
-};
-
-// The solve's per-variable arrays, P entries each, in the dynamic LDS after the packed triangle
-// and its row / column bytes (sized by P, not by the largest P: more runs' workgroups fit a CU).
-struct SolveLds {
-    double* rhs;
-    double* delta;
-    double* step;
-    double* aq;
-    double* ratio;
-    double* col; // column j of the Cholesky factor while rows below it are updated
-    int* idx;
-    uint8_t* fixed;
-    double& diag;
-    int& f;
-};
-
-__host__ __device__ __forceinline__ size_t solve_arrays_offset(int P) {
-    return (size_t(tri_size(P)) * (sizeof(double) + 2) + 7) / 8 * 8;
+// Orders the wave's LDS accesses across its lanes (one wavefront per workgroup: they execute in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ SolveLds solve_lds(double* m, int P, SolveScalars& sc) {
-    double* v = reinterpret_cast<double*>(reinterpret_cast<unsigned char*>(m) +
-                                          solve_arrays_offset(P));
-    int* idx = reinterpret_cast<int*>(v + 6 * size_t(P));
-    return SolveLds{v,          v + P,     v + 2 * P, v + 3 * P,
-                    v + 4 * P,  v + 5 * P, idx,       reinterpret_cast<uint8_t*>(idx + P),
-                    sc.diag,    sc.f};
+// The solve's LDS: the packed lower triangle of the free variables' matrix with the right-hand side
+// as one more row (columns of P + 1, P, ... 2 entries), a step per variable and the free
+// variables' indices; sized by P, so that more runs' workgroups fit a CU.
+__host__ __device__ __forceinline__ size_t solve_entries(int P) { return size_t(P + 1) * (P + 2) / 2; }
+struct SolveLds {
+    double* m;
+    double* delta;
+    int* idx;
+};
+__device__ __forceinline__ SolveLds solve_lds(double* lds, int P) {
+    double* delta = lds + solve_entries(P);
+    return SolveLds{lds, delta, reinterpret_cast<int*>(delta + P)};
 }
 
 // solve_step: (A_FF + mu D_FF) delta_F = -g_F on the free variables with the active set; writes
 // trial, step_norm, predicted and solved of the run (trial, step_norm and predicted only when
 // the factorisation succeeds, like the host).
-// a, g: the run's normal equations (row-major a[q * P + p]). Variable k belongs to lane k % 64,
-// slot k / 64 (two slots: up to 128 variables); values a lane keeps per variable sit in
-// two-element arrays indexed by the slot.
+// a, g: the run's normal equations (a symmetric). Variable k, and row i of the free variables'
+// matrix, belong to lane k % 64, slot k / 64 (two slots: up to 127 variables and the right-hand
+// side's row).
+//
+// One wave works through dependent chains, so what bounds it is their latency, not the arithmetic
+// (0.04 MFLOP at 48 variables): the matrix is loaded 8 columns at a time, the Cholesky is
+// left-looking as the host's (a column's products are loaded 8 at a time ahead of the chain of
+// subtractions, no index tables, no barriers), the right-hand side rides along as its last row
+// (the forward substitution's operations in the same order), and the sums of the step's model are
+// chains over values from other lanes' registers. 256 runs of 48 variables: 150 -> 120 us (a CU
+// holds one wave then; half of it issue, half latency).
 __device__ void solve_step(const State& S, int run, const double* a, const double* g, double mu,
-                           SolveLds& L, double* __restrict__ m) {
+                           const SolveLds& L) {
     const int n = S.P;
     const int lane = threadIdx.x;
-    const double* x = S.x + size_t(run) * n;
-    const double* d = S.d + size_t(run) * n;
-    for (int k = lane; k < n; k += kLanes) L.fixed[k] = blocks(S, k, x[k], -g[k]) ? 1 : 0;
-    __syncthreads();
-    for (int round = 0; round <= n; ++round) {
-        if (lane == 0) {
-            int f = 0;
-            for (int k = 0; k < n; ++k)
-                if (!L.fixed[k]) L.idx[f++] = k;
-            L.f = f;
+    double* __restrict__ m = L.m;
+    double x[kSlots], delta[kSlots];
+    bool fixed[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+        const int k = lane + s * kLanes;
+        x[s] = delta[s] = 0.0;
+        fixed[s] = true;
+        if (k < n) {
+            x[s] = S.x[size_t(run) * n + k];
+            fixed[s] = blocks(S, k, x[s], -g[k]);
         }
-        for (int k = lane; k < n; k += kLanes) L.delta[k] = 0.0;
-        __syncthreads();
-        const int f = L.f;
+    }
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    for (int round = 0; round <= n; ++round) {
+        const uint64_t free0 = __ballot(!fixed[0]), free1 = __ballot(!fixed[1]);
+        const int f0 = __popcll(free0), f = f0 + __popcll(free1);
+        if (!fixed[0]) L.idx[__popcll(free0 & below)] = lane;
+        if (!fixed[1]) L.idx[f0 + __popcll(free1 & below)] = lane + kLanes;
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) delta[s] = 0.0;
         if (f == 0) break;
-        for (int j = 0; j < f; ++j) {
-            for (int i = j + ((lane - j) % kLanes + kLanes) % kLanes; i < f; i += kLanes) {
-                double v = a[size_t(L.idx[j]) * n + L.idx[i]];
-                if (i == j) v += mu * d[L.idx[j]];
-                m[tri(j, i, f)] = v;
+        wave_sync();
+        const int F = f + 1;
+        const bool two = F > kLanes; // uniform
+        // column j of the packed matrix at m + c(j), rows j ... f at their own index
+        const auto c = [&](int j) { return j * F - (j * (j - 1)) / 2 - j; };
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const int i = lane + s * kLanes;
+            if (s == 1 && !two) break;
+            const int var = i < f ? L.idx[i] : 0;
+            const double d = i < f ? S.d[size_t(run) * n + var] : 0.0;
+            for (int j0 = 0; j0 < f; j0 += 8) {
+                double v[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int j = j0 + q;
+                    v[q] = 0.0;
+                    if (j < f && i >= j && i <= f) {
+                        const int vj = L.idx[j];
+                        v[q] = i < f ? a[size_t(vj) * n + var] : -g[vj];
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int j = j0 + q;
+                    if (j < f && i >= j && i <= f) m[c(j) + i] = i == j ? v[q] + mu * d : v[q];
+                }
             }
         }
-        for (int i = lane; i < f; i += kLanes) L.rhs[i] = -g[L.idx[i]];
-        __syncthreads();
-        // row and column of every packed entry (the trailing columns' entries are spread over the
-        // lanes below)
-        {
-            uint8_t* rowof = reinterpret_cast<uint8_t*>(m + tri_size(n));
-            uint8_t* colof = rowof + tri_size(n);
-            for (int c = 0; c < f; ++c)
-                for (int i = lane; i < f; i += kLanes)
-                    if (i >= c) {
-                        const int e = tri(c, i, f);
-                        rowof[e] = uint8_t(i);
-                        colof[e] = uint8_t(c);
-                    }
+        wave_sync();
+        // Cholesky, left-looking: entry (i, j) receives the subtractions of l(i, k) l(j, k), k < j,
+        // in ascending order, as in the host's loop; the row f of the right-hand side receives
+        // those of the forward substitution, y_j = (b_j - sum_k l(j, k) y_k) / l(j, j)
+        int row[kSlots];
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const int i = lane + s * kLanes;
+            row[s] = i < f ? i : f; // lanes beyond the last row read it again
         }
-        __syncthreads();
-        // Cholesky, right-looking: after column j is final, every entry (i, k), j < k <= i,
-        // receives l(i, j) l(k, j). Each entry receives the same subtractions in the same
-        // (ascending j) order as in the host's left-looking loop, so the factor is bitwise the
-        // host's. The trailing columns j+1 ... f-1 are one contiguous range of the packed layout,
-        // whose entries are spread evenly over the lanes.
-        const uint8_t* rowof = reinterpret_cast<const uint8_t*>(m + tri_size(n));
-        const uint8_t* colof = rowof + tri_size(n);
-        const int e_end = tri(f - 1, f - 1, f) + 1;
         for (int j = 0; j < f; ++j) {
-            if (lane == (j & (kLanes - 1))) L.diag = m[tri(j, j, f)];
-            __syncthreads();
-            const double diag = L.diag;
+            const int cj = c(j);
+            double acc[kSlots];
+            acc[0] = m[cj + (row[0] < j ? j : row[0])];
+            acc[1] = two ? m[cj + (row[1] < j ? j : row[1])] : 0.0;
+            int ck = 0; // c(k)
+            int k = 0;
+            for (; k + 8 <= j; k += 8) {
+                double u[8], w0[8], w1[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    u[q] = m[ck + j];
+                    w0[q] = m[ck + row[0]];
+                    w1[q] = two ? m[ck + row[1]] : 0.0;
+                    ck += F - (k + q) - 1;
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    acc[0] -= w0[q] * u[q];
+                    if (two) acc[1] -= w1[q] * u[q];
+                }
+            }
+            for (; k < j; ++k) {
+                const double u = m[ck + j];
+                acc[0] -= m[ck + row[0]] * u;
+                if (two) acc[1] -= m[ck + row[1]] * u;
+                ck += F - k - 1;
+            }
+            const double diag = lane_value(j < kLanes ? acc[0] : acc[1], j % kLanes);
             if (!(diag > 0.0) || !isfinite(diag)) {
                 if (lane == 0) S.solved[run] = 0;
                 return;
             }
             const double l = __dsqrt_rn(diag);
-            for (int i = lane; i < f; i += kLanes) {
-                if (i == j) {
-                    m[tri(j, j, f)] = l;
-                } else if (i > j) {
-                    const double v = __ddiv_rn(m[tri(j, i, f)], l);
-                    m[tri(j, i, f)] = v;
-                    L.col[i] = v;
-                }
-            }
-            __syncthreads();
-            if (j + 1 < f) {
-                for (int e = tri(j + 1, j + 1, f) + lane; e < e_end; e += kLanes)
-                    m[e] -= L.col[rowof[e]] * L.col[colof[e]];
-            }
-            __syncthreads();
-        }
-        // forward substitution: row i subtracts l(i, k) y_k for k = 0, 1, ... as y_k is final;
-        // y_k = (row k's sum) / l(k, k) is formed in every lane alike, so no LDS round trip
-        {
-            double acc[kSlots];
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 const int i = lane + s * kLanes;
-                acc[s] = i < f ? L.rhs[i] : 0.0;
+                if (s == 1 && !two) break;
+                const double v = __ddiv_rn(acc[s], l);
+                if (i >= j && i <= f) m[cj + i] = i == j ? l : v;
             }
-            for (int k = 0; k < f; ++k) {
-                const double yk = __ddiv_rn(lane_value(k < kLanes ? acc[0] : acc[1], k % kLanes), m[tri(k, k, f)]);
-#pragma unroll
-                for (int s = 0; s < kSlots; ++s) {
-                    const int i = lane + s * kLanes;
-                    if (i == k) acc[s] = yk;
-                    else if (i > k && i < f) acc[s] -= m[tri(k, i, f)] * yk;
-                }
-            }
-#pragma unroll
-            for (int s = 0; s < kSlots; ++s) {
-                const int i = lane + s * kLanes;
-                if (i < f) L.rhs[i] = acc[s];
-            }
+            wave_sync();
         }
-        // back substitution, x_i = (b_i - sum_{k > i} l(k, i) x_k) / l(i, i) for i = f-1 ... 0:
-        // the lane of row k keeps b_k, then x_k, in a register and forms the product l(k, i) x_k;
-        // every lane subtracts the products from b_i in ascending k, as the host does, and
-        // divides, so x_i is the same in all lanes and the lane of row i keeps it (no LDS round
-        // trip between rows)
-        {
-            __syncthreads();
-            double xk[kSlots];
+        // back substitution, x_i = (y_i - sum_{k > i} l(k, i) x_k) / l(i, i) for i = f-1 ... 0:
+        // the lane of row k keeps y_k, then x_k, in a register and forms the product l(k, i) x_k;
+        // every lane subtracts the products from y_i in ascending k, as the host does, and
+        // divides, so x_i is the same in all lanes and the lane of row i keeps it
+        double xk[kSlots];
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const int k = lane + s * kLanes;
+            xk[s] = k < f ? m[c(k) + f] : 0.0;
+        }
+        for (int i = f - 1; i >= 0; --i) {
+            const int ci = c(i);
+            double p[kSlots];
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 const int k = lane + s * kLanes;
-                xk[s] = k < f ? L.rhs[k] : 0.0;
+                p[s] = (k > i && k < f) ? m[ci + k] * xk[s] : 0.0;
             }
-            for (int i = f - 1; i >= 0; --i) {
-                double p[kSlots];
+            const double lii = m[ci + i];
+            double acc = lane_value(i < kLanes ? xk[0] : xk[1], i % kLanes);
+            const int end0 = f < kLanes ? f : kLanes;
+            int k = i + 1;
+            for (; k + 8 <= end0; k += 8) {
+                double t[8];
 #pragma unroll
-                for (int s = 0; s < kSlots; ++s) {
-                    const int k = lane + s * kLanes;
-                    p[s] = (k > i && k < f) ? m[tri(i, k, f)] * xk[s] : 0.0;
-                }
-                double acc = lane_value(i < kLanes ? xk[0] : xk[1], i % kLanes);
-                for (int k = i + 1; k < f; ++k) acc -= lane_value(k < kLanes ? p[0] : p[1], k % kLanes);
-                const double xi = __ddiv_rn(acc, m[tri(i, i, f)]);
+                for (int q = 0; q < 8; ++q) t[q] = lane_value(p[0], k + q);
 #pragma unroll
-                for (int s = 0; s < kSlots; ++s)
-                    if (lane + s * kLanes == i) xk[s] = xi;
+                for (int q = 0; q < 8; ++q) acc -= t[q];
             }
+            for (; k < end0; ++k) acc -= lane_value(p[0], k);
+            for (; k < f; ++k) acc -= lane_value(p[1], k - kLanes);
+            const double xi = __ddiv_rn(acc, lii);
 #pragma unroll
-            for (int s = 0; s < kSlots; ++s) {
-                const int k = lane + s * kLanes;
-                if (k < f) L.rhs[k] = xk[s];
-            }
+            for (int s = 0; s < kSlots; ++s)
+                if (lane + s * kLanes == i) xk[s] = xi;
         }
-        __syncthreads();
-        for (int i = lane; i < f; i += kLanes) L.delta[L.idx[i]] = L.rhs[i];
-        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const int i = lane + s * kLanes;
+            if (i < f) L.delta[L.idx[i]] = xk[s];
+        }
+        wave_sync();
         bool newly_fixed = false;
-        for (int i = lane; i < f; i += kLanes) {
-            const int k = L.idx[i];
-            if (blocks(S, k, x[k], L.delta[k])) {
-                L.fixed[k] = 1;
-                newly_fixed = true;
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const int k = lane + s * kLanes;
+            if (!fixed[s]) {
+                delta[s] = L.delta[k];
+                if (blocks(S, k, x[s], delta[s])) {
+                    fixed[s] = true;
+                    newly_fixed = true;
+                }
             }
         }
-        const bool changed = __any(newly_fixed);
-        __syncthreads();
-        if (!changed) break;
+        wave_sync();
+        if (!__any(newly_fixed)) break;
     }
-    double* trial = S.trial + size_t(run) * n;
-    for (int k = lane; k < n; k += kLanes) {
-        const double t = dmin(dmax(x[k] + L.delta[k], S.lower[k]), S.upper[k]);
-        trial[k] = t;
-        L.step[k] = t - x[k];
-        L.ratio[k] = __ddiv_rn(fabs(L.step[k]), scale_of(x[k], S.typical[k]));
-    }
-    __syncthreads();
-    for (int q = lane; q < n; q += kLanes) {
-        double aq = 0.0;
-        for (int p = 0; p < n; ++p) aq += a[size_t(q) * n + p] * L.step[p];
-        L.aq[q] = aq;
-    }
-    __syncthreads();
+    double step[kSlots], lin_p[kSlots], quad_p[kSlots];
     // dmax(0, .) per variable first: a NaN ratio drops out as in the host's sequential std::max,
     // so the butterfly only sees ordered values and every lane ends with the same maximum
     double r = 0.0;
-    for (int k = lane; k < n; k += kLanes) r = dmax(r, dmax(0.0, L.ratio[k]));
-    const double nrm = wave_max(r);
-    if (lane == 0) {
-        double lin = 0.0, quad = 0.0;
-        for (int q = 0; q < n; ++q) {
-            lin += L.step[q] * g[q];
-            quad += L.step[q] * L.aq[q];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+        const int k = lane + s * kLanes;
+        step[s] = 0.0;
+        if (k < n) {
+            const double t = dmin(dmax(x[s] + delta[s], S.lower[k]), S.upper[k]);
+            S.trial[size_t(run) * n + k] = t;
+            step[s] = t - x[s];
+            const double ratio = __ddiv_rn(fabs(step[s]), scale_of(x[s], S.typical[k]));
+            r = dmax(r, dmax(0.0, ratio));
         }
+    }
+    const double nrm = wave_max(r);
+    // a q of the step model: row q of a is its column q
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+        const int q = lane + s * kLanes;
+        const int qc = q < n ? q : n - 1;
+        double aq = 0.0;
+        for (int p0 = 0; p0 < n; p0 += 8) {
+            double v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = p0 + e < n ? a[size_t(p0 + e) * n + qc] : 0.0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int p = p0 + e;
+                if (p < n)
+                    aq += v[e] * lane_value(p < kLanes ? step[0] : step[1], p % kLanes);
+            }
+        }
+        lin_p[s] = q < n ? step[s] * g[q] : 0.0;
+        quad_p[s] = step[s] * aq;
+        if (s == 0 && n <= kLanes) {
+            lin_p[1] = quad_p[1] = 0.0;
+            break;
+        }
+    }
+    double lin = 0.0, quad = 0.0;
+    for (int q = 0; q < n; ++q) {
+        lin += lane_value(q < kLanes ? lin_p[0] : lin_p[1], q % kLanes);
+        quad += lane_value(q < kLanes ? quad_p[0] : quad_p[1], q % kLanes);
+    }
+    if (lane == 0) {
         S.step_norm[run] = nrm;
         S.predicted[run] = -(2.0 * lin + quad);
         S.solved[run] = 1;
@@ -309,15 +339,18 @@ __device__ void prepare_step(const State& S, const Options& o, int run, const do
     if (lane == 0) S.gradient_norm[run] = gmax;
 }
 
-__global__ __launch_bounds__(256) void init_kernel(State S, Options o) {
-    const int run = blockIdx.x * blockDim.x + threadIdx.x;
-    if (run >= S.n) return;
+// One wavefront per run (also in update_kernel): its variables on the lanes. 256 runs of 48
+// variables: 38 -> 4 us here, 22 -> 5 us in update_kernel (a thread per run walked its variables
+// one load at a time).
+__global__ __launch_bounds__(kLanes) void init_kernel(State S, Options o) {
+    const int run = blockIdx.x;
     const int n = S.P;
-    for (int k = 0; k < n; ++k) {
+    for (int k = threadIdx.x; k < n; k += kLanes) {
         S.trial[size_t(run) * n + k] = S.x[size_t(run) * n + k];
         S.g[size_t(run) * n + k] = 0.0;
         S.d[size_t(run) * n + k] = 0.0;
     }
+    if (threadIdx.x != 0) return;
     S.mu[run] = o.initial_damping;
     S.nu[run] = 2.0;
     S.step_norm[run] = 0.0;
@@ -487,20 +520,26 @@ __global__ __launch_bounds__(kLanes) void prepare_kernel(State S, Options o, con
                                                          int count, const int32_t* dcount,
                                                          const double* a_c,
                                                          const double* g_c) {
-    __shared__ SolveScalars sc;
-    __shared__ int finite_s;
-    extern __shared__ double m_tri[]; // packed lower triangle, P (P + 1) / 2 doubles, then the
-                                      // row and column (uint8) of each entry, then the arrays
-    SolveLds L = solve_lds(m_tri, S.P, sc);
+    extern __shared__ double m_tri[];
+    const SolveLds L = solve_lds(m_tri, S.P);
     const int j = blockIdx.x;
     if (j >= count || (dcount && j >= *dcount)) return;
     const int run = list[j];
     const int n = S.P, lane = threadIdx.x;
     bool finite = true;
-    for (int e = lane; e < n * n; e += kLanes) {
-        const double v = a_c[size_t(j) * n * n + e];
-        S.a[size_t(run) * n * n + e] = v;
-        finite = finite && isfinite(v);
+    for (int e0 = lane; e0 < n * n; e0 += 8 * kLanes) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int e = e0 + q * kLanes;
+            v[q] = e < n * n ? a_c[size_t(j) * n * n + e] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int e = e0 + q * kLanes;
+            if (e < n * n) S.a[size_t(run) * n * n + e] = v[q];
+            finite = finite && isfinite(v[q]);
+        }
     }
     for (int k = lane; k < n; k += kLanes) {
         const double v = g_c[size_t(j) * n + k];
@@ -511,17 +550,15 @@ __global__ __launch_bounds__(kLanes) void prepare_kernel(State S, Options o, con
     if (lane == 0) {
         S.need_jacobian[run] = 0;
         S.jacobians[run] += 1;
-        finite_s = all_finite ? 1 : 0;
         if (!all_finite) S.status[run] = MKO_LM_NUMERICAL_ERROR;
     }
-    __syncthreads();
-    if (!finite_s) return;
+    if (!all_finite) return;
     // the compact inputs are read-only in this kernel; the state copies serve later kernels
     const double* a = a_c + size_t(j) * n * n;
     const double* g = g_c + size_t(j) * n;
     prepare_step(S, o, run, a, g);
     __syncthreads();
-    solve_step(S, run, a, g, kModelDamping, L, m_tri);
+    solve_step(S, run, a, g, kModelDamping, L);
     if (lane == 0) {
         const bool solved = S.solved[run] != 0;
         const double merit = S.merit[run];
@@ -536,15 +573,12 @@ __global__ __launch_bounds__(kLanes) void prepare_kernel(State S, Options o, con
 
 __global__ __launch_bounds__(kLanes) void step_kernel(State S, Options o, const int32_t* list,
                                                       int count, const int32_t* dcount) {
-    __shared__ SolveScalars sc;
-    extern __shared__ double m_tri[]; // packed lower triangle, P (P + 1) / 2 doubles, then the
-                                      // row and column (uint8) of each entry, then the arrays
-    SolveLds L = solve_lds(m_tri, S.P, sc);
+    extern __shared__ double m_tri[];
+    const SolveLds L = solve_lds(m_tri, S.P);
     const int j = blockIdx.x;
     if (j >= count || (dcount && j >= *dcount)) return;
     const int run = list[j];
-    solve_step(S, run, S.a + size_t(run) * S.P * S.P, S.g + size_t(run) * S.P, S.mu[run], L,
-               m_tri);
+    solve_step(S, run, S.a + size_t(run) * S.P * S.P, S.g + size_t(run) * S.P, S.mu[run], L);
     if (threadIdx.x == 0) {
         const bool solved = S.solved[run] != 0;
         S.evaluate[run] = 0;
@@ -555,56 +589,66 @@ __global__ __launch_bounds__(kLanes) void step_kernel(State S, Options o, const 
     }
 }
 
-__global__ __launch_bounds__(256) void update_kernel(State S, Options o, const int32_t* list,
-                                                     int count, const int32_t* dcount,
-                                                     const int32_t* pos, const double* f,
-                                                     const int64_t* failed, const int64_t* hard) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kLanes) void update_kernel(State S, Options o, const int32_t* list,
+                                                        int count, const int32_t* dcount,
+                                                        const int32_t* pos, const double* f,
+                                                        const int64_t* failed,
+                                                        const int64_t* hard) {
+    const int j = blockIdx.x;
     if (j >= count || (dcount && j >= *dcount)) return;
     const int run = list[j];
-    if (S.status[run] == MKO_LM_CONVERGED_STEP) return;
-    S.iterations[run] += 1;
+    int status = S.status[run];
+    if (status == MKO_LM_CONVERGED_STEP) return;
     bool accept = false;
     const double merit = S.merit[run];
+    double now = merit, rho = 0.0;
+    int64_t failed_new = 0, hard_new = 0;
     if (S.solved[run]) {
         const int e = pos[run];
         const double f_new = f[e];
-        const int64_t failed_new = failed[e], hard_new = hard[e];
+        failed_new = failed[e];
+        hard_new = hard[e];
         const double predicted = S.predicted[run];
-        const double rho = __ddiv_rn(merit - f_new, predicted);
+        rho = __ddiv_rn(merit - f_new, predicted);
         accept = isfinite(f_new) && predicted > 0.0 && f_new < merit &&
                  !(o.reject_new_failures && hard_new > S.hard[run]);
-        if (accept) {
-            const int n = S.P;
-            for (int k = 0; k < n; ++k) S.x[size_t(run) * n + k] = S.trial[size_t(run) * n + k];
-            S.merit[run] = f_new;
-            S.failed[run] = failed_new;
-            S.hard[run] = hard_new;
-            const double t = 2.0 * rho - 1.0;
-            S.mu[run] = S.mu[run] * dmax(1.0 / 3.0, 1.0 - t * t * t);
-            S.nu[run] = 2.0;
-            S.need_jacobian[run] = 1;
-            S.rejected[run] = 0;
-            S.accepted[run] += 1;
-            if (f_new == 0.0) S.status[run] = MKO_LM_CONVERGED_MERIT;
-        }
+        if (accept) now = f_new;
     }
-    if (!accept) {
-        S.mu[run] = S.mu[run] * S.nu[run];
+    if (accept) {
+        const int n = S.P;
+        for (int k = threadIdx.x; k < n; k += kLanes)
+            S.x[size_t(run) * n + k] = S.trial[size_t(run) * n + k];
+    }
+    if (threadIdx.x != 0) return;
+    S.iterations[run] += 1;
+    if (accept) {
+        S.merit[run] = now;
+        S.failed[run] = failed_new;
+        S.hard[run] = hard_new;
+        const double t = 2.0 * rho - 1.0;
+        S.mu[run] = S.mu[run] * dmax(1.0 / 3.0, 1.0 - t * t * t);
+        S.nu[run] = 2.0;
+        S.need_jacobian[run] = 1;
+        S.rejected[run] = 0;
+        S.accepted[run] += 1;
+        if (now == 0.0) status = MKO_LM_CONVERGED_MERIT;
+    } else {
+        const double mu = S.mu[run] * S.nu[run];
+        S.mu[run] = mu;
         S.nu[run] = S.nu[run] * 2.0;
         S.rejected[run] = 1;
-        if (S.mu[run] > o.max_damping) S.status[run] = MKO_LM_DAMPING_LIMIT;
+        if (mu > o.max_damping) status = MKO_LM_DAMPING_LIMIT;
     }
-    const double now = S.merit[run];
     push_history(S, run, now);
-    if (o.stall_window > 0 && S.status[run] == MKO_LM_RUNNING) {
+    if (o.stall_window > 0 && status == MKO_LM_RUNNING) {
         const int w = o.stall_window;
         const int size = S.history_len[run];
         if (size > w) {
             const double old = S.history[size_t(run) * S.H + ((size - 1 - w) % S.H)];
-            if (old - now <= o.stall_tolerance * old) S.status[run] = MKO_LM_CONVERGED_STALL;
+            if (old - now <= o.stall_tolerance * old) status = MKO_LM_CONVERGED_STALL;
         }
     }
+    S.status[run] = status;
 }
 
 __global__ __launch_bounds__(64) void fd_pattern_kernel(int count, int P, const double* xs,
@@ -647,17 +691,15 @@ __global__ __launch_bounds__(64) void fd_pattern_kernel(int count, int P, const 
 }
 
 inline hipStream_t st(void* s) { return static_cast<hipStream_t>(s); }
-inline size_t tri_bytes(int P) {
-    // the triangle with its entries' row and column bytes, then the solve's arrays (6 doubles,
-    // an int and a byte per variable)
-    return solve_arrays_offset(P) + size_t(P) * (6 * sizeof(double) + sizeof(int) + 1);
+inline size_t solve_bytes(int P) {
+    return (solve_entries(P) + size_t(P)) * sizeof(double) + size_t(P) * sizeof(int);
 }
 inline unsigned blocks_of(int n, int per) { return unsigned((n + per - 1) / per); }
 
 } // namespace
 
 void launch_init(const State& s, const Options& o, void* stream) {
-    if (s.n > 0) hipLaunchKernelGGL(init_kernel, dim3(blocks_of(s.n, 256)), dim3(256), 0, st(stream), s, o);
+    if (s.n > 0) hipLaunchKernelGGL(init_kernel, dim3(unsigned(s.n)), dim3(kLanes), 0, st(stream), s, o);
 }
 
 void launch_start(const State& s, const double* merit, const int64_t* failed, const int64_t* hard,
@@ -696,14 +738,14 @@ void launch_gather(const State& s, const int32_t* list, int count, bool trial,
 void launch_prepare(const State& s, const Options& o, const int32_t* list, int count,
                     const double* a_c, const double* g_c, void* stream, const int32_t* dcount) {
     if (count > 0)
-        hipLaunchKernelGGL(prepare_kernel, dim3(unsigned(count)), dim3(kLanes), tri_bytes(s.P),
+        hipLaunchKernelGGL(prepare_kernel, dim3(unsigned(count)), dim3(kLanes), solve_bytes(s.P),
                            st(stream), s, o, list, count, dcount, a_c, g_c);
 }
 
 void launch_step(const State& s, const Options& o, const int32_t* list, int count, void* stream,
                  const int32_t* dcount) {
     if (count > 0)
-        hipLaunchKernelGGL(step_kernel, dim3(unsigned(count)), dim3(kLanes), tri_bytes(s.P),
+        hipLaunchKernelGGL(step_kernel, dim3(unsigned(count)), dim3(kLanes), solve_bytes(s.P),
                            st(stream), s, o, list, count, dcount);
 }
 
@@ -711,7 +753,7 @@ void launch_update(const State& s, const Options& o, const int32_t* list, int co
                    const int32_t* pos, const double* f, const int64_t* failed,
                    const int64_t* hard, void* stream, const int32_t* dcount) {
     if (count > 0)
-        hipLaunchKernelGGL(update_kernel, dim3(blocks_of(count, 256)), dim3(256), 0, st(stream), s,
+        hipLaunchKernelGGL(update_kernel, dim3(unsigned(count)), dim3(kLanes), 0, st(stream), s,
                            o, list, count, dcount, pos, f, failed, hard);
 }
 
