@@ -1183,21 +1183,34 @@ __global__ void rows_merit_kernel(int V, const double* rows, int64_t stride, int
     if (t_sum) t_sum[v] = t;
 }
 
-// merit[v] = sum over tuples in (f, l) order + extra[v] (merit_finalize_kernel, merit.cu:207)
-__global__ void merit_finalize_kernel(int V, int T, const double* partial, const int* pfailed,
-                                      const int* phard, const double* extra,
-                                      const double* traced, double* merit, int64_t* failed,
-                                      int64_t* hard, const int32_t* live) {
+// merit[v] = sum over tuples in (f, l) order + extra[v] (merit_finalize_kernel, merit.cu:207). A
+// wave per variant, 4 to a workgroup: the partials of 64 tuples in one load, added in tuple order
+// from the lanes' registers (a thread per variant waited for each tuple's three loads: 256 variants
+// of 35 tuples 21 -> 5 us).
+__global__ __launch_bounds__(256) void merit_finalize_kernel(
+    int V, int T, const double* partial, const int* pfailed, const int* phard, const double* extra,
+    const double* traced, double* merit, int64_t* failed, int64_t* hard, const int32_t* live) {
 #pragma clang fp contract(off)
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int v = int(blockIdx.x) * 4 + int(threadIdx.x >> 6);
     if (v >= V || (live && v >= *live)) return;
     double s = 0.0;
     int64_t f = 0, h = 0;
-    for (int t = 0; t < T; ++t) {
-        s += partial[size_t(v) * T + t];
-        f += pfailed[size_t(v) * T + t];
-        h += phard[size_t(v) * T + t];
+    for (int t0 = 0; t0 < T; t0 += 64) {
+        const int t = t0 + lane;
+        const size_t at = size_t(v) * T + t;
+        const double x = t < T ? partial[at] : 0.0;
+        f += t < T ? pfailed[at] : 0;
+        h += t < T ? phard[at] : 0;
+        const int n = min(64, T - t0);
+        const int lo = __double2loint(x), hi = __double2hiint(x);
+        for (int i = 0; i < n; ++i)
+            s += __hiloint2double(__builtin_amdgcn_readlane(hi, i),
+                                  __builtin_amdgcn_readlane(lo, i));
     }
+    f = wave_sum(f);
+    h = wave_sum(h);
+    if (lane != 0) return;
     // (ray merit + sum e^2) + sum t^2 (CpuLmBackend::merit, levenberg_marquardt.cpp:866-888)
     double m = extra ? s + extra[v] : s;
     if (traced) m = m + traced[v];
@@ -1551,8 +1564,8 @@ __global__ void point_batch_kernel(ConstBatchPtrs src, BatchPtrs dst, int runs, 
     // variables: x0 of the run, component k replaced for FD variants
     const int kk = j == 0 ? -1 : (j - 1) / 2;
     bool glass = false;
-    for (int k = 0; k < P; ++k) glass = glass || var_type[k] == MKO_VAR_GLASS;
     for (int k = threadIdx.x; k < P; k += blockDim.x) {
+        glass = glass || var_type[k] == MKO_VAR_GLASS;
         double x = x0[size_t(run) * P + k];
         if (k == kk) x = (j & 1) ? plus[size_t(run) * P + k] : minus[size_t(run) * P + k];
         const int s = var_surface[k];
@@ -1564,7 +1577,7 @@ __global__ void point_batch_kernel(ConstBatchPtrs src, BatchPtrs dst, int runs, 
         } else
             dst.thickness[size_t(vv) * S + s] = x;
     }
-    if (!glass) return;
+    if (!__any(glass)) return; // one wavefront
     __syncthreads();
     // index of the glass-variable surfaces from their Buchdahl coefficients
     // (VariableSet::apply, variable_set.cpp:271-284; buchdahl_index, dispersion.hpp:93);
@@ -2320,7 +2333,16 @@ __global__ void vjp_finalize_kernel(int V, int T, int Pn, const double* part, do
     if (i >= int64_t(V) * Pn) return;
     const int64_t v = i / Pn, p = i - v * Pn;
     double x = 0.0;
-    for (int t = 0; t < T; ++t) x += part[(v * T + t) * Pn + p];
+    const double* at = part + v * T * Pn + p;
+    int t = 0;
+    for (; t + 8 <= T; t += 8) { // 8 loads in flight
+        double y[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) y[q] = at[int64_t(t + q) * Pn];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x += y[q];
+    }
+    for (; t < T; ++t) x += at[int64_t(t) * Pn];
     out[i] = x;
 }
 
@@ -2838,22 +2860,23 @@ void adjoint_normal_kernel(TraceParams P, ParamMap map, float* partC, double* pa
 }
 
 // a = sum_t s_t^2 (C_t - S_t S_t^T / W_t), g = sum_t s_t^2 (Tr_t - (piston_t - o_t) S_t), tuples
-// in (field, wavelength) order; one workgroup per run. Each thread owns up to 19 entries of the
-// upper triangle (mirrored on output); the tuples' S, Tr and factors are staged through LDS in
-// chunks of 8 tuples.
-constexpr int kFinalizeChunk = 8;
-// kE entries per thread: 5 up to 49 variables, 10 up to 71, 19 up to 96 (the kernel is
-// instantiated per bound, so the accumulators of the smaller counts do not hold registers and
-// more workgroups fit a CU).
-constexpr int kFinalizeEntries = (kMaxVariablesFused * (kMaxVariablesFused + 1) / 2 + 255) / 256;
+// in (field, wavelength) order; `parts` workgroups per run, each with 256 kE entries of the upper
+// triangle (mirrored on output), kE per thread; the tuples' S, Tr and factors are staged through
+// LDS 16 tuples at a time and the C of 4 tuples are loaded together (the sum over the tuples is
+// one dependent chain per entry, their loads are not). What bounds it is latency up to some
+// hundred runs, then the reading of C (4 P^2 bytes per tuple): with few runs one entry per thread
+// and more workgroups, from 512 on five (fewer workgroups stage S again). Runs of 35 tuples and 48
+// variables, before (one workgroup per run, a tuple at a time) and now: 256 runs 98 -> 25 us, 512
+// runs 95 -> 34 us. The contraction is spelled out, so both instantiations give the same bits.
+constexpr int kFinalizeChunk = 16;
 
 template <int kE>
 __global__ __launch_bounds__(256) void adjoint_normal_finalize_kernel(
-    int T, int Pn, const float* partC, const double* partST, const TupleNormal* partT, double* a,
-    double* g, const int32_t* live) {
-    __shared__ double S_l[kFinalizeChunk][2 * kMaxVariablesFused];
+    int T, int Pn, int parts, const float* partC, const double* partST, const TupleNormal* partT,
+    double* a, double* g, const int32_t* live) {
+    extern __shared__ double S_l[]; // [kFinalizeChunk][2 P]
     __shared__ double f1[kFinalizeChunk], f2[kFinalizeChunk], pist[kFinalizeChunk];
-    const int v = blockIdx.x;
+    const int v = int(blockIdx.x) / parts, part = int(blockIdx.x) - v * parts;
     if (live && v >= *live) return;
     const int tid = threadIdx.x;
     const int nu = Pn * (Pn + 1) / 2;
@@ -2862,23 +2885,22 @@ __global__ __launch_bounds__(256) void adjoint_normal_finalize_kernel(
 #pragma unroll
     for (int i = 0; i < kE; ++i) {
         acc[i] = 0.0;
-        // upper-triangle index u -> (q, p), q <= p, row-major over q
-        const int u = tid + i * 256;
-        int q = 0, rem = u;
-        while (q < Pn && rem >= Pn - q) {
-            rem -= Pn - q;
-            ++q;
-        }
+        // upper-triangle index u -> (q, p), q <= p, row-major over q: row q starts at
+        // q (2 P + 1 - q) / 2; the root of that quadratic, corrected to the row
+        const int u = min((part * kE + i) * 256 + tid, nu - 1);
+        const float b = float(2 * Pn + 1);
+        int q = int(0.5f * (b - __builtin_sqrtf(fmaxf(b * b - 8.0f * float(u), 0.0f))));
+        while (q > 0 && q * (2 * Pn + 1 - q) / 2 > u) --q;
+        while ((q + 1) * (2 * Pn - q) / 2 <= u) ++q;
         eq[i] = q;
-        ep[i] = q + rem;
+        ep[i] = q + u - q * (2 * Pn + 1 - q) / 2;
     }
     double gacc = 0.0;
+    const float* C0 = partC + size_t(v) * T * size_t(Pn) * Pn;
     for (int t0 = 0; t0 < T; t0 += kFinalizeChunk) {
         const int nt = min(kFinalizeChunk, T - t0);
-        for (int e = tid; e < nt * 2 * Pn; e += 256) {
-            const int tt = e / (2 * Pn), i = e - tt * 2 * Pn;
-            S_l[tt][i] = partST[(size_t(v) * T + t0 + tt) * 2 * Pn + i];
-        }
+        for (int e = tid; e < nt * 2 * Pn; e += 256)
+            S_l[e] = partST[(size_t(v) * T + t0) * 2 * Pn + e];
         if (tid < nt) {
             const TupleNormal tn = partT[size_t(v) * T + t0 + tid];
             const bool valid = tn.w_ok > 0.0;
@@ -2887,29 +2909,39 @@ __global__ __launch_bounds__(256) void adjoint_normal_finalize_kernel(
             pist[tid] = valid ? tn.piston : 0.0;
         }
         __syncthreads();
-        for (int tt = 0; tt < nt; ++tt) {
-            const float* C = partC + (size_t(v) * T + t0 + tt) * size_t(Pn) * Pn;
+        for (int tt = 0; tt < nt; tt += 4) {
+            float c[4][kE];
 #pragma unroll
-            for (int i = 0; i < kE; ++i) {
-                if (tid + i * 256 < nu) {
-                    const int q = eq[i], p = ep[i];
-                    const double c = double(C[size_t(q) * Pn + p]);
-                    acc[i] += f1[tt] * c - f2[tt] * (S_l[tt][p] * S_l[tt][q]);
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int i = 0; i < kE; ++i) {
+                    const size_t tu = size_t(t0 + min(tt + x, nt - 1));
+                    c[x][i] = C0[(tu * Pn + eq[i]) * Pn + ep[i]];
                 }
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                if (tt + x >= nt) break; // uniform
+                const double* St = S_l + (tt + x) * 2 * Pn;
+#pragma unroll
+                for (int i = 0; i < kE; ++i)
+                    acc[i] += __builtin_fma(f1[tt + x], double(c[x][i]),
+                                            -(f2[tt + x] * (St[ep[i]] * St[eq[i]])));
+                if (part == 0 && tid < Pn)
+                    gacc = __builtin_fma(f1[tt + x],
+                                         __builtin_fma(-pist[tt + x], St[tid], St[Pn + tid]), gacc);
             }
-            if (tid < Pn) gacc += f1[tt] * (S_l[tt][Pn + tid] - pist[tt] * S_l[tt][tid]);
         }
         __syncthreads();
     }
     double* A = a + size_t(v) * Pn * Pn;
 #pragma unroll
     for (int i = 0; i < kE; ++i) {
-        if (tid + i * 256 < nu) {
+        if ((part * kE + i) * 256 + tid < nu) {
             A[size_t(eq[i]) * Pn + ep[i]] = acc[i];
             A[size_t(ep[i]) * Pn + eq[i]] = acc[i];
         }
     }
-    if (tid < Pn) g[size_t(v) * Pn + tid] = gacc;
+    if (part == 0 && tid < Pn) g[size_t(v) * Pn + tid] = gacc;
 }
 
 // ---- Gram: A = J^T J, g = J^T r0 per run ----------------------------------------------------
@@ -3581,11 +3613,14 @@ int adjoint_normal_states(const mko_batch* batch, const mko_residual_settings* s
         }
         check_hip(hipGetLastError(), "adjoint normal launch");
         const int nu = m.P * (m.P + 1) / 2;
-        const auto finalize = nu <= 5 * 256    ? adjoint_normal_finalize_kernel<5>
-                              : nu <= 10 * 256 ? adjoint_normal_finalize_kernel<10>
-                                               : adjoint_normal_finalize_kernel<kFinalizeEntries>;
-        hipLaunchKernelGGL(finalize, dim3(unsigned(P.V)), dim3(256), 0, s, P.T, m.P, partC,
-                           partST, partT, a, g, live);
+        const size_t lds = size_t(kFinalizeChunk) * 2 * m.P * sizeof(double);
+        const auto finalize = [&](auto kernel, int entries) {
+            const int parts = (nu + 256 * entries - 1) / (256 * entries);
+            hipLaunchKernelGGL(kernel, dim3(unsigned(P.V) * unsigned(parts)), dim3(256), lds, s,
+                               P.T, m.P, parts, partC, partST, partT, a, g, live);
+        };
+        if (P.V < 512) finalize(adjoint_normal_finalize_kernel<1>, 1);
+        else finalize(adjoint_normal_finalize_kernel<5>, 5);
         check_hip(hipGetLastError(), "adjoint normal finalize launch");
     })
 }
@@ -3604,7 +3639,7 @@ int merit_states(const mko_batch* batch, const mko_residual_settings* settings, 
         int* pf = partial_counts;
         int* ph = partial_counts + size_t(P.V) * P.T;
         launch_trace(1, P, nullptr, nullptr, nullptr, partial, pf, ph, nullptr, s, &states);
-        hipLaunchKernelGGL(merit_finalize_kernel, dim3((P.V + 255) / 256), dim3(256), 0, s, P.V,
+        hipLaunchKernelGGL(merit_finalize_kernel, dim3((P.V + 3) / 4), dim3(256), 0, s, P.V,
                            P.T, partial, pf, ph, nullptr, nullptr, merit, failed, hard_failed, live);
         check_hip(hipGetLastError(), "merit finalize launch");
     })
@@ -3724,7 +3759,7 @@ int merit_finalize(int V, int T, const double* partial, const int* partial_count
                    int64_t* hard_failed, void* stream) {
     MKO_TRY({
         if (V <= 0) return 0;
-        hipLaunchKernelGGL(merit_finalize_kernel, dim3((V + 255) / 256), dim3(256), 0,
+        hipLaunchKernelGGL(merit_finalize_kernel, dim3((V + 3) / 4), dim3(256), 0,
                            static_cast<hipStream_t>(stream), V, T, partial, partial_counts,
                            partial_counts + size_t(V) * T, extra, traced, merit, failed,
                            hard_failed, nullptr);
@@ -3838,7 +3873,7 @@ int mko_merit_device(const mko_batch* batch, const mko_residual_settings* settin
         int* pf = partial_counts;
         int* ph = partial_counts + size_t(P.V) * P.T;
         launch_trace(1, P, nullptr, nullptr, nullptr, partial, pf, ph, nullptr, s);
-        hipLaunchKernelGGL(merit_finalize_kernel, dim3((P.V + 255) / 256), dim3(256), 0, s, P.V,
+        hipLaunchKernelGGL(merit_finalize_kernel, dim3((P.V + 3) / 4), dim3(256), 0, s, P.V,
                            P.T, partial, pf, ph, extra_merit, nullptr, merit, failed, hard_failed,
                            nullptr);
         check_hip(hipGetLastError(), "merit finalize launch");
@@ -3867,7 +3902,7 @@ int mko_merit_device_noalloc(const mko_batch* batch, const mko_residual_settings
         // every tuple's partial and counts are written by its trace block before the finalize
         // reads them, so the previous call's contents need no clearing
         launch_trace(1, P, nullptr, nullptr, nullptr, partial, pf, ph, nullptr, s);
-        hipLaunchKernelGGL(merit_finalize_kernel, dim3((P.V + 255) / 256), dim3(256), 0, s, P.V,
+        hipLaunchKernelGGL(merit_finalize_kernel, dim3((P.V + 3) / 4), dim3(256), 0, s, P.V,
                            P.T, partial, pf, ph, extra_merit, nullptr, merit, failed, hard_failed,
                            nullptr);
         check_hip(hipGetLastError(), "merit finalize launch");
