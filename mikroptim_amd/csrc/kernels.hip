@@ -1227,13 +1227,30 @@ __global__ __launch_bounds__(256) void merit_finalize_kernel(
 // transfer, cos I = sqrt(D) at the sphere, cos I' = sqrt(k) after refraction, the reference
 // sphere's discriminant and denominator); for a failed ray the size of the violated check.
 
-struct PfLds {
-    float c[MKO_MAX_SURFACES], t[MKO_MAX_SURFACES], n[MKO_MAX_SURFACES];
+// Surface table of a (variant, wavelength) in LDS: row s >= 1 the step to surface s, row 0 the
+// image side.
+struct PfStep {
+    float c, t, n, mu; // effective curvature, thickness and index before the surface, n / n'
 };
 
+// Quotient and root in 4 and 6 instructions (the correctly rounded ones of the compiler take
+// about 10 and 15 and were half of the trace): the hardware's estimate and one step on the residual,
+// within 1 ulp. The root of a number below the smallest normal one is that one's.
+__device__ __forceinline__ float pf_div(float a, float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+__device__ __forceinline__ float pf_sqrt(float x) {
+    const float v = x < 1.17549435e-38f ? 1.17549435e-38f : x; // NaN stays
+    const float y = __builtin_amdgcn_rsqf(v);
+    const float r = v * y;
+    return __builtin_fmaf(__builtin_fmaf(-r, r, v), 0.5f * y, r);
+}
+
+// NaN in either sticks: no margin compares above eta then (uncertain).
 __device__ __forceinline__ float pf_min_margin(float acc, float x) {
-    if (x < acc) return x;
-    return x >= acc ? acc : 0.0f; // NaN: 0 (uncertain)
+    return __builtin_elementwise_minimum(acc, x);
 }
 __device__ __forceinline__ float pf_fail_linear(float x) { return -x > 0.0f ? -x : 0.0f; }
 __device__ __forceinline__ float pf_fail_root(float q) {
@@ -1245,50 +1262,49 @@ struct PfRay {
     float opl, margin;
 };
 
-__device__ __forceinline__ PfRay pf_trace(const PfLds& L, int S, V3<float> p, V3<float> d,
-                                          float opl, V3<float> M, int kind, float kappa) {
+__device__ __forceinline__ PfRay pf_trace(const PfStep* L, int S, V3<float> p, V3<float> d,
+                                          float opl, V3<float> M, float n_image, int kind,
+                                          float kappa) {
     using mkod::cross;
     using mkod::dot;
     PfRay out{MKO_STATUS_OK, 0.0f, 0.0f};
     float margin = 1.0f;
     for (int s = 1; s < S; ++s) {
-        const float c = L.c[s], nb = L.n[s - 1], na = L.n[s];
+        const PfStep e = L[s];
         if (!(d.z > 0.0f)) {
             out.status = MKO_STATUS_BACKWARD;
             out.margin = pf_fail_linear(d.z);
             return out;
         }
-        const V3<float> db = d;
-        p.z -= L.t[s - 1];
-        const float s0 = -p.z / d.z;
+        const float dz = d.z;
+        p.z -= e.t;
+        const float s0 = pf_div(-p.z, dz);
         p.x += s0 * d.x;
         p.y += s0 * d.y;
         p.z = 0.0f;
-        const float H = c * (p.x * p.x + p.y * p.y);
-        const float B = d.z - c * (p.x * d.x + p.y * d.y);
-        const float D = B * B - c * H;
-        const float denom = D < 0.0f ? 0.0f : B + __builtin_sqrtf(D);
+        const float H = e.c * (p.x * p.x + p.y * p.y);
+        const float B = dz - e.c * (p.x * d.x + p.y * d.y);
+        const float D = B * B - e.c * H;
+        const float denom = D < 0.0f ? 0.0f : B + pf_sqrt(D);
         if (D < 0.0f || !(denom > 0.0f)) {
             const float a = pf_fail_root(D), b = pf_fail_linear(B);
             out.status = MKO_STATUS_MISSED;
             out.margin = a > b ? a : b;
             return out;
         }
-        const float sh = H / denom;
+        const float sh = pf_div(H, denom);
         p = p + sh * d;
-        opl += nb * (s0 + sh);
-        const float mu = nb / na;
-        const V3<float> N{-c * p.x, -c * p.y, 1.0f - c * p.z};
+        opl += e.n * (s0 + sh);
+        const V3<float> N{-e.c * p.x, -e.c * p.y, 1.0f - e.c * p.z};
         const float cosI = dot(d, N);
-        const float k = 1.0f - mu * mu * (1.0f - cosI * cosI);
+        const float k = 1.0f - e.mu * e.mu * (1.0f - cosI * cosI);
         if (k < 0.0f) {
             out.status = MKO_STATUS_TIR;
             out.margin = pf_fail_root(k);
             return out;
         }
-        d = mu * d + (__builtin_sqrtf(k) - mu * cosI) * N;
-        margin = pf_min_margin(margin, db.z);
-        margin = pf_min_margin(margin, dot(db, N));
+        d = e.mu * d + (pf_sqrt(k) - e.mu * cosI) * N;
+        margin = pf_min_margin(pf_min_margin(margin, dz), cosI);
         margin = pf_min_margin(margin, dot(d, N));
     }
     if (!(d.z > 0.0f)) {
@@ -1297,7 +1313,6 @@ __device__ __forceinline__ PfRay pf_trace(const PfLds& L, int S, V3<float> p, V3
         return out;
     }
     margin = pf_min_margin(margin, d.z);
-    const float n_image = L.n[S - 1];
     if (kind != MKO_REF_LAST_SURFACE) {
         const V3<float> q = p - M;
         const V3<float> ci = cross(q, d);
@@ -1364,59 +1379,116 @@ __device__ __forceinline__ float block_max_f(float v, float* lds) {
     return m;
 }
 
-// One workgroup per (variant, field, wavelength) tuple: the tuple's float surface table in LDS,
-// OPL relative to the axial optical length (prefilter_opl_offset), classes 0 certain valid /
-// 1 certain failed / 2, 3 uncertain (margin <= eta), the piston over the certain-valid rays and
-// the tuple's sum of squared residuals; partials per tuple: merit (as double), largest optical
-// length, counts [3] (certain failed, uncertain valid, uncertain failed).
-template <int kRpl>
-__global__ __launch_bounds__(kBlock) void prefilter_kernel(TraceParams P, float eta,
+// LDS slots of a tuple's n rays: a multiple of the q lanes by an odd number, so that the tuples
+// side by side fall on different banks.
+__host__ __device__ __forceinline__ int prefilter_slots(int n, int q) { return q * (((n + q - 1) / q) | 1); }
+
+// OPL relative to the axial optical length (prefilter_opl_offset), classes 0 certain valid / 1
+// certain failed / 2, 3 uncertain (margin <= eta), the piston over the certain-valid rays and the
+// tuple's sum of squared residuals; partials per tuple: merit (as double), largest optical length,
+// counts [3] (certain failed, uncertain valid, uncertain failed).
+// A multistart's tuples are small (6 to some hundred rays of a few surfaces), so what bounds it is
+// the instruction issue, of which a workgroup per tuple spent two thirds on idle waves, on the
+// tuple's weights and on every ray's sine and cosine. A workgroup takes one (field, wavelength) of
+// 256 / Q variants, Q lanes per variant: the spokes' and rings' samples and the weight are formed
+// once for all and the surface tables sit side by side (an odd stride spreads them over the banks).
+// The rays' path lengths and classes wait in LDS for the sums, which q <= Q lanes of the variant
+// form, without a barrier where Q = q (kWide: q = 256, sums over the workgroup). q depends on the
+// tuple's size alone, so the sums' order, hence their bits, are the same in every batch; Q is
+// larger where the batch is too small for the chip (prefilter_stats). 20000 variants of 9 tuples
+// of up to 72 rays and 3 surfaces: 637 -> 113 us.
+template <bool kWide>
+__global__ __launch_bounds__(kBlock) void prefilter_kernel(TraceParams P, int Q, int q, float eta,
                                                            double* pmerit, float* plength,
                                                            int* pcounts) {
-    __shared__ PfLds L;
+    extern __shared__ __align__(16) unsigned char pf_lds[];
+    __shared__ float rho_l[MKO_MAX_RINGS], w_l[MKO_MAX_RINGS], scale_l;
     __shared__ float fred[kWaves];
     __shared__ int ired[kWaves];
-    const Tuple t = tuple_of(P, blockIdx.x);
+    const int G = kBlock / Q, pitch = P.S | 1;
+    const int group = int(blockIdx.x) / P.T, tt = int(blockIdx.x) - group * P.T;
+    const int v0 = group * G, f = tt / P.L, l = tt - f * P.L;
     const int tid = threadIdx.x;
-    if (tid < P.S) {
-        const size_t vs = size_t(t.v) * P.S + tid;
-        L.c[tid] = ((P.sphere_mask >> tid) & 1ull) ? float(P.curvature[vs]) : 0.0f;
-        L.t[tid] = float(P.thickness[vs]);
-        L.n[tid] = float(P.index[vs * P.L + t.l]);
+    const uint8_t mode = P.pupil_mode[f];
+    const int M = mode == MKO_PUPIL_AXIS ? 1 : P.spokes, n = P.rings * M;
+    PfStep* steps = reinterpret_cast<PfStep*>(pf_lds);        // [G][pitch]
+    float2* spoke = reinterpret_cast<float2*>(steps + G * pitch); // [M]
+    float* opl_l = reinterpret_cast<float*>(spoke + M);           // [G][rays]
+    const int rays = prefilter_slots(n, q);
+    uint8_t* cls_l = reinterpret_cast<uint8_t*>(opl_l + G * rays); // [G][rays]
+    for (int e = tid; e < G * P.S; e += kBlock) {
+        const int g = e / P.S, s = e - g * P.S;
+        if (v0 + g >= P.V) break;
+        const size_t vs = size_t(v0 + g) * P.S + s;
+        PfStep k{};
+        const float na = float(P.index[vs * P.L + l]);
+        if (s > 0) {
+            k.c = ((P.sphere_mask >> s) & 1ull) ? float(P.curvature[vs]) : 0.0f;
+            k.t = float(P.thickness[vs - 1]);
+            k.n = float(P.index[(vs - 1) * P.L + l]);
+            k.mu = k.n / na;
+        } else {
+            const size_t last = vs + P.S - 1;
+            k.t = float(P.thickness[last]);
+            k.n = float(P.index[last * P.L + l]);
+        }
+        steps[g * pitch + s] = k;
+    }
+    const float pi = float(kPi);
+    for (int j = tid; j < M; j += kBlock) {
+        const float phi = mode == MKO_PUPIL_HALF   ? float(2 * j + 1) * pi / float(2 * M)
+                          : mode == MKO_PUPIL_FULL ? float(2 * j + 1) * pi / float(M)
+                                                   : 0.0f;
+        spoke[j] = make_float2(sinf(phi), cosf(phi));
+    }
+    if (tid < P.rings) {
+        rho_l[tid] = __builtin_sqrtf(float(P.gl_u[tid]));
+        w_l[tid] = float(P.gl_w[tid]) / float(M);
+    }
+    if (tid >= kBlock - 64) { // one wave
+        const Tuple t = tuple_of(P, tt);
+        if (tid == kBlock - 1) scale_l = float(t.scale);
     }
     __syncthreads();
+    const int mine = tid / Q, lane = tid & (Q - 1);
+    const bool in = v0 + mine < P.V;
+    const int v = in ? v0 + mine : P.V - 1;
+    const PfStep* L = steps + (v - v0) * pitch;
+    opl_l += mine * rays;
+    cls_l += mine * rays;
     float offset = 0.0f;
-    for (int s = 0; s + 1 < P.S; ++s) offset += L.n[s] * L.t[s];
-    const size_t vf = size_t(t.v) * P.F + t.f;
-    const float a = float(P.pupil_radius[t.v]);
+    for (int s = 1; s < P.S; ++s) offset += L[s].n * L[s].t;
+    const size_t vf = size_t(v) * P.F + f;
+    const float a = float(P.pupil_radius[v]);
     const float th = float(P.field_angle[vf]);
     const float sth = sinf(th), cth = cosf(th);
-    const V3<float> M{0.0f, float(P.field_target[vf]), L.t[P.S - 1]};
+    const V3<float> center{0.0f, float(P.field_target[vf]), L[0].t};
+    const float n_image = L[0].n;
     const float kappa = P.ref_kind != MKO_REF_LAST_SURFACE ? float(P.reference_curvature[vf]) : 0.0f;
-    const float pi = float(kPi);
-    float opl[kRpl], wts[kRpl];
-    uint8_t cls[kRpl];
-    float wok = 0.0f, wopl = 0.0f, optical = 0.0f;
-    int nf = 0, nuo = 0, nuf = 0;
-#pragma unroll
-    for (int i = 0; i < kRpl; ++i) {
-        const int k = tid + i * kBlock;
-        cls[i] = 4;
-        opl[i] = 0.0f;
-        wts[i] = 0.0f;
-        if (k >= t.n) continue;
-        const int ri = k / t.M, j = k - ri * t.M;
-        const float rho = __builtin_sqrtf(float(P.gl_u[ri]));
-        const float w = float(P.gl_w[ri]) / float(t.M);
-        const uint8_t mode = P.pupil_mode[t.f];
-        const float phi = mode == MKO_PUPIL_HALF   ? float(2 * j + 1) * pi / float(2 * t.M)
-                          : mode == MKO_PUPIL_FULL ? float(2 * j + 1) * pi / float(t.M)
-                                                   : 0.0f;
-        const float sp = sinf(phi), cp = cosf(phi);
+    // ray k = ri M + j of the lane: lane, lane + stride, ...
+    int ri, j, step_r, step_j;
+    const auto first_ray = [&](int stride) {
+        step_r = stride / M;
+        step_j = stride - step_r * M;
+        ri = lane / M;
+        j = lane - ri * M;
+    };
+    const auto next_ray = [&] {
+        ri += step_r;
+        j += step_j;
+        if (j >= M) {
+            j -= M;
+            ++ri;
+        }
+    };
+    first_ray(Q);
+    for (int k = lane; in && k < n; k += Q, next_ray()) {
+        const float rho = rho_l[ri];
+        const float sp = spoke[j].x, cp = spoke[j].y;
         V3<float> p, d;
         float o;
         if (P.source == MKO_SOURCE_POINT) {
-            const float sin_max = float(P.src_na) / L.n[0];
+            const float sin_max = float(P.src_na) / L[1].n;
             const float sr = sin_max * rho;
             p = V3<float>{float(P.src_pt[0]), float(P.src_pt[1]), float(P.src_pt[2])};
             d = V3<float>{sr * sp, sr * cp, __builtin_sqrtf((1.0f - sr) * (1.0f + sr))};
@@ -1427,46 +1499,64 @@ __global__ __launch_bounds__(kBlock) void prefilter_kernel(TraceParams P, float 
             d = V3<float>{0.0f, sth, cth};
             o = mkod::dot(p, d);
         }
-        const PfRay rr = pf_trace(L, P.S, p, d, o - offset, M, P.ref_kind, kappa);
+        const PfRay rr = pf_trace(L, P.S, p, d, o - offset, center, n_image, P.ref_kind, kappa);
         const bool ok = rr.status == MKO_STATUS_OK;
         const bool certain = rr.margin > eta;
-        const uint8_t c = uint8_t(ok ? (certain ? 0 : 2) : (certain ? 1 : 3));
-        cls[i] = c;
-        opl[i] = rr.opl;
-        wts[i] = w;
+        opl_l[k] = rr.opl;
+        cls_l[k] = uint8_t(ok ? (certain ? 0 : 2) : (certain ? 1 : 3));
+    }
+    if (Q != q) __syncthreads();
+    const bool sums = in && lane < q;
+    float wok = 0.0f, wopl = 0.0f, optical = 0.0f;
+    int fail_unsure = 0, nuf = 0; // certain failed + 2^16 uncertain valid, uncertain failed
+    first_ray(q);
+    for (int k = lane; sums && k < n; k += q, next_ray()) {
+        const float opl = opl_l[k];
+        const int c = cls_l[k];
         if (c == 0) {
+            const float w = w_l[ri];
             wok += w;
-            wopl += w * rr.opl;
-            const float len = fabsf(offset) + fabsf(rr.opl);
+            wopl += w * opl;
+            const float len = fabsf(offset) + fabsf(opl);
             optical = len > optical ? len : optical;
         }
-        nf += c == 1;
-        nuo += c == 2;
+        fail_unsure += c == 1 ? 1 : c == 2 ? 1 << 16 : 0;
         nuf += c == 3;
     }
-    const float w_ok = block_sum(wok, fred);
-    const float sum_o = block_sum(wopl, fred);
+    const auto sum = [&](auto x, auto* lds) {
+        if constexpr (kWide) return block_sum(x, lds);
+        for (int off = q >> 1; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
+        return x;
+    };
+    const float w_ok = sum(wok, fred);
+    const float sum_o = sum(wopl, fred);
     const bool valid = w_ok > 0.0f;
     const float piston = valid ? sum_o / w_ok : 0.0f;
-    const float scale = float(t.scale);
+    const float scale = scale_l;
     float r2 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kRpl; ++i) {
-        const float e = (valid && cls[i] == 0) ? opl[i] - piston : 0.0f;
-        const float r = scale * __builtin_sqrtf(wts[i]) * e;
+    first_ray(q);
+    for (int k = lane; sums && valid && k < n; k += q, next_ray()) {
+        const float e = cls_l[k] == 0 ? opl_l[k] - piston : 0.0f;
+        const float r = scale * __builtin_sqrtf(w_l[ri]) * e;
         r2 += r * r;
     }
-    const float tr2 = block_sum(r2, fred);
-    const float tl = block_max_f(optical, fred);
-    const int tf = block_sum(nf, ired);
-    const int tuo = block_sum(nuo, ired);
-    const int tuf = block_sum(nuf, ired);
-    if (tid == 0) {
-        pmerit[blockIdx.x] = double(tr2);
-        plength[blockIdx.x] = tl;
-        pcounts[size_t(blockIdx.x) * 3] = tf;
-        pcounts[size_t(blockIdx.x) * 3 + 1] = tuo;
-        pcounts[size_t(blockIdx.x) * 3 + 2] = tuf;
+    const float tr2 = sum(r2, fred);
+    float tl = optical;
+    if constexpr (kWide) tl = block_max_f(optical, fred);
+    else
+        for (int off = q >> 1; off >= 1; off >>= 1) {
+            const float o = __shfl_xor(tl, off, 64);
+            tl = o > tl ? o : tl;
+        }
+    const int tfu = sum(fail_unsure, ired);
+    const int tuf = sum(nuf, ired);
+    if (lane == 0 && in) {
+        const size_t at = size_t(v) * P.T + tt;
+        pmerit[at] = double(tr2);
+        plength[at] = tl;
+        pcounts[at * 3] = tfu & 0xffff;
+        pcounts[at * 3 + 1] = tfu >> 16;
+        pcounts[at * 3 + 2] = tuf;
     }
 }
 
@@ -3267,6 +3357,16 @@ int largest_tuple(const TraceParams& P) {
     return nmax;
 }
 
+// Lanes per tuple of the prefilter, by its largest tuple: the most of 8 ... 64 that idle on at most
+// 1/8 of the rays' slots (72 rays: 16 lanes of 5 rays; 8 lanes if none does), a whole workgroup
+// above 256 rays.
+int prefilter_lanes(int n) {
+    if (n > 256) return kBlock;
+    for (int q = 64; q > 8; q /= 2)
+        if (8 * n >= 7 * q * ((n + q - 1) / q)) return q;
+    return 8;
+}
+
 int rays_per_lane(const TraceParams& P) {
     const int r = (largest_tuple(P) + kBlock - 1) / kBlock;
     return r <= 1 ? 1 : r <= 2 ? 2 : r <= 4 ? 4 : 8;
@@ -3735,14 +3835,22 @@ int prefilter_stats(const mko_batch* batch, const mko_residual_settings* setting
         float* pl = reinterpret_cast<float*>(w + tuples * 8);
         int* pc = reinterpret_cast<int*>(w + tuples * 12);
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        const dim3 grid{unsigned(tuples)}, block{unsigned(kBlock)};
         const float eta = float(boundary);
-        switch (rays_per_lane(P)) {
-        case 1: hipLaunchKernelGGL((prefilter_kernel<1>), grid, block, 0, s, P, eta, pm, pl, pc); break;
-        case 2: hipLaunchKernelGGL((prefilter_kernel<2>), grid, block, 0, s, P, eta, pm, pl, pc); break;
-        case 4: hipLaunchKernelGGL((prefilter_kernel<4>), grid, block, 0, s, P, eta, pm, pl, pc); break;
-        default: hipLaunchKernelGGL((prefilter_kernel<8>), grid, block, 0, s, P, eta, pm, pl, pc); break;
-        }
+        // lanes per tuple: those of the sums, doubled (up to one ray per lane) while the launch has
+        // less than 4 workgroups per CU. One variant of 35 tuples of 72 rays and 25 surfaces, the
+        // whole call: 211 us with 16 lanes, 176 with 128; 2000 variants of 9 tuples of 72 rays and
+        // more keep the lanes of the sums (512 variants of 35 tuples: 550 -> 418 us)
+        const int n = largest_tuple(P), q = prefilter_lanes(n);
+        int Q = q;
+        const auto groups = [&] { return (P.V + kBlock / Q - 1) / (kBlock / Q); };
+        while (Q < kBlock && Q < n && int64_t(groups()) * P.T < 1024) Q *= 2;
+        const int G = kBlock / Q;
+        const size_t lds = size_t(G) * (P.S | 1) * sizeof(PfStep) +
+                           size_t(std::max(1, P.spokes)) * sizeof(float2) +
+                           size_t(G) * prefilter_slots(n, q) * (sizeof(float) + 1);
+        const auto kernel = q == kBlock ? prefilter_kernel<true> : prefilter_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(groups()) * unsigned(P.T)), dim3(kBlock), lds, s,
+                           P, Q, q, eta, pm, pl, pc);
         check_hip(hipGetLastError(), "prefilter launch");
         hipLaunchKernelGGL(prefilter_finalize_kernel, dim3((P.V + 255) / 256), dim3(256), 0, s,
                            P.V, P.T, pm, pl, pc, merit, optical, failed, uncertain_ok,
