@@ -22,6 +22,7 @@
 #include <cstdint>
 #include <cstring>
 #include <functional>
+#include <initializer_list>
 #include <limits>
 #include <map>
 #include <memory>
@@ -88,6 +89,179 @@ struct DeviceGuard {
         hip_check(hipSetDevice(dev), "hipSetDevice");
     }
     ~DeviceGuard() { (void)hipSetDevice(old); }
+};
+
+// Transfers between host arrays and device memory through pinned slots, ordered on the null stream.
+// A copy of pageable memory stops the host at each array (11.5 us for the smallest) and runs at
+// 12 ... 40 GB/s; a pinned one takes 2.5 us to issue and runs at 53 GB/s, and the host's copies in
+// and out of the slots overlap it (11.5 MB to the host: 710 us pageable, 430 us this way, 210 us of
+// it the copy). kSlots slots of 1 MiB (a copy costs some 20 us of its own: 256 KB slots take twice
+// as long), each allocated at its first use, belong to one engine: its calls are not concurrent. A
+// slot in flight is waited for before it is filled again.
+class Staging {
+public:
+    struct Piece {
+        void* host;
+        const void* dev;
+        size_t bytes;
+        bool joined = false; // follows the piece before it in the same allocation
+    };
+    Staging() = default;
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    ~Staging() {
+        for (Slot& s : slots_) {
+            if (s.done) {
+                (void)hipEventSynchronize(s.done);
+                (void)hipEventDestroy(s.done);
+            }
+            if (s.ptr) (void)hipHostFree(s.ptr);
+        }
+    }
+    // Host to device; the source may change once this returns.
+    void in(void* dev, const void* host, size_t bytes) {
+        stage(dev, host, bytes);
+        push();
+    }
+    // The same for several arrays of one allocation: adjacent ones go in one copy, the last of which
+    // push() issues. An array of 2 MiB or more goes without a slot, as long as the source stays
+    // until the null stream has passed the copy: 4 MiB take 135 us that way, through slots 82 us and
+    // 64 of the host's copies.
+    void stage(void* dev, const void* host, size_t bytes) {
+        char* d = static_cast<char*>(dev);
+        const char* h = static_cast<const char*>(host);
+        if (bytes >= 2 * kSlot) {
+            push();
+            hip_check(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, nullptr), "upload");
+            return;
+        }
+        while (bytes > 0) {
+            try {
+                if (run_bytes_ > 0 && d != run_dev_ + run_bytes_) push();
+                if (room() == 0) advance();
+            } catch (...) {
+                run_bytes_ = 0; // a later call must not issue it
+                throw;
+            }
+            const size_t n = std::min(bytes, room());
+            char* slot = slots_[cur_].ptr + used_;
+            if (run_bytes_ == 0) {
+                run_dev_ = d;
+                run_host_ = slot;
+            }
+            std::memcpy(slot, h, n);
+            used_ += n;
+            run_bytes_ += n;
+            d += n;
+            h += n;
+            bytes -= n;
+        }
+    }
+    void push() {
+        const size_t n = run_bytes_;
+        run_bytes_ = 0;
+        used_ = std::min(kSlot, (used_ + 255) & ~size_t(255));
+        if (n > 0)
+            hip_check(hipMemcpyAsync(run_dev_, run_host_, n, hipMemcpyHostToDevice, nullptr),
+                      "upload");
+    }
+    // Device to host; the pieces' host arrays hold the data when this returns. Joined pieces go in
+    // one copy. On an error nothing is left in flight.
+    void out(std::initializer_list<Piece> pieces) {
+        size_t total = 0;
+        for (const Piece& p : pieces) total += p.bytes;
+        if (total == 0) return;
+        try {
+            const char* run = nullptr; // copy to the current slot that is not issued yet
+            size_t run_bytes = 0;
+            const auto issue = [&] {
+                const size_t n = run_bytes;
+                run_bytes = 0;
+                if (n == 0) return;
+                hip_check(hipMemcpyAsync(slots_[cur_].ptr + used_, run, n, hipMemcpyDeviceToHost,
+                                         nullptr),
+                          "download");
+                used_ = std::min(kSlot, (used_ + n + 255) & ~size_t(255));
+            };
+            for (const Piece& p : pieces) {
+                char* h = static_cast<char*>(p.host);
+                const char* d = static_cast<const char*>(p.dev);
+                if (!p.joined) issue();
+                for (size_t left = p.bytes; left > 0;) {
+                    if (room() == run_bytes) { // the slot is full
+                        issue();
+                        advance();
+                    }
+                    const size_t n = std::min(left, room() - run_bytes);
+                    if (run_bytes == 0) run = d;
+                    slots_[cur_].back.push_back({h, slots_[cur_].ptr + used_ + run_bytes, n});
+                    run_bytes += n;
+                    h += n;
+                    d += n;
+                    left -= n;
+                }
+            }
+            issue();
+            hip_check(hipEventRecord(slots_[cur_].done, nullptr), "download");
+            slots_[cur_].busy = true;
+            for (int i = 1; i <= kSlots; ++i) settle(slots_[(cur_ + i) % kSlots]);
+        } catch (...) {
+            (void)hipDeviceSynchronize();
+            for (Slot& s : slots_) {
+                s.back.clear();
+                s.busy = false;
+            }
+            used_ = 0;
+            throw;
+        }
+        used_ = 0; // the null stream has passed everything before the last event
+    }
+
+private:
+    static constexpr size_t kSlot = size_t(1) << 20;
+    static constexpr int kSlots = 8;
+    struct Back {
+        void* host;
+        const char* slot;
+        size_t bytes;
+    };
+    struct Slot {
+        char* ptr = nullptr;
+        hipEvent_t done = nullptr;
+        bool busy = false;      // `done` is recorded behind the slot's last copy
+        std::vector<Back> back; // to be copied to the host arrays after `done`
+    };
+    Slot slots_[kSlots];
+    int cur_ = 0;
+    size_t used_ = 0;
+    char* run_dev_ = nullptr; // copy to the device being staged, at the end of the current slot
+    const char* run_host_ = nullptr;
+    size_t run_bytes_ = 0;
+
+    size_t room() {
+        Slot& s = slots_[cur_];
+        if (!s.ptr) {
+            if (!s.done)
+                hip_check(hipEventCreateWithFlags(&s.done, hipEventDisableTiming), "staging");
+            hip_check(hipHostMalloc(reinterpret_cast<void**>(&s.ptr), kSlot, hipHostMallocDefault),
+                      "staging");
+        }
+        return kSlot - used_;
+    }
+    void settle(Slot& s) {
+        if (s.busy) hip_check(hipEventSynchronize(s.done), "staging");
+        s.busy = false;
+        for (const Back& b : s.back) std::memcpy(b.host, b.slot, b.bytes);
+        s.back.clear();
+    }
+    void advance() {
+        push();
+        hip_check(hipEventRecord(slots_[cur_].done, nullptr), "staging");
+        slots_[cur_].busy = true;
+        cur_ = (cur_ + 1) % kSlots;
+        used_ = 0;
+        settle(slots_[cur_]);
+    }
 };
 
 inline int64_t rays_of(const mko_batch& b, const mko_residual_settings& s) {
@@ -356,7 +530,7 @@ void validate_paraxial(const mko_batch& b, int first, int count) {
 struct DeviceBatch {
     Buffer mem;
     mko_batch view{};
-    void upload(const mko_batch& h, int first, int count, hipStream_t stream) {
+    void upload(const mko_batch& h, int first, int count, Staging& io) {
         const Strides st(h);
         const size_t V = size_t(count);
         double* base = mem.as<double>(std::max<size_t>(1, V * st.doubles()));
@@ -368,9 +542,7 @@ struct DeviceBatch {
                 *dst = nullptr;
                 return;
             }
-            hip_check(hipMemcpyAsync(p, src + size_t(first) * per, V * per * sizeof(double),
-                                     hipMemcpyHostToDevice, stream),
-                      "upload batch");
+            io.stage(p, src + size_t(first) * per, V * per * sizeof(double));
             *dst = p;
             p += V * per;
         };
@@ -383,6 +555,7 @@ struct DeviceBatch {
         put(st.refc ? h.reference_curvature : nullptr, st.F, &view.reference_curvature);
         put(h.paraxial_index, st.S, &view.paraxial_index);
         put(h.buchdahl, 4 * st.S, &view.buchdahl);
+        io.push();
     }
     // Uninitialised device batch of `count` variants shaped like h (filled by a kernel).
     void allocate(const mko_batch& h, int count) {
@@ -702,7 +875,7 @@ public:
         const int tranche = tranche_size(b.variants, per);
         for (int first = 0; first < b.variants; first += tranche) {
             const int count = std::min(tranche, b.variants - first);
-            batch_.upload(b, first, count, nullptr);
+            batch_.upload(b, first, count, io_);
             double* dres = out_res_.as<double>(size_t(count) * R);
             double* dopd = opd ? out_opd_.as<double>(size_t(count) * rays) : nullptr;
             uint8_t* dst = status ? out_st_.as<uint8_t>(size_t(count) * rays) : nullptr;
@@ -717,9 +890,10 @@ public:
                 dev_check(mko_internal::constraint_rows(&batch_.view, rp.dev, rp.count(),
                                                         rp.paraxial, ex, dres, R, T, nullptr,
                                                         rp.hull));
-            if (res) copy_out(res + size_t(first) * R, dres, size_t(count) * R * 8);
-            if (opd) copy_out(opd + size_t(first) * rays, dopd, size_t(count) * rays * 8);
-            if (status) copy_out(status + size_t(first) * rays, dst, size_t(count) * rays);
+            const size_t n = size_t(count) * rays, at = size_t(first) * rays;
+            io_.out({{res ? res + size_t(first) * R : nullptr, dres, res ? size_t(count) * R * 8 : 0},
+                     {opd ? opd + at : nullptr, dopd, opd ? n * 8 : 0},
+                     {status ? status + at : nullptr, dst, status ? n : 0}});
         }
         hip_check(hipDeviceSynchronize(), "residuals");
     }
@@ -739,20 +913,21 @@ public:
         const int tranche = tranche_size(b.variants, per);
         for (int first = 0; first < b.variants; first += tranche) {
             const int count = std::min(tranche, b.variants - first);
-            batch_.upload(b, first, count, nullptr);
+            batch_.upload(b, first, count, io_);
             void* ws = part_.reserve(size_t(count) * T * 24);
-            double* dm = out_merit_.as<double>(size_t(count) * 2);
-            int64_t* dc = out_failed_.as<int64_t>(size_t(count) * 3);
+            double* dm = out_merit_.as<double>(size_t(count) * 5); // one copy to the host
+            int64_t* dc = reinterpret_cast<int64_t*>(dm + 2 * size_t(count));
             timer.run(kTrace, [&] {
                 dev_check(mko_internal::prefilter_stats(&batch_.view, &s, o.boundary, ws, dm,
                                                         dm + count, dc, dc + count,
                                                         dc + 2 * size_t(count), nullptr));
             });
-            copy_out(r.merit + first, dm, size_t(count) * 8);
-            copy_out(r.optical_length + first, dm + count, size_t(count) * 8);
-            copy_out(r.failed + first, dc, size_t(count) * 8);
-            copy_out(r.uncertain_ok + first, dc + count, size_t(count) * 8);
-            copy_out(r.uncertain_failed + first, dc + 2 * size_t(count), size_t(count) * 8);
+            const size_t n = size_t(count) * 8;
+            io_.out({{r.merit + first, dm, n},
+                     {r.optical_length + first, dm + count, n, true},
+                     {r.failed + first, dc, n, true},
+                     {r.uncertain_ok + first, dc + count, n, true},
+                     {r.uncertain_failed + first, dc + 2 * size_t(count), n, true}});
         }
         hip_check(hipDeviceSynchronize(), "prefilter");
         prefilter_decide(b, s, o, extra, r);
@@ -768,7 +943,7 @@ public:
         const int tranche = tranche_size(b.variants, per);
         for (int first = 0; first < b.variants; first += tranche) {
             const int count = std::min(tranche, b.variants - first);
-            batch_.upload(b, first, count, nullptr);
+            batch_.upload(b, first, count, io_);
             double* part = part_.as<double>(size_t(count) * T);
             int* pc = partc_.as<int>(size_t(count) * T * 2);
             double* ep = ext_part_.as<double>(size_t(count) * T * S * 2);
@@ -778,7 +953,7 @@ public:
                                                       nullptr, part, pc, nullptr, ep, ex, ~0ull,
                                                       nullptr));
             });
-            copy_out(out + size_t(first) * S * 2, ex, size_t(count) * S * 2 * 8);
+            io_.out({{out + size_t(first) * S * 2, ex, size_t(count) * S * 2 * 8}});
         }
         hip_check(hipDeviceSynchronize(), "surface extrema");
     }
@@ -796,11 +971,12 @@ public:
         const int tranche = tranche_size(b.variants, per);
         for (int first = 0; first < b.variants; first += tranche) {
             const int count = std::min(tranche, b.variants - first);
-            batch_.upload(b, first, count, nullptr);
+            batch_.upload(b, first, count, io_);
             merit_device(batch_.view, s, rp, extra ? extra + first : nullptr, count);
-            copy_out(merit + first, d_merit_, size_t(count) * 8);
-            copy_out(failed + first, d_failed_, size_t(count) * 8);
-            copy_out(hard + first, d_hard_, size_t(count) * 8);
+            const size_t n = size_t(count) * 8;
+            io_.out({{merit + first, d_merit_, n},
+                     {failed + first, d_failed_, n, true},
+                     {hard + first, d_hard_, n, true}});
         }
         hip_check(hipDeviceSynchronize(), "merit");
     }
@@ -815,14 +991,14 @@ public:
         double* part = part_.as<double>(size_t(count) * T);
         int* pc = partc_.as<int>(size_t(count) * T * 2);
         if (!md) {
-            md = d_merit_ = out_merit_.as<double>(size_t(count));
-            fd = d_failed_ = out_failed_.as<int64_t>(size_t(count));
-            hd = d_hard_ = out_hard_.as<int64_t>(size_t(count));
+            md = d_merit_ = out_merit_.as<double>(3 * size_t(count)); // one copy to the host
+            fd = d_failed_ = reinterpret_cast<int64_t*>(md + count);
+            hd = d_hard_ = fd + count;
         }
         const double* dextra = nullptr;
         if (extra_host) {
             double* e = extra_.as<double>(size_t(count));
-            hip_check(hipMemcpy(e, extra_host, size_t(count) * 8, hipMemcpyHostToDevice), "extra");
+            io_.in(e, extra_host, size_t(count) * 8);
             dextra = e;
         }
         double* ep = rp.Et ? ext_part_.as<double>(size_t(count) * T * S * 2) : nullptr;
@@ -916,13 +1092,12 @@ public:
             for (size_t i = 0; i < size_t(runs) * P; ++i)
                 if (!std::isfinite(x0[i])) throw std::invalid_argument("x0 not finite");
         }
-        if (base.variants == 1) tmpl_.upload(base, 0, 1, nullptr);
+        if (base.variants == 1) tmpl_.upload(base, 0, 1, io_);
         for (int first = 0; first < runs; first += chunk) {
             const int count = std::min(chunk, runs - first);
-            if (base.variants != 1) tmpl_.upload(base, first, count, nullptr);
+            if (base.variants != 1) tmpl_.upload(base, first, count, io_);
             double* dx = x_.as<double>(size_t(count) * P);
-            hip_check(hipMemcpy(dx, x0 + size_t(first) * P, size_t(count) * P * 8,
-                                hipMemcpyHostToDevice), "x0");
+            io_.in(dx, x0 + size_t(first) * P, size_t(count) * P * 8);
             double *dplus = nullptr, *dminus = nullptr, *dsp = nullptr, *dsm = nullptr;
             uint8_t* dsten = nullptr;
             if (pattern) {
@@ -932,11 +1107,11 @@ public:
                 dsp = sp_.as<double>(n);
                 dsm = sm_.as<double>(n);
                 dsten = sten_.as<uint8_t>(n);
-                hip_check(hipMemcpy(dplus, pat.plus.data() + o, n * 8, hipMemcpyHostToDevice), "pattern");
-                hip_check(hipMemcpy(dminus, pat.minus.data() + o, n * 8, hipMemcpyHostToDevice), "pattern");
-                hip_check(hipMemcpy(dsp, pat.step_plus.data() + o, n * 8, hipMemcpyHostToDevice), "steps");
-                hip_check(hipMemcpy(dsm, pat.step_minus.data() + o, n * 8, hipMemcpyHostToDevice), "steps");
-                hip_check(hipMemcpy(dsten, pat.stencil.data() + o, n, hipMemcpyHostToDevice), "stencil");
+                io_.in(dplus, pat.plus.data() + o, n * 8);
+                io_.in(dminus, pat.minus.data() + o, n * 8);
+                io_.in(dsp, pat.step_plus.data() + o, n * 8);
+                io_.in(dsm, pat.step_minus.data() + o, n * 8);
+                io_.in(dsten, pat.stencil.data() + o, n);
             }
             work_.allocate(base, count * per_run);
             dev_check(mko_internal::point_batch(
@@ -985,8 +1160,7 @@ public:
                             dsm, dsten, rs, rp, P, Je, re, E, 0);
                     dev_check(mko_internal::extra_normal(count, P, E, Je, re, da, dg, nullptr));
                 }
-                if (a) copy_out(a + size_t(first) * P * P, da, size_t(count) * P * P * 8);
-                if (g) copy_out(g + size_t(first) * P, dg, size_t(count) * P * 8);
+                copy_normal(a, g, first, count, P, da, dg);
                 hip_check(hipDeviceSynchronize(), "jacobian");
                 continue;
             }
@@ -1009,11 +1183,10 @@ public:
                 timer.run(kGram, [&] {
                     dev_check(gram(precision, dJ, dr0, count, P, R, da, dg));
                 });
-                if (a) copy_out(a + size_t(first) * P * P, da, size_t(count) * P * P * 8);
-                if (g) copy_out(g + size_t(first) * P, dg, size_t(count) * P * 8);
+                copy_normal(a, g, first, count, P, da, dg);
             }
-            if (J) copy_out(J + size_t(first) * P * R, dJ, size_t(count) * P * R * 8);
-            if (r0) copy_out(r0 + size_t(first) * R, dr0, size_t(count) * R * 8);
+            io_.out({{J ? J + size_t(first) * P * R : nullptr, dJ, J ? size_t(count) * P * R * 8 : 0},
+                     {r0 ? r0 + size_t(first) * R : nullptr, dr0, r0 ? size_t(count) * R * 8 : 0}});
             hip_check(hipDeviceSynchronize(), "jacobian");
         }
     }
@@ -1034,13 +1207,12 @@ public:
         const int chunk = tranche_size(runs, per);
         check_glass(base, vars);
         upload_vars(vars);
-        if (base.variants == 1) tmpl_.upload(base, 0, 1, nullptr);
+        if (base.variants == 1) tmpl_.upload(base, 0, 1, io_);
         for (int first = 0; first < runs; first += chunk) {
             const int count = std::min(chunk, runs - first);
-            if (base.variants != 1) tmpl_.upload(base, first, count, nullptr);
+            if (base.variants != 1) tmpl_.upload(base, first, count, io_);
             double* dx = x_.as<double>(size_t(count) * P);
-            hip_check(hipMemcpy(dx, x + size_t(first) * P, size_t(count) * P * 8,
-                                hipMemcpyHostToDevice), "x");
+            io_.in(dx, x + size_t(first) * P, size_t(count) * P * 8);
             work_.allocate(base, count);
             dev_check(mko_internal::point_batch(
                 &tmpl_.view, nullptr, base.variants != 1, count, 1, &dvars_, dx, nullptr, nullptr,
@@ -1050,9 +1222,10 @@ public:
                 work_.mut(work_.view.reference_curvature), work_.mut(work_.view.paraxial_index),
                 work_.mut(work_.view.buchdahl), nullptr));
             merit_device(work_.view, s, rp, nullptr, count);
-            copy_out(merit + first, d_merit_, size_t(count) * 8);
-            copy_out(failed + first, d_failed_, size_t(count) * 8);
-            copy_out(hard + first, d_hard_, size_t(count) * 8);
+            const size_t n = size_t(count) * 8;
+            io_.out({{merit + first, d_merit_, n},
+                     {failed + first, d_failed_, n, true},
+                     {hard + first, d_hard_, n, true}});
         }
         hip_check(hipDeviceSynchronize(), "point merit");
     }
@@ -1067,6 +1240,8 @@ public:
         if (owner && owner == vars_owner_) return;
         DeviceGuard guard(device_);
         upload_vars(v);
+        // the LM's cycles run on a stream of their own
+        hip_check(hipStreamSynchronize(nullptr), "variables");
         vars_owner_ = owner;
     }
 
@@ -1399,6 +1574,7 @@ public:
     int device() const { return device_; }
     const mko_internal::Tuning& tuning() const { return tuning_; }
     void set_tuning(const mko_internal::Tuning& t) { tuning_ = t; }
+    Staging& staging() { return io_; }
     KernelTimer timer;
 
 private:
@@ -1609,21 +1785,24 @@ private:
         if (n == 0) throw DeviceError("too little device memory for one variant");
         return int(std::min<size_t>(n, size_t(items)));
     }
-    void copy_out(void* host, const void* dev, size_t bytes) {
-        hip_check(hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost), "download");
+    void copy_normal(double* a, double* g, int first, int count, int P, const double* da,
+                     const double* dg) {
+        const size_t n = size_t(count) * P * 8;
+        io_.out({{a ? a + size_t(first) * P * P : nullptr, da, a ? n * P : 0},
+                 {g ? g + size_t(first) * P : nullptr, dg, g ? n : 0}});
     }
     void upload_vars(const mko_variables& v) {
         int32_t* t = vtype_.as<int32_t>(size_t(v.count));
         int32_t* s = vsurf_.as<int32_t>(size_t(v.count));
-        hip_check(hipMemcpy(t, v.type, size_t(v.count) * 4, hipMemcpyHostToDevice), "vars");
-        hip_check(hipMemcpy(s, v.batch_surface, size_t(v.count) * 4, hipMemcpyHostToDevice), "vars");
+        io_.in(t, v.type, size_t(v.count) * 4);
+        io_.in(s, v.batch_surface, size_t(v.count) * 4);
         dvars_ = v;
         dvars_.type = t;
         dvars_.batch_surface = s;
         dvars_.component = nullptr;
         if (v.component) {
             int32_t* c = vcomp_.as<int32_t>(size_t(v.count));
-            hip_check(hipMemcpy(c, v.component, size_t(v.count) * 4, hipMemcpyHostToDevice), "vars");
+            io_.in(c, v.component, size_t(v.count) * 4);
             dvars_.component = c;
         }
         vars_host_dev_ = v; // the adjoint entry point reads type/surface on the host
@@ -1634,11 +1813,12 @@ private:
     size_t limit_;
     mko_internal::Tuning tuning_;
     std::map<std::string, mko_internal::Tuning> tuned_; // autotuner's choices per shape
+    Staging io_;
     DeviceBatch batch_, tmpl_, work_, rowfd_, rowbase_;
     Buffer cand_part_, cand_pc_, cand_ep_, cand_ex_, cand_flags_, cand_tcount_, cand_tstart_,
         cand_list_, cand_count_, cand_over_, cand_flag_;
     int64_t candidate_chunks_ = 0, candidate_fallbacks_ = 0;
-    Buffer out_res_, out_opd_, out_st_, part_, partc_, out_merit_, out_failed_, out_hard_, extra_;
+    Buffer out_res_, out_opd_, out_st_, part_, partc_, out_merit_, extra_;
     Buffer ext_part_, ext_, rows_, esum_, tsum_, je_, re_, items_, hull_;
     std::vector<char> items_host_, hull_host_;
     Buffer states_, smerit_, sfailed_, shard_, spart_, spc_; // ray states of the glass mixed path
@@ -2176,7 +2356,9 @@ private:
         validate_values(base_, 0, base_.variants);
         check_glass(base_, vars_);
         eng_.set_variables(vars_, id_);
-        dev_tmpl_.upload(base_, 0, base_.variants, nullptr);
+        dev_tmpl_.upload(base_, 0, base_.variants, eng_.staging());
+        // the captured cycles run on a stream of their own
+        hip_check(hipStreamSynchronize(nullptr), "LM template");
         double* bnd = bounds_d_.as<double>(3 * P_);
         hip_check(hipMemcpy(bnd, vars_.lower, P_ * 8, hipMemcpyHostToDevice), "bounds");
         hip_check(hipMemcpy(bnd + P_, vars_.upper, P_ * 8, hipMemcpyHostToDevice), "bounds");
@@ -2705,20 +2887,17 @@ private:
         std::vector<double> x(n * P_), merit(n), mu(n), gn(n), md(n);
         std::vector<int64_t> failed(n), hard(n);
         std::vector<int32_t> status(n), it(n), acc(n), jac(n);
-        auto get = [](void* h, const void* d, size_t b) {
-            hip_check(hipMemcpy(h, d, b, hipMemcpyDeviceToHost), "LM state");
-        };
-        get(x.data(), ds_.x, n * P_ * 8);
-        get(merit.data(), ds_.merit, n * 8);
-        get(mu.data(), ds_.mu, n * 8);
-        get(gn.data(), ds_.gradient_norm, n * 8);
-        get(md.data(), ds_.model_decrease, n * 8);
-        get(failed.data(), ds_.failed, n * 8);
-        get(hard.data(), ds_.hard, n * 8);
-        get(status.data(), ds_.status, n * 4);
-        get(it.data(), ds_.iterations, n * 4);
-        get(acc.data(), ds_.accepted, n * 4);
-        get(jac.data(), ds_.jacobians, n * 4);
+        eng_.staging().out({{x.data(), ds_.x, n * P_ * 8},
+                            {merit.data(), ds_.merit, n * 8},
+                            {mu.data(), ds_.mu, n * 8},
+                            {gn.data(), ds_.gradient_norm, n * 8},
+                            {md.data(), ds_.model_decrease, n * 8},
+                            {failed.data(), ds_.failed, n * 8},
+                            {hard.data(), ds_.hard, n * 8},
+                            {status.data(), ds_.status, n * 4},
+                            {it.data(), ds_.iterations, n * 4},
+                            {acc.data(), ds_.accepted, n * 4},
+                            {jac.data(), ds_.jacobians, n * 4}});
         for (size_t i = 0; i < n; ++i) {
             Run& r = state_[i];
             r.x.assign(x.begin() + std::ptrdiff_t(i * P_), x.begin() + std::ptrdiff_t((i + 1) * P_));
