@@ -34,6 +34,7 @@
 
 #include "error.hpp"
 #include "internal.hpp"
+#include "launch_plan.hpp"
 #include "lm_device.hpp"
 #include "mikroptim_hip.h"
 
@@ -1077,7 +1078,9 @@ public:
                                   : size_t(P) * R * 8 + size_t(R) * 8 + size_t(rays)) +
                            size_t(P) * (P + 1) * 8 + 64 * size_t(P) +
                            (!fd ? rows_fd_bytes(rp, base, P) : 0);
-        const int chunk = tranche_size(runs, per);
+        int chunk = tranche_size(runs, per);
+        if (fd && !fd_stored)
+            chunk = int(std::min<int64_t>(chunk, mko_internal::fd_direct_runs(P, int64_t(Tt))));
         check_glass(base, vars);
         upload_vars(vars);
         Pattern pat;
@@ -1275,7 +1278,9 @@ public:
                            (fused ? Tt * (size_t(P) * P * 4 + size_t(P) * 64 + 24) + 1024
                                   : size_t(P) * R * 8 + size_t(R) * 8) +
                            size_t(P) * 48 + 64 + (!fd ? rows_fd_bytes(rp, tmpl, P) : 0);
-        const int chunk = tranche_size(count, per);
+        int chunk = tranche_size(count, per);
+        if (fd && !fd_stored)
+            chunk = int(std::min<int64_t>(chunk, mko_internal::fd_direct_runs(P, int64_t(Tt))));
         for (int first = 0; first < count; first += chunk) {
             const int c = std::min(chunk, count - first);
             const double* x = xd + size_t(first) * P;

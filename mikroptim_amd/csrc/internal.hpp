@@ -134,7 +134,8 @@ int gram_chain(const double* jacobian, const double* r0, int runs, int variables
 // variants, device), J / r0 rows at jstride: the values of RESIDUALS of every variant and
 // mko_fd_difference_device, bit for bit, without the differences' residuals in memory.
 // fd_direct: whether it applies (FP64 trace, no glass variable on the medium before the first
-// surface, up to 320 variables whose moved steps fit the LDS); vars: host arrays.
+// surface, up to 320 variables whose moved steps fit the LDS); vars: host arrays. A call takes at
+// most fd_direct_runs (launch_plan.hpp) runs.
 bool fd_direct(const mko_batch& batch, const mko_residual_settings& s, const mko_variables& vars);
 int fd_jacobian(const mko_batch* fd_batch, const mko_residual_settings* settings,
                 const mko_variables* vars, int runs, const double* step_plus,

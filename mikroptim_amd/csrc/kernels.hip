@@ -29,6 +29,7 @@
 #include "error.hpp"
 #include "gauss_legendre_table.h"
 #include "internal.hpp"
+#include "launch_plan.hpp"
 #include "mikroptim_hip.h"
 #include "constraints.hpp"
 #include "trace_device.hpp"
@@ -4163,7 +4164,7 @@ int fd_jacobian(const mko_batch* fd_batch, const mko_residual_settings* settings
                 const int f = curv && s == 0 ? S : glass || curv ? s : s + 1;
                 if (f == first) plan.var[at++] = k | (f << 16) | (int(glass) << 24);
             }
-        if (int64_t(runs) * P.T > 0x1fffffffLL) throw std::invalid_argument("batch too large");
+        if (runs > fd_direct_runs(plan.P, P.T)) throw std::invalid_argument("batch too large");
         // A tuple's variables are dealt out to 1, 2 or 4 workgroups (each traces the point itself,
         // 2 of the about 2 + P passes) where there are few tuples: 1024 workgroups run at once, and
         // 1120 (32 runs of the 35-tuple objective) leave most of a second round empty (2.25 ms in
