@@ -3070,6 +3070,7 @@ __global__ __launch_bounds__(512) void gram_kernel(const double* J, const double
     const int tg = (P + 15) / 16, gw = (P + 63) / 64;
     const int units = gw + tg * (tg + 1) / 2;
     const int first = part * upp, last = min(units, first + upp);
+    if (first >= last) return; // no such part (gram_plan makes none)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m = lane & 15, kk = lane >> 4;
     f64x4 acc[kT];
@@ -4101,16 +4102,11 @@ int gram_chain(const double* jacobian, const double* r0, int runs, int variables
             check_hip(hipGetLastError(), "gram launch");
             return 0;
         }
-        const int tg = (variables + 15) / 16, gw = (variables + 63) / 64;
-        const int units = gw + tg * (tg + 1) / 2;
-        // Workgroups per run: at least 4 units (one tile per SIMD) each, and only while the runs
-        // leave CUs idle (up to 512 workgroups): beyond that a second workgroup only reads most
-        // of the run's J again.
-        const int parts = std::max(1, std::min((units + 3) / 4, 512 / runs));
-        const int upp = (units + parts - 1) / parts;
+        const GramPlan plan = gram_plan(variables, runs);
+        const int parts = plan.parts, upp = plan.upp;
         const auto launch = [&](auto kernel, int stage) {
             hipLaunchKernelGGL(kernel, dim3(unsigned(runs) * unsigned(parts)), dim3(512),
-                               size_t(16 * tg + 1) * size_t(stage + 2) * sizeof(double), s,
+                               size_t(16 * plan.tg + 1) * size_t(stage + 2) * sizeof(double), s,
                                jacobian, r0, variables, rows, parts, upp, a, g, live);
         };
         // staged values per thread: (variables + 1) columns / 8 waves x (rows of a stage) / 64;

@@ -2,8 +2,8 @@
 per element, ascending rows) where the kernel's shapes change: edges of 16-column tiles and of
 64-column g units, the column counts with another stage (55 / 56, 64 / 65), the most variables of
 the tile kernel (127) and the wide kernel above them, rows around the staged 64 / 128, and run
-counts with one or several workgroups per run. Values of mixed signs over 24 decades, so that
-another order of any sum shows."""
+counts with one or several workgroups per run, also where they do not divide its tiles. Values of
+mixed signs over 24 decades, so that another order of any sum shows."""
 
 import ctypes as C
 
@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1, 1), (2, 1, 5), (3, 15, 3), (1, 16, 127), (5, 17, 128), (2, 47, 129),
           (1, 48, 1000), (600, 48, 131), (3, 55, 257), (2, 56, 64), (3, 64, 300), (2, 65, 63),
-          (7, 96, 193), (520, 96, 65), (2, 127, 130), (600, 127, 33), (2, 128, 70), (1, 200, 40)]
+          (7, 96, 193), (520, 96, 65), (2, 127, 130), (600, 127, 33), (2, 128, 70), (1, 200, 40),
+          (70, 100, 70), (54, 120, 65)]
 
 
 @pytest.mark.parametrize("runs,P,rows", SHAPES)

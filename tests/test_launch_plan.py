@@ -89,3 +89,31 @@ int main() {
 
 def test_fd_jacobian_refuses_more_tuples_than_it_can_count(tmp_path):
     run_program(tmp_path, FD_RUNS)
+
+
+GRAM_PARTS = r"""
+#include "launch_plan.hpp"
+#include <cstdio>
+using namespace mko_internal;
+
+int main() {
+    int fails = 0;
+    for (int P = 1; P <= 127; ++P)
+        for (int runs = 1; runs <= 600; ++runs) {
+            const GramPlan p = gram_plan(P, runs);
+            // every unit belongs to a part and every part has one; a wave's units fit the
+            // accumulators of the kernels launched (2 of 8 waves up to 64 variables, else 5)
+            if (p.parts < 1 || p.upp < 1 || (p.parts - 1) * p.upp >= p.units ||
+                p.parts * p.upp < p.units || p.upp > 8 * (P <= 64 ? 2 : 5)) {
+                if (++fails <= 10)
+                    std::printf("P %d runs %d: %d units, %d parts of %d\n", P, runs, p.units,
+                                p.parts, p.upp);
+            }
+        }
+    return fails != 0;
+}
+"""
+
+
+def test_gram_parts_cover_the_units_and_none_is_empty(tmp_path):
+    run_program(tmp_path, GRAM_PARTS)
