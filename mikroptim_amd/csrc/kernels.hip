@@ -4093,7 +4093,8 @@ int adjoint_jacobian(const mko_batch* batch, const mko_residual_settings* settin
 int gram_chain(const double* jacobian, const double* r0, int runs, int variables, int64_t rows,
                double* a, double* g, void* stream, const int32_t* live) {
     MKO_TRY({
-        if (runs <= 0) return 0;
+        if (runs <= 0 || variables == 0) return 0;
+        if (variables < 0) throw std::invalid_argument("negative variable count");
         const hipStream_t s = static_cast<hipStream_t>(stream);
         if (variables > 127) {
             const int T = (variables + 1 + 63) / 64;

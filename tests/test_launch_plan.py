@@ -117,3 +117,9 @@ int main() {
 
 def test_gram_parts_cover_the_units_and_none_is_empty(tmp_path):
     run_program(tmp_path, GRAM_PARTS)
+
+
+def test_gram_without_variables_has_nothing_to_do():
+    lib = engine.library()
+    assert lib.mko_gram_device(None, None, 3, 0, 40, None, None, None) == 0
+    assert lib.mko_gram_device(None, None, 3, -1, 40, None, None, None) != 0
