@@ -49,3 +49,14 @@ def test_points_after_a_refused_call(engine):
     for i in range(5):
         ai, gi = engine.normal_equations(b.take([0]), s, v, x[i:i + 1], method="fd")
         assert np.array_equal(ai[0], a[i]) and np.array_equal(gi[0], g[i])
+
+
+def test_points_of_more_than_two_slots(engine):
+    b, v = systems.singlet(2)
+    runs = (5 << 19) // (8 * v.size) + 1  # 2.5 MiB of points and of each array of the pattern
+    x = v.extract(b)[1] * (1.0 + 1e-3 * np.random.default_rng(8).standard_normal((runs, v.size)))
+    s = ResidualSettings(rings=1, spokes=2, failure=abi.FAILURE_HARD)
+    a, g = engine.normal_equations(b.take([0]), s, v, x, method="fd")
+    ids = np.unique(np.linspace(0, runs - 1, 40).astype(int))
+    a1, g1 = engine.normal_equations(b.take([0]), s, v, x[ids], method="fd")
+    assert np.array_equal(a[ids], a1) and np.array_equal(g[ids], g1)
