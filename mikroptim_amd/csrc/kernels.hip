@@ -1233,6 +1233,7 @@ __global__ __launch_bounds__(256) void merit_finalize_kernel(
 struct PfStep {
     float c, t, n, mu; // effective curvature, thickness and index before the surface, n / n'
 };
+static_assert(sizeof(PfStep) == mko_internal::kPrefilterStepBytes);
 
 // Quotient and root in 4 and 6 instructions (the correctly rounded ones of the compiler take
 // about 10 and 15 and were half of the trace): the hardware's estimate and one step on the residual,
@@ -1380,10 +1381,6 @@ __device__ __forceinline__ float block_max_f(float v, float* lds) {
     return m;
 }
 
-// LDS slots of a tuple's n rays: a multiple of the q lanes by an odd number, so that the tuples
-// side by side fall on different banks.
-__host__ __device__ __forceinline__ int prefilter_slots(int n, int q) { return q * (((n + q - 1) / q) | 1); }
-
 // OPL relative to the axial optical length (prefilter_opl_offset), classes 0 certain valid / 1
 // certain failed / 2, 3 uncertain (margin <= eta), the piston over the certain-valid rays and the
 // tuple's sum of squared residuals; partials per tuple: merit (as double), largest optical length,
@@ -1415,7 +1412,7 @@ __global__ __launch_bounds__(kBlock) void prefilter_kernel(TraceParams P, int Q,
     PfStep* steps = reinterpret_cast<PfStep*>(pf_lds);        // [G][pitch]
     float2* spoke = reinterpret_cast<float2*>(steps + G * pitch); // [M]
     float* opl_l = reinterpret_cast<float*>(spoke + M);           // [G][rays]
-    const int rays = prefilter_slots(n, q);
+    const int rays = mko_internal::prefilter_slots(n, q);
     uint8_t* cls_l = reinterpret_cast<uint8_t*>(opl_l + G * rays); // [G][rays]
     for (int e = tid; e < G * P.S; e += kBlock) {
         const int g = e / P.S, s = e - g * P.S;
@@ -3359,16 +3356,6 @@ int largest_tuple(const TraceParams& P) {
     return nmax;
 }
 
-// Lanes per tuple of the prefilter, by its largest tuple: the most of 8 ... 64 that idle on at most
-// 1/8 of the rays' slots (72 rays: 16 lanes of 5 rays; 8 lanes if none does), a whole workgroup
-// above 256 rays.
-int prefilter_lanes(int n) {
-    if (n > 256) return kBlock;
-    for (int q = 64; q > 8; q /= 2)
-        if (8 * n >= 7 * q * ((n + q - 1) / q)) return q;
-    return 8;
-}
-
 int rays_per_lane(const TraceParams& P) {
     const int r = (largest_tuple(P) + kBlock - 1) / kBlock;
     return r <= 1 ? 1 : r <= 2 ? 2 : r <= 4 ? 4 : 8;
@@ -3838,21 +3825,10 @@ int prefilter_stats(const mko_batch* batch, const mko_residual_settings* setting
         int* pc = reinterpret_cast<int*>(w + tuples * 12);
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const float eta = float(boundary);
-        // lanes per tuple: those of the sums, doubled (up to one ray per lane) while the launch has
-        // less than 4 workgroups per CU. One variant of 35 tuples of 72 rays and 25 surfaces, the
-        // whole call: 211 us with 16 lanes, 176 with 128; 2000 variants of 9 tuples of 72 rays and
-        // more keep the lanes of the sums (512 variants of 35 tuples: 550 -> 418 us)
-        const int n = largest_tuple(P), q = prefilter_lanes(n);
-        int Q = q;
-        const auto groups = [&] { return (P.V + kBlock / Q - 1) / (kBlock / Q); };
-        while (Q < kBlock && Q < n && int64_t(groups()) * P.T < 1024) Q *= 2;
-        const int G = kBlock / Q;
-        const size_t lds = size_t(G) * (P.S | 1) * sizeof(PfStep) +
-                           size_t(std::max(1, P.spokes)) * sizeof(float2) +
-                           size_t(G) * prefilter_slots(n, q) * (sizeof(float) + 1);
-        const auto kernel = q == kBlock ? prefilter_kernel<true> : prefilter_kernel<false>;
-        hipLaunchKernelGGL(kernel, dim3(unsigned(groups()) * unsigned(P.T)), dim3(kBlock), lds, s,
-                           P, Q, q, eta, pm, pl, pc);
+        const PrefilterPlan p = prefilter_plan(P.V, P.T, P.S, P.rings, largest_tuple(P));
+        const auto kernel = p.q == kBlock ? prefilter_kernel<true> : prefilter_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(p.groups) * unsigned(P.T)), dim3(kBlock), p.lds, s,
+                           P, p.Q, p.q, eta, pm, pl, pc);
         check_hip(hipGetLastError(), "prefilter launch");
         hipLaunchKernelGGL(prefilter_finalize_kernel, dim3((P.V + 255) / 256), dim3(256), 0, s,
                            P.V, P.T, pm, pl, pc, merit, optical, failed, uncertain_ok,

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cstddef>
 #include <cstdint>
 
 namespace mko_internal {
@@ -31,6 +32,45 @@ inline GramPlan gram_plan(int variables, int runs) {
     p.parts = std::max(1, std::min((p.units + 3) / 4, 512 / runs));
     p.upp = (p.units + p.parts - 1) / p.parts;
     p.parts = (p.units + p.upp - 1) / p.upp; // rounding upp up may leave fewer
+    return p;
+}
+
+// LDS slots of a tuple's n rays: a multiple of the q lanes by an odd number, so that the tuples
+// side by side fall on different banks.
+constexpr int prefilter_slots(int n, int q) { return q * (((n + q - 1) / q) | 1); }
+
+// Lanes of prefilter_kernel that sum a tuple, by the largest tuple: the most of 8 ... 64 that idle on
+// at most 1/8 of the rays' slots (72 rays: 16 lanes of 5 rays; 8 lanes if none does), a whole
+// workgroup above 256 rays.
+inline int prefilter_lanes(int n) {
+    if (n > 256) return 256;
+    for (int q = 64; q > 8; q /= 2)
+        if (8 * n >= 7 * q * ((n + q - 1) / q)) return q;
+    return 8;
+}
+
+constexpr size_t kPrefilterStepBytes = 16;
+
+// prefilter_kernel's lanes per tuple (q sum it, Q trace it), workgroups per tuple index and dynamic
+// LDS for `variants` of `tuples` tuples of up to n rays on `rings` rings.
+struct PrefilterPlan {
+    int q, Q, groups;
+    size_t lds;
+};
+// Q is q, doubled (up to one ray per lane) while the launch has less than 4 workgroups per CU. One
+// variant of 35 tuples of 72 rays and 25 surfaces, the whole call: 211 us with 16 lanes, 176 with
+// 128; 2000 variants of 9 tuples of 72 rays and more keep the lanes of the sums (512 variants of 35
+// tuples: 550 -> 418 us).
+inline PrefilterPlan prefilter_plan(int variants, int tuples, int surfaces, int rings, int n) {
+    PrefilterPlan p{};
+    p.q = p.Q = prefilter_lanes(n);
+    const auto groups = [&] { return (variants + 256 / p.Q - 1) / (256 / p.Q); };
+    while (p.Q < 256 && p.Q < n && int64_t(groups()) * tuples < 1024) p.Q *= 2;
+    p.groups = groups();
+    const size_t G = size_t(256 / p.Q);
+    p.lds = G * size_t(surfaces | 1) * kPrefilterStepBytes +
+            size_t(n / rings) * 2 * sizeof(float) + // the most spokes of a field
+            G * size_t(prefilter_slots(n, p.q)) * (sizeof(float) + 1);
     return p;
 }
 

@@ -54,3 +54,13 @@ def test_many_surfaces(engine, rings, spokes):
     m, f, _ = engine.merit(b, s)
     assert np.all(g.failed == 0) and np.all(f == 0)
     assert np.all(g.merit_lower <= m) and np.all(m <= g.merit_upper)
+
+
+def test_axis_fields_take_any_number_of_spokes(engine):
+    """An axis field has one spoke, whatever the settings say."""
+    b, _ = systems.singlet_multistart(40, seed=5)
+    b.pupil_mode = np.full(b.fields, abi.PUPIL_AXIS, dtype=np.uint8)
+    g = [engine.prefilter(b, ResidualSettings(rings=6, spokes=n, failure=abi.FAILURE_HARD))
+         for n in (1, 50000)]
+    for name in NAMES:
+        assert np.array_equal(getattr(g[0], name), getattr(g[1], name)), name

@@ -123,3 +123,36 @@ def test_gram_without_variables_has_nothing_to_do():
     lib = engine.library()
     assert lib.mko_gram_device(None, None, 3, 0, 40, None, None, None) == 0
     assert lib.mko_gram_device(None, None, 3, -1, 40, None, None, None) != 0
+
+
+PREFILTER_LDS = r"""
+#include "launch_plan.hpp"
+#include <cstdio>
+using namespace mko_internal;
+
+int main() {
+    int fails = 0;
+    for (int V : {1, 3, 100, 2001, 20000})
+        for (int T : {1, 9, 35, 1024})
+            for (int S : {2, 3, 25, 64})
+                for (int rings = 1; rings <= 16; ++rings)
+                    for (int M = 1; rings * M <= 2048; ++M) {
+                        const PrefilterPlan p = prefilter_plan(V, T, S, rings, rings * M);
+                        // beside it 1 KB of static LDS; 64 KB always fit a workgroup
+                        const bool fits = p.lds + 1024 <= 65536 &&
+                            p.lds >= size_t(256 / p.Q) * (S * kPrefilterStepBytes +
+                                                          size_t(rings) * M * 5) + size_t(M) * 8;
+                        const bool lanes = p.q >= 8 && p.q <= p.Q && p.Q <= 256 &&
+                            int64_t(p.groups) * (256 / p.Q) >= V &&
+                            int64_t(p.groups - 1) * (256 / p.Q) < V;
+                        if ((!fits || !lanes) && ++fails <= 10)
+                            std::printf("V %d T %d S %d rings %d spokes %d: q %d Q %d lds %zu\n", V,
+                                        T, S, rings, M, p.q, p.Q, p.lds);
+                    }
+    return fails != 0;
+}
+"""
+
+
+def test_prefilter_lds_holds_the_samples_of_the_largest_tuple(tmp_path):
+    run_program(tmp_path, PREFILTER_LDS)
