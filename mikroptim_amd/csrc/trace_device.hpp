@@ -475,10 +475,8 @@ struct alignas(16) Step {
     double cna; // c n_after^2
 };
 
-// sqrt(x) and 1 / (2 sqrt(x)) for x > 0 (rev_sqrt_half_rcp without its branch); 0 for x = 0. A
-// negative or NaN x gives an unspecified value: the callers test x.
-__device__ __forceinline__ double sqrt_pos(double x, double& half_rcp) {
-    const double y = __builtin_amdgcn_rsq(__builtin_fmax(x, 0x1p-900));
+// sqrt(x) and 1 / (2 sqrt(x)) from the estimate y of 1 / sqrt(x): rev_sqrt_half_rcp's iteration.
+__device__ __forceinline__ double sqrt_from(double x, double y, double& half_rcp) {
     double g = x * y, h = 0.5 * y;
     const double r = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, r, g);
@@ -486,9 +484,19 @@ __device__ __forceinline__ double sqrt_pos(double x, double& half_rcp) {
     half_rcp = h;
     return __builtin_fma(__builtin_fma(-g, g, x), h, g);
 }
+// sqrt(x) for x > 0 without a branch; 0 for x = 0. A negative or NaN x gives an unspecified value:
+// the steps test x.
 __device__ __forceinline__ double sqrt_pos(double x) {
     double h;
-    return sqrt_pos(x, h);
+    return sqrt_from(x, __builtin_amdgcn_rsq(__builtin_fmax(x, 0x1p-900)), h);
+}
+// The root of a squared P . N (n2 = n^2 of its medium) that the reverse sweep forms from the way
+// back, and 1 / (2 root). The trace accepted the ray with a square >= 0; rounding, some 2^-52 n^2,
+// may leave this one below zero where the ray grazes the surface, so it is held at that size: the
+// gradients stay those of a grazing ray instead of overflowing.
+__device__ __forceinline__ double sweep_root(double x, double n2, double& half_rcp) {
+    const double v = __builtin_fmax(x, 0x1p-52 * n2);
+    return sqrt_from(v, __builtin_amdgcn_rsq(v), half_rcp);
 }
 
 // The line through Q (in the frame of surface s) along +-P: its point nearest the vertex, where
@@ -656,7 +664,7 @@ __device__ __forceinline__ SweepState sweep_start(V3<double> p, V3<double> P, V3
 // surface; returns the curvature gradient. On entry a = P' . N.
 __device__ __forceinline__ double sweep_refract(SweepState& w, const Step& k) {
     double h;
-    const double a = sqrt_pos(__builtin_fma(w.a, w.a, -k.dn2), h);
+    const double a = sweep_root(__builtin_fma(w.a, w.a, -k.dn2), k.n2, h);
     const double g = w.a - a;
     const double u = dot(w.dP, w.N) - k.c * dot(w.P, w.dq); // change of P' . N
     const double dg = u * g * (h + h);                      // minus the change of g
@@ -675,7 +683,7 @@ template <bool kIndex>
 __device__ __forceinline__ void sweep_transfer(SweepState& w, const Step& k, double c, double cna,
                                                double n, double& length) {
     const StepFoot f = step_foot(V3<double>{w.q.x, w.q.y, w.q.z + k.t}, w.P, c, k.ni2, cna);
-    w.a = sqrt_pos(f.D, w.ha);
+    w.a = sweep_root(f.D, k.n2, w.ha);
     const double lam = rev_div(f.H, w.P.z + w.a);
     w.q = V3<double>{f.x + lam * w.P.x, f.y + lam * w.P.y, f.z + lam * w.P.z};
     const double back = f.l0 + lam; // q = Q + back P

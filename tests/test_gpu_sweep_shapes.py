@@ -97,3 +97,36 @@ def test_unswept_column_is_zero(engine):
     x = v.extract(b)[:2].copy()
     J = _check(engine, b.take([0]), s, v, x)
     assert np.all(J[:, 1] == 0.0) and np.all(np.any(J[:, [0, 2, 3]] != 0.0, axis=2))
+
+
+def test_grazing_rays_leave_finite_gradients(engine):
+    """The outer ring meets the first sphere within rounding of grazing (its radius is the ring's, to a
+    few units in the last place): whatever rounding makes of the sweep's cosine there, the columns,
+    the products with them and the fused normal equations stay finite wherever the trace accepts
+    the rays with a cosine above zero."""
+    import torch
+    from mikroptim_amd.autograd import trace_residuals
+
+    b, v = systems.singlet(2)
+    base = b.take([0])
+    base.index[:, 2] = base.index[:, 1]  # the second sphere refracts nothing
+    base.field_angle[:] = base.field_target[:] = 0.0
+    base.pupil_mode[:] = abi.PUPIL_FULL
+    base.thickness[:, 2] = 400.0
+    s = ResidualSettings(rings=2, spokes=6, failure=abi.FAILURE_HARD)
+    u = np.polynomial.legendre.leggauss(2)[0][1]
+    edge = 1.0 / (base.pupil_radius[0] * np.sqrt(0.5 * (u + 1.0)))
+    x = np.tile(v.extract(base), (40, 1))
+    # the last variable is the working distance; curvature 0 towards the edge, 1 to 40 units below
+    x[:, 0] = edge * (1.0 - np.arange(1, 41) * 2.0 ** -52)
+    v.upper[0] = 1.0
+    J, _, a, g = engine.jacobian(base, s, v, x, method="adjoint", precision="fp64")
+    assert np.isfinite(J).all() and np.isfinite(a).all() and np.isfinite(g).all()
+    Jo = oracle().adjoint_jacobian(base, s, v, x)[0]
+    grazing = np.abs(Jo[:, 0]).max(axis=1)
+    assert np.sum(grazing > 1e5) > 10  # the rays are accepted and graze
+    am, gm = engine.normal_equations(base, s, v, x, method="adjoint", precision="mixed")
+    assert np.isfinite(am).all() and np.isfinite(gm).all()
+    xt = torch.tensor(x, dtype=torch.float64, device="cuda", requires_grad=True)
+    trace_residuals(xt, engine, base, s, v).sum().backward()
+    assert torch.isfinite(xt.grad).all()
