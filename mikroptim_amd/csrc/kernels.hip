@@ -1688,12 +1688,14 @@ __global__ void point_batch_kernel(ConstBatchPtrs src, BatchPtrs dst, int runs, 
     }
 }
 
-// fd_derivative (fd_formula.hpp:39) from the residual at the point and at its two differences.
+// fd_derivative (fd_formula.hpp:39) from the residual at the point and at its two differences. The
+// contraction is spelled out, so every kernel that inlines it computes the same bits.
 __device__ __forceinline__ double fd_derivative(double a0, double aa, double ab, double da,
                                                 double db, uint8_t stencil) {
+#pragma clang fp contract(off)
     if (stencil == MKO_STENCIL_ONE_SIDED) {
         const double ga = aa - a0, gb = ab - a0;
-        return (db * db * ga - da * da * gb) / (da * db * (db - da));
+        return __builtin_fma(db * db, ga, -(da * da * gb)) / (da * db * (db - da));
     }
     return (aa - ab) / (da - db);
 }

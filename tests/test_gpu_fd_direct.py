@@ -155,3 +155,58 @@ def test_general_path_kept(engine):
     sd.precision = abi.PRECISION_DF64
     Jd = engine.jacobian(base, sd, v, x, method="fd")[0]
     assert np.all(np.linalg.norm(Jd - J, axis=2) <= 1e-2 * np.linalg.norm(J, axis=2))
+
+
+@pytest.mark.parametrize("failure", [abi.FAILURE_HARD, abi.FAILURE_SOFT])
+def test_equal_bits_to_the_difference_kernel(engine, failure):
+    """Every stencil against mko_fd_difference_device on the residuals of the same points."""
+    import ctypes as C
+
+    import torch
+    from mikroptim_amd.engine import library
+
+    b, v = systems.singlet(6, seed=3)
+    base, x = b.take([0]), v.extract(b)
+    v.lower[0] = x[1, 0]  # central, one-sided, truncated by the run and the variable
+    v.upper[1] = x[2, 1]
+    v.lower[2], v.upper[2] = x[0, 2] - 4e-8, x[0, 2] + 4e-8
+    x[:, 0] = np.maximum(x[:, 0], v.lower[0])
+    x[:, 1] = np.minimum(x[:, 1], v.upper[1])
+    s = ResidualSettings(rings=5, spokes=13, failure=failure)
+    runs, P = x.shape
+    patterns = [oracle().fd_pattern(base, v, xi) for xi in x]
+    sten = np.array([p[5] for p in patterns], dtype=np.uint8)
+    assert {0, 1, 2} == set(int(q) for q in sten.ravel())
+    pts = []
+    for xi, (_, plus, minus, _, _, _) in zip(x, patterns):
+        pts.append(xi)
+        for k in range(P):
+            for value in (plus[k], minus[k]):
+                p = xi.copy()
+                p[k] = value
+                pts.append(p)
+    many = base.take(np.zeros(len(pts), dtype=np.int64))
+    v.apply(many, np.array(pts))
+    r, _, _ = engine.residuals(many, s)
+    rows = r.shape[1]
+
+    def dev(a):
+        return torch.tensor(np.ascontiguousarray(a), device="cuda")
+
+    res, sp, sm, st = dev(r), dev(np.array([p[3] for p in patterns])), \
+        dev(np.array([p[4] for p in patterns])), dev(sten)
+    Jd = torch.full((runs, P, rows), float("nan"), dtype=torch.float64, device="cuda")
+    rd = torch.full((runs, rows), float("nan"), dtype=torch.float64, device="cuda")
+    d, u = C.POINTER(C.c_double), C.POINTER(C.c_uint8)
+
+    def ptr(t, kind=d):
+        return C.cast(C.c_void_p(t.data_ptr()), kind)
+
+    rc = library().mko_fd_difference_device(
+        ptr(res), C.c_int64(rows), C.cast(None, u), C.c_int64(0), runs, P, C.c_int64(rows), ptr(sp),
+        ptr(sm), ptr(st, u), ptr(Jd), ptr(rd), C.cast(None, C.POINTER(C.c_int64)), None)
+    assert rc == 0, library().mko_last_error()
+    torch.cuda.synchronize()
+    J, r0, _, _ = engine.jacobian(base, s, v, x, method="fd", precision="fp64")
+    assert np.array_equal(r0, rd.cpu().numpy())
+    assert np.array_equal(J, Jd.cpu().numpy())
