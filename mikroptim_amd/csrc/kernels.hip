@@ -3041,8 +3041,8 @@ typedef __attribute__((ext_vector_type(4))) double f64x4;
 // Each element is one FMA chain over the rows in ascending order starting from 0 (gram_dot,
 // normal_equations.hpp:19), products of the stored J values: bitwise the host definition.
 // v_mfma_f64_16x16x4_f64 adds its four products to the accumulator as that chain does (measured
-// bit for bit on MI355X against the VALU chain over rows of mixed signs and 24 decades; the GPU
-// tests hold it), so J^T J runs on it in 16 x 16 tiles; operand lane l: A(m = l % 16, k = l / 16),
+// bit for bit on MI355X against the VALU chain over rows of mixed signs and 24 decades, subnormal
+// numbers, zeros of either sign, infinities and NaN; the GPU tests hold it), so J^T J runs on it in 16 x 16 tiles; operand lane l: A(m = l % 16, k = l / 16),
 // B(k = l / 16, n = l % 16), result lane l, element e: row 4 e + l / 16, column l % 16. g is a
 // VALU chain per column beside the tiles: as a matrix column it would cost a row of tiles of its
 // own (10 instead of 6 at 48 variables).
@@ -3130,8 +3130,7 @@ __global__ __launch_bounds__(512) void gram_kernel(const double* J, const double
             if (tI[i] >= 0) {
                 const double* xa = Xs + size_t(tI[i] * 16 + m) * kLd + kk;
                 const double* xb = Xs + size_t(tJ[i] * 16 + m) * kLd + kk;
-                // rows beyond n are staged as zeros: their products leave the sums as they are
-                const int steps = (n + 3) / 4;
+                const int steps = n >> 2; // the last 1 ... 3 rows below
 #pragma unroll 8
                 for (int st = 0; st < steps; ++st)
                     acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[4 * st], xb[4 * st], acc[i],
@@ -3143,6 +3142,19 @@ __global__ __launch_bounds__(512) void gram_kernel(const double* J, const double
                 for (int r = 0; r < n; ++r) gacc[i] = __fma_rn(x[r], Xr[r], gacc[i]);
             }
         }
+    }
+    // the rows beyond the last multiple of 4, still staged: the instruction's other rows are zeros
+    // times -0, which leave every sum as it is, also -0
+    const int rest = int(rows & 3), at = int((rows & ~int64_t(3)) % kC);
+    if (rest) {
+#pragma unroll
+        for (int i = 0; i < kT; ++i)
+            if (tI[i] >= 0) {
+                const double* xa = Xs + size_t(tI[i] * 16 + m) * kLd + kk + at;
+                const double* xb = Xs + size_t(tJ[i] * 16 + m) * kLd + kk + at;
+                acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(*xa, kk < rest ? *xb : -0.0, acc[i],
+                                                              0, 0, 0);
+            }
     }
     double* A = a + size_t(run) * P * P;
 #pragma unroll
