@@ -2954,8 +2954,8 @@ void adjoint_normal_kernel(TraceParams P, ParamMap map, float* partC, double* pa
 // triangle (mirrored on output), kE per thread; the tuples' S, Tr and factors are staged through
 // LDS 16 tuples at a time and the C of 4 tuples are loaded together (the sum over the tuples is
 // one dependent chain per entry, their loads are not). What bounds it is latency up to some
-// hundred runs, then the reading of C (4 P^2 bytes per tuple): with few runs one entry per thread
-// and more workgroups, from 512 on five (fewer workgroups stage S again). Runs of 35 tuples and 48
+// hundred runs, then the reading of C (4 P^2 bytes per tuple): one entry per thread and more
+// workgroups, or five and fewer that stage S (finalize_entries). Runs of 35 tuples and 48
 // variables, before (one workgroup per run, a tuple at a time) and now: 256 runs 98 -> 25 us, 512
 // runs 95 -> 34 us. The contraction is spelled out, so both instantiations give the same bits.
 constexpr int kFinalizeChunk = 16;
@@ -3722,7 +3722,7 @@ int adjoint_normal_states(const mko_batch* batch, const mko_residual_settings* s
             hipLaunchKernelGGL(kernel, dim3(unsigned(P.V) * unsigned(parts)), dim3(256), lds, s,
                                P.T, m.P, parts, partC, partST, partT, a, g, live);
         };
-        if (P.V < 512) finalize(adjoint_normal_finalize_kernel<1>, 1);
+        if (finalize_entries(m.P, P.V) == 1) finalize(adjoint_normal_finalize_kernel<1>, 1);
         else finalize(adjoint_normal_finalize_kernel<5>, 5);
         check_hip(hipGetLastError(), "adjoint normal finalize launch");
     })

@@ -16,6 +16,17 @@ inline int64_t fd_direct_runs(int variables, int64_t tuples) {
     return std::min(int64_t(0x7fffffff) / per_run, int64_t(0xffffffff) / (256 * tuples));
 }
 
+// Entries of the upper triangle per thread of adjoint_normal_finalize_kernel: five read the tuples'
+// S once for all of them, which pays where many runs fill the chip and a workgroup's 1280 entries
+// are nearly all there. us with 1 / 5: 48 variables of 35 tuples, 256 runs 21 / 23, 400 runs 35 / 28,
+// 1024 runs 78 / 74; 96 variables of 20 tuples, 1024 runs 182 / 155; but 5 variables, 512 runs 10 /
+// 20 and 2048 runs 20 / 70; 36 variables, 1024 runs 21 / 26; 56 variables (two workgroups, 62 % of
+// their entries), 1024 runs 46 / 57.
+inline int finalize_entries(int variables, int runs) {
+    const int nu = variables * (variables + 1) / 2, places = 1280 * ((nu + 1279) / 1280);
+    return runs >= 400 && 8 * nu >= 7 * places ? 5 : 1;
+}
+
 // gram_kernel's split of a run's units (gw waves of 64 columns of g, then the upper 16 x 16 tiles of
 // a tg x tg grid) over `parts` workgroups of up to `upp` units, 1 ... 127 variables.
 struct GramPlan {
