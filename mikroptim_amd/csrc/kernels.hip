@@ -4152,15 +4152,12 @@ int fd_jacobian(const mko_batch* fd_batch, const mko_residual_settings* settings
                 if (f == first) plan.var[at++] = k | (f << 16) | (int(glass) << 24);
             }
         if (runs > fd_direct_runs(plan.P, P.T)) throw std::invalid_argument("batch too large");
-        // A tuple's variables are dealt out to 1, 2 or 4 workgroups (each traces the point itself,
-        // 2 of the about 2 + P passes) where there are few tuples: 1024 workgroups run at once, and
-        // 1120 (32 runs of the 35-tuple objective) leave most of a second round empty (2.25 ms in
-        // one part, 1.95 in two)
-        plan.parts = runs * P.T >= 4096 || plan.P < 8 ? 1 : runs * P.T >= 1024 || plan.P < 16 ? 2 : 4;
+        const int lanes = tuple_lanes(largest_tuple(P));
+        plan.parts = fd_parts(plan.P, int64_t(runs) * P.T, lanes / 64);
         const hipStream_t st = static_cast<hipStream_t>(stream);
         const auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(unsigned(runs) * unsigned(P.T * plan.parts)),
-                               dim3(tuple_lanes(largest_tuple(P))), fd_lds_bytes(S, vars->count),
+                               dim3(lanes), fd_lds_bytes(S, vars->count),
                                st, P, plan, step_plus, step_minus, stencil, jacobian, r0, jstride);
         };
         const int rpl = rays_per_lane(P);

@@ -10,10 +10,29 @@ namespace mko_internal {
 
 // Most runs of one fd_jacobian launch: the kernel counts the tuples of every variant, 2 P + 1
 // variants a run, in 32 bits, and a launch holds fewer than 2^32 threads (up to 256 a tuple; a
-// tuple's variables go to several workgroups only where there are fewer than 4096 tuples).
+// tuple's variables go to several workgroups only where there are fewer than 6144 tuples).
 inline int64_t fd_direct_runs(int variables, int64_t tuples) {
     const int64_t per_run = (2 * int64_t(variables) + 1) * tuples;
     return std::min(int64_t(0x7fffffff) / per_run, int64_t(0xffffffff) / (256 * tuples));
+}
+
+// Workgroups (of 1 ... 4 waves) that share a tuple's variables in fd_jacobian_kernel. Each traces the
+// point itself, 2 of its about 2 + P / parts passes, so parts pay where the tuples alone leave
+// places on the chip empty: some 4 waves per SIMD are resident, and at most about 9 workgroups of
+// small tuples per CU (LDS). us in 1 / 2 / 4 parts, 25 surfaces, 512 rays (4 waves) and 72 rays (2
+// waves) a tuple, or 22 surfaces and 48 rays (1 wave):
+//   48 variables, 512 rays   140 tuples 712 /  518 /  398,   840 1658 / 1430 / 1502,
+//                           1120 2028 / 1788 / 1910,        1680 2754 / 2841 / 2941
+//   24 variables, 72 rays    560 tuples 286 /  203 /  193,  1015  365 /  265 /  290,
+//                           2240  555 /  519 /  591,        3500  757 /  766 /  887
+//   47 variables, 48 rays    600 tuples 446 /  323 /  235,  1020  442 /  336 /  393,
+//                           4080 1310 / 1236 / 1242
+//   4 variables, 72 rays     144 tuples  18 /   16 /   13,   576   22 /   20 /   24,
+//                           1800   31 /   39 /   54
+inline int fd_parts(int variables, int64_t tuples, int waves) {
+    const int64_t load = tuples * std::max(waves, 2);
+    if (variables < 8) return load < 2560 ? 2 : 1;
+    return load < 1792 ? 4 : tuples * waves < 6144 ? 2 : 1;
 }
 
 // Entries of the upper triangle per thread of adjoint_normal_finalize_kernel: five read the tuples'

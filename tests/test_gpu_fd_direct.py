@@ -210,3 +210,14 @@ def test_equal_bits_to_the_difference_kernel(engine, failure):
     J, r0, _, _ = engine.jacobian(base, s, v, x, method="fd", precision="fp64")
     assert np.array_equal(r0, rd.cpu().numpy())
     assert np.array_equal(J, Jd.cpu().numpy())
+
+
+def test_shared_tuples(engine):
+    """Tuples whose variables are shared by 4, 2 and 1 workgroups (by the number of tuples)."""
+    b, v = systems.objective(variants=200, seed=4)
+    s = ResidualSettings(rings=2, spokes=3, failure=abi.FAILURE_HARD)
+    base, x = b.take([0]), v.extract(b)
+    J, r0, _, _ = engine.jacobian(base, s, v, x, method="fd", precision="fp64")
+    for runs in (3, 60):
+        Jp, rp, _, _ = engine.jacobian(base, s, v, x[:runs], method="fd", precision="fp64")
+        assert np.array_equal(Jp, J[:runs]) and np.array_equal(rp, r0[:runs])
