@@ -86,10 +86,11 @@ __device__ __forceinline__ bool is_soft(uint8_t s) {
     return s == MKO_STATUS_SOFT_MISSED || s == MKO_STATUS_SOFT_TIR;
 }
 
-// Division, reciprocal and square root of the FP64 traces and of the reverse sweep: hardware reciprocal / reciprocal square root refined by
-// Newton steps (a few ulp) instead of the correctly rounded IEEE sequences with their scaling and
-// fix-up steps. These paths need ~1e-15 relative accuracy (Jacobian columns are compared to
-// 1e-10, OPD to 1e-12 mm per ray); the df64 trace keeps its own operations.
+// Division, reciprocal and square root of the FP64 traces and of the reverse sweep: hardware
+// reciprocal / reciprocal square root refined by Newton steps (a few ulp) instead of the correctly
+// rounded IEEE sequences with their scaling and fix-up steps. These paths need ~1e-15 relative
+// accuracy (Jacobian columns are compared to 1e-10, OPD to 1e-12 mm per ray); the df64 trace keeps its
+// own operations.
 // Measured on MI355X (2^20 arguments over 2^+-30): v_rcp_f64 and v_rsq_f64 are accurate to
 // ~5e-8; one Newton step gives 2.1e-15, two give <= 0.5 ulp. The quotient a * r with one residual
 // correction and the square root after one Goldschmidt step plus one correction are within
@@ -522,6 +523,17 @@ __device__ __forceinline__ StepFoot step_foot(V3<double> Q, V3<double> P, double
     return f;
 }
 
+// P + g N, N the unit normal at p. N_z first, then g N_z into P_z: the rounding of a sum P_z + g before
+// the rest of the term is that of a number of n's size, and P strays further from Snell's law and from
+// length n (path lengths 1.05 times further off, of rays near a failure 1.27 times, at the same number
+// of operations).
+__device__ __forceinline__ V3<double> add_normal(V3<double> P, double g, V3<double> p, double c) {
+#pragma clang fp contract(off)
+    const double cg = c * g, Nz = __builtin_fma(-c, p.z, 1.0);
+    return V3<double>{__builtin_fma(-cg, p.x, P.x), __builtin_fma(-cg, p.y, P.y),
+                      __builtin_fma(g, Nz, P.z)};
+}
+
 // One surface step in hard failure mode: (p, P, opl) from surface s - 1 to s. Every operation runs
 // for every ray and one test ends a failed one (precedence: backward, missed, TIR; its state is
 // then of no use). Missed: no intersection (D < 0), or the ray meets the tangent plane beyond the
@@ -539,11 +551,7 @@ __device__ __forceinline__ uint8_t momentum_step(V3<double>& p, V3<double>& P, d
                    __builtin_fma(lam, P.z, f.z)};
     opl = __builtin_fma(k.n2, f.l0 + lam, opl);
     const double k2 = f.D + k.dn2;
-    const double g = sqrt_pos(k2) - a;
-    const double cg = k.c * g;
-    const double pz = P.z + g;
-    P = V3<double>{__builtin_fma(-cg, p.x, P.x), __builtin_fma(-cg, p.y, P.y),
-                   __builtin_fma(-cg, p.z, pz)};
+    P = add_normal(P, sqrt_pos(k2) - a, p, k.c);
     const bool missed = !(f.D >= 0.0) || !(__builtin_fma(k.cn2, f.z, f.E) > 0.0);
     if (backward || missed || k2 < 0.0) [[unlikely]]
         return backward ? uint8_t(MKO_STATUS_BACKWARD)
@@ -613,11 +621,7 @@ __device__ __forceinline__ uint8_t momentum_step_soft(V3<double>& p, V3<double>&
         soft_refract(p, P, k, nb, a, k2, missed, soft, branch);
         return MKO_STATUS_OK;
     }
-    const double g = sqrt_pos(k2) - a;
-    const double cg = k.c * g;
-    const double pz = P.z + g;
-    P = V3<double>{__builtin_fma(-cg, p.x, P.x), __builtin_fma(-cg, p.y, P.y),
-                   __builtin_fma(-cg, p.z, pz)};
+    P = add_normal(P, sqrt_pos(k2) - a, p, k.c);
     branch = kBranchRegular;
     return MKO_STATUS_OK;
 }
