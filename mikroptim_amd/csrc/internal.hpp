@@ -8,10 +8,6 @@
 
 namespace mko_internal {
 
-// Final ray states of a MERIT trace, kept for the fused adjoint at the same point: per ray the
-// position and direction on the last surface and the OPL at the reference sphere (NaN for a ray
-// that failed), structure of arrays: data[(c * slots + slot) * rays + row], c = p.x, p.y, p.z,
-// d.x, d.y, d.z, opl. Variant v of a launch uses slot slot[v] (slot == NULL: slot_offset + v).
 // Launch shapes the engine's autotuner chooses: pack_rays (0: automatic; 32, 64, 128: the
 // segment of a tuple pack, used where the tuples fit it; 256: one tuple per workgroup) and
 // fused_waves (0: automatic; 1, 2, 4: waves per workgroup of the fused normal equations). The
@@ -31,6 +27,10 @@ struct TuningScope {
     TuningScope& operator=(const TuningScope&) = delete;
 };
 
+// Final ray states of a MERIT trace, kept for the fused adjoint at the same point: per ray the
+// position and direction on the last surface and the OPL at the reference sphere (NaN for a ray
+// that failed), structure of arrays: data[(c * slots + slot) * rays + row], c = p.x, p.y, p.z,
+// d.x, d.y, d.z, opl. Variant v of a launch uses slot slot[v] (slot == NULL: slot_offset + v).
 struct RayStates {
     double* data;
     const int32_t* slot;

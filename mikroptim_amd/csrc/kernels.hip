@@ -1,13 +1,15 @@
 // gfx950 kernels of the batched forward-and-Jacobian path and their device-level C entry points.
 //
-// Work decomposition (all kernels): one workgroup of 256 lanes (4 wave64) per (variant, tuple),
-// tuple = (field f, wavelength l), t = f * L + l; the tuple's rays sit on lanes, ray k of the
-// tuple on lane k mod 256 (iteration k / 256). The surface table of the (variant, wavelength)
-// is staged once per workgroup in LDS (curvature, vertex distance, index, mu = n/n'), so the
-// per-ray surface loop reads wave-uniform LDS broadcasts. Every reduction over rays (piston,
-// merit partials, piston projection of the Jacobian) is a fixed-order tree: lane-local sum in
-// iteration order, xor-butterfly inside the wave, waves summed in index order; results depend
-// only on the tuple, never on the batch composition or the launch.
+// Work decomposition, where a kernel's own comment says nothing else: one workgroup per (variant,
+// tuple), tuple = (field f, wavelength l), t = f * L + l, of 256 lanes or of the waves that the
+// largest tuple's rays fill; the tuple's rays sit on lanes, ray k on lane k mod lanes (iteration k /
+// lanes). Small tuples share workgroups (trace_pack_kernel, prefilter_kernel). The surface table of
+// the (variant, wavelength) is staged once per workgroup in LDS (Step: curvature, vertex distance and
+// the products of the media that a step takes; the df64 trace: curvature, vertex distance, index, mu =
+// n/n'), so the per-ray surface loop reads wave-uniform LDS broadcasts. Every reduction over rays
+// (piston, merit partials, piston projection of the Jacobian) has a fixed order: lane-local sum in
+// iteration order, xor-butterfly inside the wave, waves summed in index order; results depend only
+// on the tuple, never on the batch composition or the launch.
 //
 // Reference counterparts: residuals_kernel src/cuda/residuals.cu:58, merit_kernel +
 // merit_finalize_kernel src/cuda/merit.cu:63/207, fd_difference_kernel src/cuda/fd_jacobian.cu:65,
@@ -1757,12 +1759,11 @@ struct FdPlan {
 // of the system for both differences of the variables that start there. About half of the
 // surface steps of tracing every variant (P = 48, 25 surfaces: 1250 instead of 2328 per ray), and
 // the differences' residuals stay in registers: 32 runs x 17920 rays 3.5 + 0.2 ms (every variant
-// traced, then differenced in a second kernel) -> 1.95 ms, 0.74 of the vector ALU's issue slots.
+// traced, then differenced in a second kernel) -> 1.95 ms, 0.79 vector instructions per quad cycle.
 // Registers capped for 4 waves per SIMD up to 512 rays per tuple in hard mode (28 bytes of spill).
 // Both differences of a ray in one pass of the surface loop (two chains): 1.92 ms, not kept. Same
-// step, reference sphere, sums
-// in the order of trace_kernel's and difference formula, so J and r0 are those of the two kernels
-// bit for bit.
+// step, reference sphere, sums in the order of trace_kernel's and difference formula, so J and r0 are
+// those of the two kernels bit for bit.
 template <bool kSoft, int kRpl>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(kSoft ? (kRpl <= 1 ? 3 : 1) : kRpl <= 2 ? 4 : 1)))
@@ -2254,8 +2255,9 @@ __global__ __launch_bounds__(kBlock) void adjoint_kernel(TraceParams P, ParamMap
 // ones (v_mfma_f64_4x4x4_4b: lane l holds the sum of the group l / 4 in all four lanes) and added
 // to the wave's own 16 sums of the column: 128 bytes of LDS per column and wave, a quarter of a
 // slot per lane, so 5 workgroups fit a CU at 48 variables (0.42 ms for 128 runs x 17920 rays; 1.99
-// ms with two traces, a record in private memory and a slot per lane: 1.5 waves per SIMD). Every lane of a wave runs the sweep
-// (the matrix instruction takes all lanes); those without a regular ray give zeros.
+// ms with two traces, a record in private memory and a slot per lane: 1.5 waves per SIMD). Every lane
+// of a wave runs the sweep (the matrix instruction takes all lanes); those without a regular ray give
+// zeros.
 struct GroupSink {
     double* acc; // [P][16] of this wave
     int slot;    // lane / 4
@@ -3042,10 +3044,10 @@ typedef __attribute__((ext_vector_type(4))) double f64x4;
 // normal_equations.hpp:19), products of the stored J values: bitwise the host definition.
 // v_mfma_f64_16x16x4_f64 adds its four products to the accumulator as that chain does (measured
 // bit for bit on MI355X against the VALU chain over rows of mixed signs and 24 decades, subnormal
-// numbers, zeros of either sign, infinities and NaN; the GPU tests hold it), so J^T J runs on it in 16 x 16 tiles; operand lane l: A(m = l % 16, k = l / 16),
-// B(k = l / 16, n = l % 16), result lane l, element e: row 4 e + l / 16, column l % 16. g is a
-// VALU chain per column beside the tiles: as a matrix column it would cost a row of tiles of its
-// own (10 instead of 6 at 48 variables).
+// numbers, zeros of either sign, infinities and NaN; the GPU tests hold it), so J^T J runs on it in
+// 16 x 16 tiles; operand lane l: A(m = l % 16, k = l / 16), B(k = l / 16, n = l % 16), result lane l,
+// element e: row 4 e + l / 16, column l % 16. g is a VALU chain per column beside the tiles: as a
+// matrix column it would cost a row of tiles of its own (10 instead of 6 at 48 variables).
 //
 // One workgroup of 8 waves per (run, part): the units (a wave of 64 columns of g, or one upper
 // tile) are cut into `parts` ranges, a wave takes kT of its range; the columns that the range
@@ -3177,9 +3179,9 @@ __global__ __launch_bounds__(512) void gram_kernel(const double* J, const double
 }
 
 // More than 127 variables (their columns do not fit the LDS stages above): 64 x 64 output tile per
-// workgroup over the upper tiles of the (P+1) x (P+1) matrix, 256 threads
-// each holding a 4 x 4 block of elements: 16 independent FMA chains per thread (the chains' latency
-// is what bounds a Gram of long columns). Rows are staged through LDS 32 at a time, row-major
+// workgroup over the upper tiles of the (P+1) x (P+1) matrix, 256 threads each holding a 4 x 4 block
+// of elements: 16 independent FMA chains per thread (the chains' latency is what bounds a Gram of
+// long columns). Rows are staged through LDS 32 at a time, row-major
 // [row][column], so a thread reads its 4 consecutive columns as two 16-byte words. Each element is
 // one FMA chain over the rows in ascending order starting from 0 (gram_dot,
 // normal_equations.hpp:19), products of the stored J values: bitwise the host definition.
