@@ -492,6 +492,13 @@ __device__ __forceinline__ uint8_t trace_ray_ext(const TraceParams& P, Table L, 
     return reference_end<kSoft>(P, L, r, M, kappa, soft, rec);
 }
 
+// A wave-uniform value, into scalar registers.
+__device__ __forceinline__ double first_lane(double x) {
+    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(x));
+    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(x));
+    return __hiloint2double(hi, lo);
+}
+
 // ---- deterministic block reductions -----------------------------------------------------------
 
 template <class T>
@@ -2076,6 +2083,7 @@ __device__ __forceinline__ void sweep_ray(const TraceParams& P, const Step* L, c
                                           V3<double> p, V3<double> d, V3<double> M, double kappa,
                                           const Sink& sink, int l) {
     const int S = P.S;
+    const double least = first_lane(mkod::sweep_least(L[0].n));
     double mz, length;
     mkod::SweepState w = mkod::sweep_reference(p, d, M, kappa, P.ref_kind, L[S - 1].n, L[S - 1].c,
                                                mz, length);
@@ -2088,7 +2096,7 @@ __device__ __forceinline__ void sweep_ray(const TraceParams& P, const Step* L, c
             sink.write(map.glass_col[j][1], length * wl);
             sink.write(map.glass_col[j][2], length * (wl * wl));
         }
-        const double cb = mkod::sweep_refract(w, L[j]);
+        const double cb = mkod::sweep_refract(w, L[j], least);
         if ((P.sphere_mask >> j) & 1ull) sink.write(map.curv_col[j], cb);
         if (kFine) {
             const double n = L[j - 1].n;
@@ -2098,7 +2106,8 @@ __device__ __forceinline__ void sweep_ray(const TraceParams& P, const Step* L, c
             sink.write(map.thick_col[j - 1], w.P.z + w.dP.z);
         }
         if (j == 1) break;
-        mkod::sweep_transfer<kGlass>(w, L[j], L[j - 1].c, L[j - 1].cna, L[j - 1].n, length);
+        mkod::sweep_transfer<kGlass>(w, L[j], L[j - 1].c, L[j - 1].cna, L[j - 1].n, least,
+                                     length);
     }
 }
 
@@ -2482,13 +2491,6 @@ struct GradLayout {
         return p * kRowBytes + 32 * s + ((((s >> 3) & 1) ^ 1) << 4);
     }
 };
-
-
-__device__ __forceinline__ double first_lane(double x) {
-    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(x));
-    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(x));
-    return __hiloint2double(hi, lo);
-}
 
 // Gradient sink of the fused kernel. Every lane of the wave runs the sweep (those without a
 // reached ray on a placeholder state), so column p is written by all lanes together: the value of

@@ -491,12 +491,14 @@ __device__ __forceinline__ double sqrt_pos(double x) {
     double h;
     return sqrt_from(x, __builtin_amdgcn_rsq(__builtin_fmax(x, 0x1p-900)), h);
 }
-// The root of a squared P . N (n2 = n^2 of its medium) that the reverse sweep forms from the way
-// back, and 1 / (2 root). The trace accepted the ray with a square >= 0; rounding, some 2^-52 n^2,
-// may leave this one below zero where the ray grazes the surface, so it is held at that size: the
-// gradients stay those of a grazing ray instead of overflowing.
-__device__ __forceinline__ double sweep_root(double x, double n2, double& half_rcp) {
-    const double v = __builtin_fmax(x, 0x1p-52 * n2);
+// The root of a squared P . N that the reverse sweep forms from the way back, and 1 / (2 root). The
+// trace accepted the ray with a square >= 0; rounding, some 2^-52 n^2, may leave this one below zero
+// where the ray grazes the surface, so it is held at `least`, 2^-54 of the first medium's n^2
+// (sweep_least): the gradients stay those of a grazing ray instead of overflowing. (2^-52 of each
+// gap's n^2 would be one product more per surface, 2 % of the fused kernel's time.)
+__device__ __forceinline__ double sweep_least(double n0) { return 0x1p-54 * (n0 * n0); }
+__device__ __forceinline__ double sweep_root(double x, double least, double& half_rcp) {
+    const double v = __builtin_fmax(x, least);
     return sqrt_from(v, __builtin_amdgcn_rsq(v), half_rcp);
 }
 
@@ -666,9 +668,9 @@ __device__ __forceinline__ SweepState sweep_start(V3<double> p, V3<double> P, V3
 
 // Backwards through the refraction at surface j (k: its step): P and dP become those before the
 // surface; returns the curvature gradient. On entry a = P' . N.
-__device__ __forceinline__ double sweep_refract(SweepState& w, const Step& k) {
+__device__ __forceinline__ double sweep_refract(SweepState& w, const Step& k, double least) {
     double h;
-    const double a = sweep_root(__builtin_fma(w.a, w.a, -k.dn2), k.n2, h);
+    const double a = sweep_root(__builtin_fma(w.a, w.a, -k.dn2), least, h);
     const double g = w.a - a;
     const double u = dot(w.dP, w.N) - k.c * dot(w.P, w.dq); // change of P' . N
     const double dg = u * g * (h + h);                      // minus the change of g
@@ -685,9 +687,9 @@ __device__ __forceinline__ double sweep_refract(SweepState& w, const Step& k) {
 // respect to the gap's index.
 template <bool kIndex>
 __device__ __forceinline__ void sweep_transfer(SweepState& w, const Step& k, double c, double cna,
-                                               double n, double& length) {
+                                               double n, double least, double& length) {
     const StepFoot f = step_foot(V3<double>{w.q.x, w.q.y, w.q.z + k.t}, w.P, c, k.ni2, cna);
-    w.a = sweep_root(f.D, k.n2, w.ha);
+    w.a = sweep_root(f.D, least, w.ha);
     const double lam = rev_div(f.H, w.P.z + w.a);
     w.q = V3<double>{f.x + lam * w.P.x, f.y + lam * w.P.y, f.z + lam * w.P.z};
     const double back = f.l0 + lam; // q = Q + back P

@@ -2,7 +2,7 @@
 hardware's reciprocal estimates replaced by the exact ones). A ray whose incidence, or whose exit
 after refraction, is within rounding of grazing is accepted by the trace; the sweep forms the same
 cosine again from the way back, where rounding may leave its square below zero. Its gradients stay
-finite and of the size that a cosine of 2^-26, the root of that rounding, gives."""
+finite and of the size that a cosine of 2^-27, half the root of that rounding, gives."""
 
 import os
 import subprocess
@@ -45,7 +45,7 @@ Result ray(const double* c, const double* t, const double* n, double y, double a
     for (int s = 1; s < 4; ++s) L[s] = step(c[s], t[s - 1], n[s - 1], n[s]);
     V3<double> p{0.0, y, 0.0}, P{0.0, n[0] * std::sin(angle), n[0] * std::cos(angle)};
     double opl = 0.0;
-    Result r{0, 1.0, 0.0};
+    Result r{0, n[0] * n[0], 0.0};
     for (int s = 1; s < 4; ++s) {
         double a;
         r.status = momentum_step(p, P, opl, L[s], a);
@@ -59,6 +59,7 @@ Result ray(const double* c, const double* t, const double* n, double y, double a
     uint8_t branch = 0;
     r.status = reference_step<false>(end, M, 0.0, MKO_REF_LAST_SURFACE, n[3], soft, branch);
     if (r.status != MKO_STATUS_OK) return r;
+    const double least = sweep_least(n[0]);
     double mz, length;
     SweepState w = sweep_reference(p, d, M, 0.0, MKO_REF_LAST_SURFACE, n[3], L[3].c, mz, length);
     const auto see = [&](double x) {
@@ -66,10 +67,10 @@ Result ray(const double* c, const double* t, const double* n, double y, double a
     };
     see(mz);
     for (int j = 3;; --j) {
-        see(sweep_refract(w, L[j]));
+        see(sweep_refract(w, L[j], least));
         see(w.P.z + w.dP.z);
         if (j == 1) break;
-        sweep_transfer<false>(w, L[j], L[j - 1].c, L[j - 1].cna, L[j - 1].n, length);
+        sweep_transfer<false>(w, L[j], L[j - 1].c, L[j - 1].cna, L[j - 1].n, least, length);
     }
     return r;
 }
@@ -87,7 +88,9 @@ int main() {
         const int at = i % 2 ? 1 : 2;
         double c[4] = {0.0, u(-0.01, 0.01), u(-0.01, 0.01), u(-0.01, 0.01)};
         const double scale = i % 3 ? 1.0 : u(0.5, 3.0); // media other than air around the glass
-        const double n[4] = {scale, at == 1 ? scale * u(1.3, 1.9) : scale * u(1.4, 1.9), scale, scale};
+        const double unit = i % 5 ? 1.0 : 1e-9;         // indices in another unit
+        const double glass = at == 1 ? u(1.3, 1.9) : u(1.4, 1.9), n0 = scale * unit;
+        const double n[4] = {n0, n0 * glass, n0, n0};
         const double t[3] = {u(0.0, 2.0), u(0.5, 3.0), u(0.5, 3.0)};
         const double y = u(1.0, 4.0), angle = u(-0.1, 0.1);
         double lo = 0.0, hi = at == 1 ? 2.0 / y : -2.0 / y;
@@ -100,11 +103,12 @@ int main() {
         }
         for (int back = 0; back < 6; ++back, lo = std::nextafter(lo, 0.0)) {
             c[at] = lo;
-            const Result r = ray(c, t, n, y, angle);
-            if (r.status != MKO_STATUS_OK || !(r.smallest < 1e-13)) continue;
+            Result r = ray(c, t, n, y, angle);
+            if (r.status != MKO_STATUS_OK || !(r.smallest < 1e-13 * unit * unit)) continue;
+            r.largest /= unit;
             ++grazing;
             // a gradient, of order 1 to 100 where no cosine is small, grows by the reciprocals of the
-            // grazing surface's two cosines, at most 2^26 each, in practice by one of them
+            // grazing surface's two cosines, at most some 2^27 each, in practice by one of them
             if (!(r.largest <= 0x1p52)) {
                 if (++fails <= 5)
                     std::printf("ray %d back %d: smallest %.2e gradient %.3e\n", i, back, r.smallest,
