@@ -321,16 +321,16 @@ def main():
     it_fd = n_fd / t_fd
 
     # roofline of the dominant kernel of the measured path, the fused adjoint + normal equations.
-    # Algorithmic FLOP (div/sqrt counted as 1, FMA as 2): FLOP_fwd = 59 (S-1) + 60 per ray for a
-    # forward trace, FLOP_adj = FLOP_fwd + 210 (S-1) + 6 P per ray for an adjoint Jacobian (its
-    # recording forward pass plus the reverse sweep). In the LM the fused kernel starts from the
-    # ray states that the MERIT trace of the same point stored, so its work is the reverse part,
-    # 210 (S-1) + 6 P per ray, plus the MFMA products (3 x 2 P^2 per ray, bf16). The MERIT trace
-    # (FLOP_fwd per ray) is reported beside it.
+    # FLOP of the operations that the kernels do (div/sqrt counted as 1, FMA as 2): 50 (S-1) + 60
+    # per ray for a forward trace (a step in optical direction cosines; source and reference sphere),
+    # 113 (S-1) + 6 P per ray for the reverse sweep with its row sums. In the LM the fused kernel
+    # starts from the ray states that the MERIT trace of the same point stored, so its work is the
+    # reverse part plus the MFMA products (3 x 2 P^2 per ray, bf16). The MERIT trace is reported
+    # beside it.
     S, P = batch.surfaces, variables.size
     rays = 17920
-    flop_fwd = 59 * (S - 1) + 60
-    flop_rev = 210 * (S - 1) + 6 * P
+    flop_fwd = 50 * (S - 1) + 60
+    flop_rev = 113 * (S - 1) + 6 * P
     adj_ms, adj_n = kt_adj["adjoint"]
     achieved = None
     runs_per_launch = jac_adj / adj_n if adj_n else 0.0
