@@ -1766,7 +1766,7 @@ struct FdPlan {
 // of the system for both differences of the variables that start there. About half of the
 // surface steps of tracing every variant (P = 48, 25 surfaces: 1250 instead of 2328 per ray), and
 // the differences' residuals stay in registers: 32 runs x 17920 rays 3.5 + 0.2 ms (every variant
-// traced, then differenced in a second kernel) -> 1.95 ms, 0.79 vector instructions per quad cycle.
+// traced, then differenced in a second kernel) -> 1.95 ms, 0.78 vector instructions per quad cycle.
 // Registers capped for 4 waves per SIMD up to 512 rays per tuple in hard mode (28 bytes of spill).
 // Both differences of a ray in one pass of the surface loop (two chains): 1.92 ms, not kept. Same
 // step, reference sphere, sums in the order of trace_kernel's and difference formula, so J and r0 are
