@@ -1,6 +1,7 @@
 """The FD Jacobian whose differences restart at the variable's surface (fd_jacobian) against the
 general path it replaces: RESIDUALS of every difference's point and the difference formula, bit for
-bit, for every kind of variable (curvatures of spheres, of a plane and of the stop, thicknesses,
+bit (the one-sided formula's bits by the difference kernel, elsewhere to rounding), for every kind of
+variable (curvatures of spheres, of a plane and of the stop, thicknesses,
 working distance, glass coefficients on the first, inner and last media), central, one-sided and
 truncated stencils, hard and soft failure with failing rays, tuples of 1 ... 2048 rays, image
 reference spheres and a point source. And what keeps the general path: constraint rows, df64."""
@@ -221,3 +222,20 @@ def test_shared_tuples(engine):
     for runs in (3, 60):
         Jp, rp, _, _ = engine.jacobian(base, s, v, x[:runs], method="fd", precision="fp64")
         assert np.array_equal(Jp, J[:runs]) and np.array_equal(rp, r0[:runs])
+
+
+@pytest.mark.parametrize("extra", [0, 90])
+def test_most_variables(engine, extra):
+    """217 and 307 variables of 63 surfaces: moved steps of 59 and 82 KB in LDS."""
+    b, v = systems.uneven_topology(0, variants=2, surfaces=62, variables=300)
+    base = b.take([0])
+    glass = {int(s) for s in v.batch_surface[v.type == abi.VAR_GLASS]}
+    air = [s for s in range(1, base.surfaces) if s not in glass]
+    base.buchdahl = base.buchdahl.copy()
+    base.buchdahl[:, air] = (1.0, 0.0, 0.0, 0.0)
+    items = [(int(t), int(q), int(c)) for t, q, c in zip(v.type, v.batch_surface, v.component)]
+    items += [(abi.VAR_GLASS, s, c) for s in air for c in range(3)][:extra]
+    w = _variables(items, [-1e3] * len(items), [1e3] * len(items))
+    assert w.size == 217 + extra
+    _check(engine, base, ResidualSettings(rings=1, spokes=2, failure=abi.FAILURE_HARD), w,
+           w.extract(base))
